@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -73,7 +74,7 @@ struct acc_gpu_matrix {
     // FP32 CSR
     bool has_csr = false;
     uint32_t *d_ptr = nullptr;
-    int32_t *d_idx = nullptr;
+    colx_t *d_idx = nullptr;         // 4 * column per entry
     float *d_val = nullptr;
     float *d_y = nullptr;            // FP32 scores of the plain path
     // select state of the FP32 path
@@ -751,14 +752,17 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         std::vector<uint32_t> p32(csr->ptr.size());
         for (size_t i = 0; i < p32.size(); ++i) p32[i] = (uint32_t)csr->ptr[i];
         TRY(dalloc(m, &m->d_ptr, p32.size()));
-        TRY(dalloc(m, &m->d_idx, (size_t)nnz + 4));  // 4 entries of padding for fp32_spmv's 16-byte loads
-        TRY(dalloc(m, &m->d_val, (size_t)nnz + 4));
+        TRY(dalloc(m, &m->d_idx, (size_t)nnz + 8));  // 8 entries of padding for fp32_spmv's 16-byte loads
+        TRY(dalloc(m, &m->d_val, (size_t)nnz + 8));
         TRY(dalloc(m, &m->d_y, (size_t)m->rows));
         COPY(m->d_ptr, p32.data(), p32.size() * 4);
-        COPY(m->d_idx, csr->idx.data(), (size_t)nnz * 4);
+        {
+            const std::unique_ptr<uint16_t[]> cx = acc::column_offsets(csr);
+            COPY(m->d_idx, cx.get(), (size_t)nnz * sizeof(colx_t));
+        }
         COPY(m->d_val, csr->val.data(), (size_t)nnz * 4);
-        ZERO(m->d_idx + nnz, 16);
-        ZERO(m->d_val + nnz, 16);
+        ZERO(m->d_idx + nnz, 8 * sizeof(colx_t));
+        ZERO(m->d_val + nnz, 32);
         select_geometry(m->rows, m->cus, m->sel_blocks, m->sel_chunk);
         TRY(dalloc(m, &m->d_sthr, 1));
         TRY(dalloc(m, &m->d_scnt, 1));
@@ -882,7 +886,7 @@ extern "C" int acc_gpu_matrix_info(const acc_gpu_matrix *m, acc_gpu_info_t *info
     info->group = m->group;
     info->work_items = m->nitems;
     info->nnz = m->nnz;
-    info->csr_bytes = m->has_csr ? m->nnz * 8 + ((int64_t)m->rows + 1) * 4 : 0;
+    info->csr_bytes = m->has_csr ? m->nnz * (int64_t)(4 + sizeof(colx_t)) + ((int64_t)m->rows + 1) * 4 : 0;
     info->stream_bytes = m->stream_bytes;
     info->device_bytes = m->device_bytes;
     info->batch_mode = m->batch_mode;
@@ -1062,20 +1066,21 @@ extern "C" int acc_gpu_spmv_fp64(acc_gpu_matrix *m, const float *x_dev, double *
 // FP32 CSR path
 // ---------------------------------------------------------------------------
 
-size_t fp32_spmv_lds(int cols, int G);  // k_fp32.hip
-
 static int launch_spmv_fp32(acc_gpu_matrix *m, const float *x_dev, float *y, hipStream_t st) {
-    spmv_fn k = get_fp32_spmv(m->group);
+    const int B = fp32_step_blocks(m->group, m->rows > 0 ? (double)m->nnz / m->rows : 0.0);
+    spmv_fn k = get_fp32_spmv(m->group, B);
     if (!k) return fail(ACC_ERR_ARG, "unsupported group size");
-    const int rpi = 64 / m->group;
-    const int nblocks = (m->rows + rpi - 1) / rpi;
-    // as many workgroups as run at once (each wavefront then owns one contiguous row range, and no
-    // second wave of workgroups leaves part of the chip idle at the end), fewer for small matrices
-    const size_t lds = fp32_spmv_lds(m->cols, m->group);
+    const int step_rows = B * (64 / m->group);
+    const int64_t steps = ((int64_t)m->rows + step_rows - 1) / step_rows;
+    // as many workgroups as run at once (a second wave of workgroups would leave part of the chip idle
+    // at the end), fewer for small matrices
+    const size_t lds = fp32_spmv_lds(m->cols, m->group, B);
     int occ = 1;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *)k, ACC_WG, lds) != hipSuccess || occ < 1)
         occ = 1;
-    const int blocks = std::max(1, std::min((nblocks + ACC_WAVES * 4 - 1) / (ACC_WAVES * 4), m->cus * occ));
+    const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((steps + ACC_WAVES - 1) / ACC_WAVES, (int64_t)m->cus * occ));
+    int rc = lds_limit((const void *)k, lds);
+    if (rc != ACC_OK) return rc;
     LAUNCH(m, 0, k, dim3(blocks), dim3(ACC_WG), lds, st, m->d_ptr, m->d_idx, m->d_val, x_dev, m->rows, m->cols, y);
     return check_launch();
 }

@@ -355,6 +355,16 @@ extern "C" int acc_csr_create(int32_t rows, int32_t cols, int64_t nnz, const int
     return ACC_OK;
 }
 
+std::unique_ptr<uint16_t[]> acc::column_offsets(const acc_csr *csr) {
+    const int64_t n = csr->nnz();
+    std::unique_ptr<uint16_t[]> out(new uint16_t[(size_t)std::max<int64_t>(n, 1)]);
+    const int32_t *idx = csr->idx.data();
+    uint16_t *o = out.get();
+#pragma omp parallel for schedule(static)
+    for (int64_t i = 0; i < n; ++i) o[i] = (uint16_t)(idx[i] * 4);
+    return out;
+}
+
 extern "C" int acc_csr_info(const acc_csr *m, int32_t *rows, int32_t *cols, int64_t *nnz) {
     if (!m) return fail(ACC_ERR_ARG, "null handle");
     if (rows) *rows = m->rows;

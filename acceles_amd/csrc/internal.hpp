@@ -4,6 +4,7 @@
 #include "../../include/acceles.h"
 
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -61,6 +62,10 @@ inline uint32_t ordered_f32(float f) {
 }
 
 int bits_for(int32_t n);  // ceil(log2(n)), at least 1
+
+// 4 * column of every entry (cols <= 8192): the columns as the device reads them.
+std::unique_ptr<uint16_t[]> column_offsets(const acc_csr *csr);
+
 // Batched low-bit queries with a workspace of the caller's (acc_gpu_topk_
 // lowbit_batch uses the handle's own, so one handle runs one batch at a
 // time): several workspaces keep several batches of one matrix in flight on

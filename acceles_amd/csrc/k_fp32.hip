@@ -8,40 +8,110 @@
 //   spmv_fp64       FP64 exact scores for precision/recall reporting.
 #include "kernels_common.hpp"
 
+#include <algorithm>
+#include <type_traits>
+
 // ---------------------------------------------------------------------------
 // FP32 CSR path
 // ---------------------------------------------------------------------------
 
+// p + the value of lane ^ S, S a power of two below 32: the rounding of p +
+// __shfl_xor(p, S) without the LDS crossbar.  Lane ^ 4 is the quad reversal
+// of the half-row mirror; lane ^ 16 comes from v_permlane16_swap, whose two
+// results hold the even and the odd 16-lane rows.
+template <int S>
+__device__ __forceinline__ float xor_add(float p) {
+    const int v = __float_as_int(p);
+    if constexpr (S == 1) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+    if constexpr (S == 2) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+    if constexpr (S == 4) {
+        const int t = __builtin_amdgcn_update_dpp(v, v, 0x1B, 0xF, 0xF, false);
+        return p + __int_as_float(__builtin_amdgcn_update_dpp(t, t, 0x141, 0xF, 0xF, false));
+    }
+    if constexpr (S == 8) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));
+    if constexpr (S == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return p;
+}
+template <int G>
+__device__ __forceinline__ float butterfly(float p) {
+    if constexpr (G > 16) p = xor_add<16>(p);
+    if constexpr (G > 8) p = xor_add<8>(p);
+    if constexpr (G > 4) p = xor_add<4>(p);
+    if constexpr (G > 2) p = xor_add<2>(p);
+    return xor_add<1>(p);
+}
+
 // y = A x with G lanes per row.  Lane g of a row sums its entries
 // g, g+G, g+2G, ... in that order with fmaf, then an xor butterfly of plain
-// adds.  A step is B blocks of 64/G rows; the steps are dealt to the
-// wavefronts in turn, so that the wavefronts in flight read neighbouring
-// entries (one contiguous range of rows per wavefront, i.e. thousands of
-// separate streams, measured 6% slower on a 20M-row matrix).  The step's rows
-// hold one contiguous range of entries:
-// for short rows (G <= 8) and when it fits kFp32Stage entries, it is first
-// copied into the wavefront's LDS area with 16-byte loads (whole cache lines,
-// each byte read once), one step ahead, and the G-lane order then reads LDS;
-// otherwise the lanes load the entries directly, the
-// first U per lane of all B blocks together (rows longer than U*G entries
-// continue block by block).  The next step's bounds are fetched early.  x is
-// staged in LDS.  idx and val hold 4 entries of padding past nnz (the last
-// 16-byte load may reach 3 entries past the range).
-static constexpr int kFp32Stage = 1024;  // entries per wavefront staged in LDS (value and column: 8 KB)
+// adds.
+//
+// Bound: HBM, 6 bytes per entry; the LDS pipe is next (three LDS reads per
+// entry slot).  A step is RS = B * 64/G rows, one contiguous range of
+// entries; the steps are dealt to the wavefronts in turn, so that the
+// wavefronts in flight read neighbouring entries.  A step's entries are read
+// with 16-byte loads (whole cache lines, each byte once) into registers one
+// step ahead, written to the wavefront's LDS area and summed from there in
+// the G-lane order.  The loads go through buffer resources that end with the
+// step's range, so they are unconditional (a conditional load is waited for
+// before the next is issued) and fetch nothing else; past the range they
+// leave zeros.  The row starts of a step are one load, two steps ahead, and
+// reach the rows' lanes through LDS.  x is staged in LDS at offset 0, where a
+// stored column is its address.
+//
+// The area: 896 entries at 6 bytes leave five workgroups per CU at 900
+// columns.  2,000,000 x 900 (rows of 30-90, G = 16): 141 us, 5.1 TB/s; with
+// areas of 768 / 1024 / 1536 entries 145 / 162 / 143 us; loading the rows'
+// entries with 4-byte loads and 4-byte columns 286 us.  4,999,999 x 1024
+// power-law rows (G = 8): 196 us (768: 211, 1024: 232; before: 258).
+// 100,000 x 500 (rows of 50-90, G = 32): 11.2 us (before: 15.3).
+static constexpr int kFp32Stage = 896;   // entries per wavefront staged in LDS
+static constexpr int kFp32Slack = 128;   // readable past them (the last batch of a row reads up to U*G - 1 further)
+static constexpr int kFp32Area = kFp32Stage + kFp32Slack;
 
-// LDS of an fp32_spmv<G> workgroup: x, then (G <= 8) each wavefront's staging area.
-size_t fp32_spmv_lds(int cols, int G) {
-    return (((size_t)cols * 4 + 15) & ~(size_t)15) + (G <= 8 ? (size_t)ACC_WAVES * kFp32Stage * 8 : 0);
+template <int G, int B>
+struct SpmvShape {
+    static constexpr int RPI = 64 / G;              // rows per block
+    static constexpr int RS = B * RPI;              // rows per step
+    static constexpr int NP = RS / 64 + 1;          // loads of its RS + 1 row starts
+    // entries per lane in the first batch (of all blocks) and in one further
+    // batch of a block: the slots past a row's end are wasted LDS reads
+    // (power-law rows: 206 us with further batches of four, 196 with two)
+    static constexpr int U = G >= 16 ? 3 : 4, kTail = 2;
+    static constexpr int kWave = kFp32Area * 6 + NP * 256;  // LDS bytes of a wavefront
+};
+
+// B of a matrix of this mean row length: a mean step fills at most 85% of the
+// staging area (row lengths vary; 75% and 95%, i.e. two and four blocks
+// instead of three, were slower at 2,000,000 x 900: 145 and 188 against 141
+// us), at most 4 blocks (6 of the two-row blocks of G = 32) so that a step's
+// registers leave five wavefronts per SIMD.
+int fp32_step_blocks(int G, double mean_row) {
+    const double per_block = std::max(mean_row, 1.0) * (64 / G);
+    const int fit = (int)std::min(6.0, 0.85 * kFp32Stage / per_block);
+    if (G == 32 && fit >= 6) return 6;
+    return fit >= 4 ? 4 : fit >= 3 ? 3 : fit >= 2 ? 2 : 1;
 }
 
 template <int G, int B>
-__global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const int32_t *idx, const float *val,
+__global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const colx_t *idx, const float *val,
                                                    const float *x, int rows, int cols, float *y) {
+    using S = SpmvShape<G, B>;
+    constexpr int RPI = S::RPI, RS = S::RS, NP = S::NP, U = S::U, kTail = S::kTail;
+    static_assert(U * G <= kFp32Slack, "a batch stays in the slack");
+    static_assert((kFp32Stage + 255) / 256 * 256 - kFp32Area <= kFp32Area / 2, "value loads end within the columns");
+    static_assert((kFp32Stage + 511) / 512 * 512 >= kFp32Area, "the slack's columns are written (zeros)");
+    static_assert(((kFp32Stage + 511) / 512 * 512 - kFp32Area) * 2 <= 256, "column loads end within the row starts");
     extern __shared__ __align__(16) unsigned char smem[];
     float *xs = (float *)smem;
     const uint32_t xs_bytes = ((uint32_t)cols * 4u + 15u) & ~15u;
-    float *sv = (float *)(smem + xs_bytes) + (threadIdx.x >> 6) * kFp32Stage;  // this wavefront's staged values
-    int32_t *sc = (int32_t *)(smem + xs_bytes + ACC_WAVES * kFp32Stage * 4) + (threadIdx.x >> 6) * kFp32Stage;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // uniform: steps and ranges stay scalar
+    unsigned char *area = smem + xs_bytes + wave * S::kWave;  // this wavefront's
+    float *sv = (float *)area;                                // staged values,
+    colx_t *sc = (colx_t *)(area + kFp32Area * 4);            // columns
+    uint32_t *sp = (uint32_t *)(area + kFp32Area * 6);        // and row starts of the step
     for (int c0 = 0; c0 < cols; c0 += 4 * ACC_WG) {  // four loads per thread issued together
         float t[4];
 #pragma unroll
@@ -50,176 +120,167 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const i
         for (int u = 0; u < 4; ++u)
             if (c0 + u * ACC_WG + (int)threadIdx.x < cols) xs[c0 + u * ACC_WG + threadIdx.x] = t[u];
     }
+    const int lane = lane_id(), g = lane & (G - 1), grp = lane / G;
     __syncthreads();
-    constexpr int RPI = 64 / G;  // rows per block
-    constexpr int U = 4;
-    const int lane = lane_id(), g = lane & (G - 1);
-    const int nblocks = (rows + RPI - 1) / RPI;
-    const int gw = blockIdx.x * ACC_WAVES + (threadIdx.x >> 6), nw = gridDim.x * ACC_WAVES;
-    // steps of B blocks dealt to the wavefronts in turn (wavefront gw takes
-    // steps gw, gw + nw, ...): the wavefronts in flight read neighbouring
-    // entries, not one stream each
-    const int b0 = gw * B, b1 = nblocks, SB = nw * B;
-    if (b0 >= b1) return;
-    // row bounds are loaded unconditionally (row clamped into the matrix) and
-    // masked after: a conditional load would be waited for before the step's
-    // entry loads are issued
-    uint32_t jb[B], je[B];
+    const int nsteps = (int)(((int64_t)rows + RS - 1) / RS);
+    const int gw = blockIdx.x * ACC_WAVES + wave, nw = gridDim.x * ACC_WAVES;
+    if (gw >= nsteps) return;
+
+    typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+    constexpr int NV = (kFp32Stage + 255) / 256, NC = (kFp32Stage + 511) / 512;
+    v4 lv[NV], lc[NC];
+    auto load_starts = [&](int s, uint32_t (&p)[NP]) {  // row starts of step s (past the matrix: nnz)
+        const int r0 = min(s, nsteps - 1) * RS;
 #pragma unroll
-    for (int t = 0; t < B; ++t) {
-        const int r = (b0 + t) * RPI + lane / G;
-        const bool ok = b0 + t < b1 && r < rows;
-        const int rc = min(r, rows - 1);
-        const uint32_t p0 = ptr[rc], p1 = ptr[rc + 1];
-        jb[t] = ok ? p0 : 0u;
-        je[t] = ok ? p1 : 0u;
-    }
-    // the entry range of a step: its first row's start to its last row's end
-    auto range = [&](int b, uint32_t &s, uint32_t &e) {
-        const int r0 = b * RPI, r1 = min(min(b + B, b1) * RPI, rows);
-        s = ptr[r0];
-        e = ptr[r1];
+        for (int i = 0; i < NP; ++i) p[i] = ptr[(int)min((int64_t)r0 + i * 64 + lane, (int64_t)rows)];
     };
-    // the step's entries in flight in registers: 16-byte loads over [s & ~3, e); rows of up to 8 lanes
-    // only (longer rows already read whole cache lines per lane group)
-    constexpr bool kStaged = G <= 8;
-    constexpr int NL = kFp32Stage / 256;
-    typedef float vf4 __attribute__((ext_vector_type(4)));
-    typedef int vi4 __attribute__((ext_vector_type(4)));
-    vf4 lv[NL];
-    vi4 lc[NL];
-    auto issue = [&](uint32_t s, uint32_t e) {
-        const uint32_t sa = s & ~3u, cnt = e - sa;
-        if (!kStaged || cnt > (uint32_t)kFp32Stage) return false;
+    auto first = [&](const uint32_t (&p)[NP]) { return (uint32_t)__builtin_amdgcn_readlane((int)p[0], 0); };
+    auto last = [&](const uint32_t (&p)[NP]) { return (uint32_t)__builtin_amdgcn_readlane((int)p[RS / 64], RS % 64); };
+    auto fits = [&](uint32_t b, uint32_t e) { return e - (b & ~7u) <= (uint32_t)kFp32Stage; };
+    // the entries [b & ~7, e) into lv and lc (none of a range that exceeds the area)
+    auto issue = [&](uint32_t b, uint32_t e) {
+        const uint32_t sa = b & ~7u;
+        const uint32_t cnt = fits(b, e) ? (e - sa + 7u) & ~7u : 0u;
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(val + sa), (short)0, (int)(cnt * 4u), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void *)(idx + sa), (short)0, (int)(cnt * 2u), 0x00020000);
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const uint32_t o = (uint32_t)(i * 256 + lane * 4);
-            if (o < cnt) {
-                lv[i] = __builtin_nontemporal_load((const vf4 *)(val + sa + o));
-                lc[i] = __builtin_nontemporal_load((const vi4 *)(idx + sa + o));
-            }
-        }
-        return true;
+        for (int i = 0; i < NV; ++i) lv[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, (i * 64 + lane) * 16, 0, 2 /* nt */);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) lc[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, (i * 64 + lane) * 16, 0, 2 /* nt */);
     };
-    // ranges: this step's (rs, re), the next one's (ns, ne2); the one after is fetched in the loop
-    uint32_t rs, re, ns = 0, ne2 = 0;
-    range(b0, rs, re);
-    if (b0 + SB < b1) range(b0 + SB, ns, ne2);
-    bool have = issue(rs, re);  // this step's entries are in lv/lc
-    for (int b = b0; b < b1; b += SB) {
-        uint32_t nb[B], ne[B];
+    // The loads' last bytes (zeros: they cover more than the area) may fall on
+    // what follows and is written after: the columns, then the row starts,
+    // which are read before the area is staged again.
+    auto stage = [&]() {
 #pragma unroll
-        for (int t = 0; t < B; ++t) {  // the next step's row bounds
-            const int r = (b + SB + t) * RPI + lane / G;
-            const bool ok = b + SB + t < b1 && r < rows;
-            const int rc = min(r, rows - 1);
-            const uint32_t p0 = ptr[rc], p1 = ptr[rc + 1];
-            nb[t] = ok ? p0 : 0u;
-            ne[t] = ok ? p1 : 0u;
-        }
-        uint32_t ms = 0, me = 0;
-        if (b + 2 * SB < b1) range(b + 2 * SB, ms, me);
-        if (have) {
-            const uint32_t sa = rs & ~3u, cnt = re - sa;
+        for (int i = 0; i < NV; ++i) *(v4 *)(sv + (i * 64 + lane) * 4) = lv[i];
 #pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                const uint32_t o = (uint32_t)(i * 256 + lane * 4);
-                if (o < cnt) {
-                    *(vf4 *)(sv + o) = lv[i];
-                    *(vi4 *)(sc + o) = lc[i];
-                }
-            }
-            wave_sync();
-            // the next step's entries fly while this one is summed from LDS
-            const bool next = b + SB < b1 && issue(ns, ne2);
-            // the first U entries per lane of all B blocks: their LDS reads issued together (clamped
-            // into the staged range, masked after), then longer rows entry by entry
-            const uint32_t last = cnt ? cnt - 1u : 0u;  // clamped reads stay in the staged range
-            float p[B], a[B][U], xv[B][U];
+        for (int i = 0; i < NC; ++i)
+            *(v4 *)(sc + (i * 64 + lane) * 8) = lc[i];
+    };
+    // Entries k .. of NT rows per lane, U per lane and row, added to p in order
+    // (base: the lane's first entry's place in the area, n: entries of its row
+    // from there on).  All reads are issued before the first is used; the
+    // empty asm keeps them out of the branches that the masked additions
+    // would otherwise become.
+    auto batch = [&](auto nt, auto nu, const uint32_t *base, const int *n, int k, float *p) {
+        constexpr int NT = decltype(nt)::value, U = decltype(nu)::value;
+        float a[NT][U], xv[NT][U];
+        uint32_t c[NT][U];
 #pragma unroll
-            for (int t = 0; t < B; ++t)
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t o = min(jb[t] + g + u * G - sa, last);
-                    a[t][u] = sv[o];
-                    xv[t][u] = xs[min((uint32_t)sc[o], (uint32_t)cols - 1u)];
-                }
-#pragma unroll
-            for (int t = 0; t < B; ++t) {
-                p[t] = 0.f;
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (jb[t] + g + u * G < je[t]) p[t] = __builtin_fmaf(a[t][u], xv[t][u], p[t]);
-                for (uint32_t jj = jb[t] + g + U * G; jj < je[t]; jj += G) p[t] = __builtin_fmaf(sv[jj - sa], xs[sc[jj - sa]], p[t]);
-            }
-#pragma unroll
-            for (int t = 0; t < B; ++t) {
-#pragma unroll
-                for (int s2 = G / 2; s2 >= 1; s2 >>= 1) p[t] = p[t] + __shfl_xor(p[t], s2);
-                const int r = (b + t) * RPI + lane / G;
-                if (g == 0 && b + t < b1 && r < rows) y[r] = p[t];
-            }
-            wave_sync();  // the staged entries are read before the next step overwrites them
-#pragma unroll
-            for (int t = 0; t < B; ++t) {
-                jb[t] = nb[t];
-                je[t] = ne[t];
-            }
-            rs = ns;
-            re = ne2;
-            ns = ms;
-            ne2 = me;
-            have = next;
-            continue;
-        }
-        float v[B][U];
-        int c[B][U];
-#pragma unroll
-        for (int t = 0; t < B; ++t)
+        for (int t = 0; t < NT; ++t) {
+            const uint32_t b = min(base[t] + (uint32_t)k, (uint32_t)kFp32Stage);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const uint32_t jj = jb[t] + g + u * G;
-                v[t][u] = jj < je[t] ? __builtin_nontemporal_load(val + jj) : 0.f;
-                c[t][u] = jj < je[t] ? __builtin_nontemporal_load(idx + jj) : 0;
+                c[t][u] = sc[b + u * G];
+                a[t][u] = sv[b + u * G];
             }
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u) xv[t][u] = x_at(xs, c[t][u]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u) asm volatile("" : "+v"(a[t][u]), "+v"(xv[t][u]));
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float f = __builtin_fmaf(a[t][u], xv[t][u], p[t]);
+                p[t] = n[t] > k + u * G ? f : p[t];
+            }
+    };
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, B> all{};
+    constexpr std::integral_constant<int, U> un{};
+    constexpr std::integral_constant<int, kTail> tail{};
+    uint32_t pc[NP], pn[NP];  // row starts of this step and the next
+    load_starts(gw, pc);
+    load_starts(gw + nw, pn);
+    issue(first(pc), last(pc));
+    for (int s = gw;;) {
+        const uint32_t sa = first(pc) & ~7u;
+        const bool staged = fits(first(pc), last(pc));
+        stage();
+#pragma unroll
+        for (int i = 0; i < NP; ++i) sp[i * 64 + lane] = pc[i];
+        const bool more = nw < nsteps - s;
+        uint32_t pf[NP];
+        load_starts(more ? s + nw + min(nw, nsteps - 1 - s - nw) : s, pf);  // the step after the next
+        wave_sync();
         float p[B];
+        uint32_t jb[B], je[B];
 #pragma unroll
         for (int t = 0; t < B; ++t) {
+            jb[t] = sp[t * RPI + grp];
+            je[t] = sp[t * RPI + grp + 1];
             p[t] = 0.f;
+        }
+        if (!staged) {
+            // a step of long rows: block by block, waiting for each block's
+            // entries; a block that exceeds the area entry by entry, four per
+            // lane together
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (jb[t] + g + u * G < je[t]) p[t] = __builtin_fmaf(v[t][u], xs[c[t][u]], p[t]);
-            for (uint32_t j = jb[t] + g + U * G; j < je[t]; j += U * G) {  // longer rows
-                float w[U];
-                int d[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t jj = j + u * G;
-                    w[u] = jj < je[t] ? __builtin_nontemporal_load(val + jj) : 0.f;
-                    d[u] = jj < je[t] ? __builtin_nontemporal_load(idx + jj) : 0;
+            for (int t = 0; t < B; ++t) {
+                const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane((int)jb[t], 0);
+                const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane((int)je[t], 63);
+                if (fits(b0, b1)) {
+                    issue(b0, b1);
+                    wave_sync();  // the block before has been read
+                    stage();
+                    wave_sync();
+                    const uint32_t o = jb[t] - (b0 & ~7u) + g;
+                    const int n = (int)(je[t] - jb[t]) - g;
+                    for (int k = 0; __any(n > k); k += U * G) batch(one, un, &o, &n, k, &p[t]);
+                    continue;
                 }
+                for (uint32_t j = jb[t] + g; j < je[t]; j += 4 * G) {
+                    float v[4];
+                    uint32_t c[4];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (j + u * G < je[t]) p[t] = __builtin_fmaf(w[u], xs[d[u]], p[t]);
+                    for (int u = 0; u < 4; ++u) {  // clamped into the row (j < je): the loads issue together
+                        const uint32_t jj = min(j + u * G, je[t] - 1);
+                        v[u] = __builtin_nontemporal_load(val + jj);
+                        c[u] = __builtin_nontemporal_load(idx + jj);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (j + u * G < je[t]) p[t] = __builtin_fmaf(v[u], x_at(xs, c[u]), p[t]);
+                }
             }
         }
+        // the next step's entries fly while this one is summed (none past the last step)
+        issue(first(pn), more ? last(pn) : first(pn) & ~7u);
+        if (staged) {
+            uint32_t o[B];
+            int n[B];
 #pragma unroll
-        for (int t = 0; t < B; ++t) {
+            for (int t = 0; t < B; ++t) {
+                o[t] = jb[t] - sa + g;
+                n[t] = (int)(je[t] - jb[t]) - g;
+            }
+            batch(all, un, o, n, 0, p);
+            // longer rows, block by block
 #pragma unroll
-            for (int s = G / 2; s >= 1; s >>= 1) p[t] = p[t] + __shfl_xor(p[t], s);
-            const int r = (b + t) * RPI + lane / G;
-            if (g == 0 && b + t < b1 && r < rows) y[r] = p[t];
+            for (int t = 0; t < B; ++t)
+                for (int k = U * G; __any(n[t] > k); k += kTail * G) batch(one, tail, o + t, n + t, k, p + t);
         }
 #pragma unroll
         for (int t = 0; t < B; ++t) {
-            jb[t] = nb[t];
-            je[t] = ne[t];
+            p[t] = butterfly<G>(p[t]);
+            const int64_t r = (int64_t)s * RS + t * RPI + grp;
+            if (g == 0 && r < rows) y[r] = p[t];
         }
-        have = b + SB < b1 && issue(ns, ne2);
-        rs = ns;
-        re = ne2;
-        ns = ms;
-        ne2 = me;
+        if (!more) break;
+        s += nw;
+        wave_sync();  // the staged entries are read before the next step overwrites them
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            pc[i] = pn[i];
+            pn[i] = pf[i];
+        }
     }
 }
 
@@ -349,26 +410,44 @@ __global__ void select_reset(uint64_t *thr, uint32_t *cnt) {
 
 // FP64 exact scores: 8 lanes per row, FP64 products and sums.
 
-__global__ __launch_bounds__(ACC_WG) void spmv_fp64(const uint32_t *ptr, const int32_t *idx, const float *val,
+__global__ __launch_bounds__(ACC_WG) void spmv_fp64(const uint32_t *ptr, const colx_t *idx, const float *val,
                                                     const float *x, int rows, double *y) {
     const int lane8 = threadIdx.x & 7;
     for (int r = (blockIdx.x * ACC_WG + threadIdx.x) >> 3; r < ((rows + 31) & ~31); r += (gridDim.x * ACC_WG) >> 3) {
         double p = 0.0;
         if (r < rows)
-            for (uint32_t j = ptr[r] + lane8; j < ptr[r + 1]; j += 8) p += (double)val[j] * (double)x[idx[j]];
+            for (uint32_t j = ptr[r] + lane8; j < ptr[r + 1]; j += 8) p += (double)val[j] * (double)x_at(x, idx[j]);
         for (int s = 4; s >= 1; s >>= 1) p += __shfl_xor(p, s);
         if (r < rows && lane8 == 0) y[r] = p;
     }
 }
 
 
-spmv_fn get_fp32_spmv(int G) {
+template <int G>
+static spmv_fn spmv_for(int B) {
+    switch (B) {
+        case 1: return fp32_spmv<G, 1>;
+        case 2: return fp32_spmv<G, 2>;
+        case 3: return fp32_spmv<G, 3>;
+        case 4: return fp32_spmv<G, 4>;
+        case 6: return fp32_spmv<G, G == 32 ? 6 : 4>;
+        default: return nullptr;
+    }
+}
+
+// LDS of an fp32_spmv<G, B> workgroup: x, then each wavefront's staging area.
+size_t fp32_spmv_lds(int cols, int G, int B) {
+    const size_t np = (size_t)(B * (64 / G)) / 64 + 1;
+    return (((size_t)cols * 4 + 15) & ~(size_t)15) + ACC_WAVES * ((size_t)kFp32Area * 6 + np * 256);
+}
+
+spmv_fn get_fp32_spmv(int G, int B) {
     switch (G) {
-        case 2: return fp32_spmv<2, 4>;
-        case 4: return fp32_spmv<4, 4>;
-        case 8: return fp32_spmv<8, 4>;
-        case 16: return fp32_spmv<16, 2>;
-        case 32: return fp32_spmv<32, 2>;
+        case 2: return spmv_for<2>(B);
+        case 4: return spmv_for<4>(B);
+        case 8: return spmv_for<8>(B);
+        case 16: return spmv_for<16>(B);
+        case 32: return spmv_for<32>(B);
         default: return nullptr;
     }
 }

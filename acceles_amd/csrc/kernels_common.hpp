@@ -174,12 +174,18 @@ __device__ inline void publish_and_append(WaveTopM<R> &col, uint64_t *thr, uint3
     for (int i = lane; i < keep; i += 64) dst[pos + i] = col.buf[i];
 }
 
+// Column of an FP32 CSR entry on the device: the byte offset of its x value,
+// 4 * column (cols <= 8192), so that an entry is 6 bytes instead of 8 and the
+// offset addresses x without a shift.
+typedef uint16_t colx_t;
+__device__ __forceinline__ float x_at(const float *x, uint32_t c) { return *(const float *)((const char *)x + c); }
+
 // Dot product of CSR row r with x by a group of G lanes (runtime G): lane g
 // sums entries g, g+G, ... with fmaf, then an xor butterfly of plain adds.
 // Entries are fetched U at a time (then their x values), so a row costs one
 // memory round trip per U*G entries; the fmaf order does not depend on U.
 template <int U = 4>
-__device__ __forceinline__ float group_dot_rt(const uint32_t *ptr, const int32_t *idx, const float *val, const float *x,
+__device__ __forceinline__ float group_dot_rt(const uint32_t *ptr, const colx_t *idx, const float *val, const float *x,
                                               int r, bool valid, int G) {
     const int g = lane_id() & (G - 1);
     float p = 0.f;
@@ -187,7 +193,7 @@ __device__ __forceinline__ float group_dot_rt(const uint32_t *ptr, const int32_t
         const uint32_t e = ptr[r + 1];
         for (uint32_t j = ptr[r] + g; j < e; j += U * G) {
             float v[U], xv[U];
-            int32_t c[U];
+            uint32_t c[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 // clamped into the row (j < e): unconditional loads issue
@@ -197,7 +203,7 @@ __device__ __forceinline__ float group_dot_rt(const uint32_t *ptr, const int32_t
                 c[u] = idx[jj];
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
+            for (int u = 0; u < U; ++u) xv[u] = x_at(x, c[u]);
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 if (j + u * G < e) p = __builtin_fmaf(v[u], xv[u], p);
@@ -213,7 +219,7 @@ __device__ __forceinline__ float group_dot_rt(const uint32_t *ptr, const int32_t
 // Each row is summed in the order of group_dot_rt (entries g, g+G, ... with
 // fmaf, then the butterfly), so the results are the same floats.
 template <int C, int U = 4>
-__device__ __forceinline__ void group_dot_ranges_multi(const int32_t *idx, const float *val, const float *x,
+__device__ __forceinline__ void group_dot_ranges_multi(const colx_t *idx, const float *val, const float *x,
                                                        const uint32_t (&lo)[C], const uint32_t (&hi)[C], int G,
                                                        float (&out)[C]) {
     const int g = lane_id() & (G - 1);
@@ -230,7 +236,7 @@ __device__ __forceinline__ void group_dot_ranges_multi(const int32_t *idx, const
         for (int c = 0; c < C; ++c) any = any || b[c] + o < e[c];
         if (!any) break;
         float v[C][U], xv[C][U];
-        int32_t cl[C][U];
+        uint32_t cl[C][U];
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             // clamped into the matrix (some row has entries while the loop
@@ -246,7 +252,7 @@ __device__ __forceinline__ void group_dot_ranges_multi(const int32_t *idx, const
 #pragma unroll
         for (int c = 0; c < C; ++c)
 #pragma unroll
-            for (int u = 0; u < U; ++u) xv[c][u] = x[cl[c][u]];
+            for (int u = 0; u < U; ++u) xv[c][u] = x_at(x, cl[c][u]);
 #pragma unroll
         for (int c = 0; c < C; ++c)
 #pragma unroll
@@ -261,7 +267,7 @@ __device__ __forceinline__ void group_dot_ranges_multi(const int32_t *idx, const
 // group_dot_ranges_multi for rows r[c] (r[c] is a row of the matrix also for
 // invalid candidates, so the bound loads are unconditional and issue together).
 template <int C, int U = 4>
-__device__ __forceinline__ void group_dot_rt_multi(const uint32_t *ptr, const int32_t *idx, const float *val,
+__device__ __forceinline__ void group_dot_rt_multi(const uint32_t *ptr, const colx_t *idx, const float *val,
                                                    const float *x, const int32_t (&r)[C],
                                                    const bool (&valid)[C], int G, float (&out)[C]) {
     uint32_t lo[C], hi[C];
@@ -514,7 +520,7 @@ struct LowbitArgs {
     int cols, col_bits, val_bits;
     int split, M;               // partitions, rows kept per partition
     const uint32_t *ptr;        // FP32 CSR for rescoring
-    const int32_t *idx;
+    const colx_t *idx;
     const float *val;
     int G;
     uint64_t *resc;             // split * M rescored keys
@@ -573,7 +579,7 @@ struct BatchArgs {
     int32_t *S;                  // nq x nslots INT32 scores
     int split, M;
     const uint32_t *ptr;         // FP32 CSR for rescoring
-    const int32_t *idx;
+    const colx_t *idx;
     const float *val;
     int G;
     uint64_t *resc;              // nq x split*M rescored keys
@@ -650,7 +656,7 @@ struct DenseArgs {
     uint32_t *tk;                // nq x nslices x 4 keys
     int split, M;
     const uint32_t *ptr;         // FP32 CSR for rescoring
-    const int32_t *idx;
+    const colx_t *idx;
     const float *val;
     int G;
     uint64_t *resc;              // nq x split*M rescored keys
@@ -668,18 +674,20 @@ typedef void (*lowbit_fn)(LowbitArgs);
 typedef void (*scores_fn)(ScoresArgs);
 typedef void (*select_fn)(SelectArgs);
 typedef void (*batch_fn)(BatchArgs);
-typedef void (*spmv_fn)(const uint32_t *, const int32_t *, const float *, const float *, int, int, float *);
+typedef void (*spmv_fn)(const uint32_t *, const colx_t *, const float *, const float *, int, int, float *);
 typedef void (*reset_fn)(uint64_t *, uint32_t *);
 typedef void (*radix_pass_fn)(const void *, int64_t, int, uint64_t *);
 typedef void (*radix_final_fn)(const uint64_t *, int, int, acc_element *);
-typedef void (*fp64_fn)(const uint32_t *, const int32_t *, const float *, const float *, int, double *);
+typedef void (*fp64_fn)(const uint32_t *, const colx_t *, const float *, const float *, int, double *);
 
 lowbit_fn get_lowbit_slicemax(int E, bool is_signed);  // k_lowbit.hip
 lowbit_fn get_lowbit_select(int E, bool is_signed);
 lowbit_fn get_lowbit_final(int R);
 lowbit_fn get_lowbit_final_radix();
 scores_fn get_lowbit_scores(int E, bool is_signed);
-spmv_fn get_fp32_spmv(int G);                         // k_fp32.hip
+spmv_fn get_fp32_spmv(int G, int B);                  // k_fp32.hip
+int fp32_step_blocks(int G, double mean_row);          // B of a matrix
+size_t fp32_spmv_lds(int cols, int G, int B);
 select_fn get_select_blocks(int R);
 select_fn get_select_final(int R);
 radix_pass_fn get_select_radix_pass(bool keys, int V);  // k_fp32.hip
