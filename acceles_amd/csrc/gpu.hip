@@ -553,6 +553,10 @@ size_t radix_select_keys(int64_t n, int K) {
     return total;
 }
 
+// Keys of an FP32 query's selection buffer: the radix passes', or the two
+// largest of every wavefront's rows.
+size_t fp32_sel_keys(int64_t rows) { return std::max<size_t>(radix_select_keys(rows, 256), 2 * kMaxGroups); }
+
 // Radix Top-K (K <= 256) of n scores; buf holds radix_select_keys(n, K) keys.
 int launch_select_radix(const float *y, int64_t n, int K, uint64_t *buf, acc_element *out, hipStream_t st,
                         acc_gpu_matrix *prof) {
@@ -767,7 +771,7 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         TRY(dalloc(m, &m->d_sthr, 1));
         TRY(dalloc(m, &m->d_scnt, 1));
         TRY(dalloc(m, &m->d_scand, (size_t)m->sel_blocks * kMaxK));
-        m->rsel_cap = radix_select_keys(m->rows, 256);
+        m->rsel_cap = fp32_sel_keys(m->rows);
         TRY(dalloc(m, &m->d_rsel, m->rsel_cap));
         ZERO(m->d_sthr, 8);
         ZERO(m->d_scnt, 4);
@@ -1066,40 +1070,97 @@ extern "C" int acc_gpu_spmv_fp64(acc_gpu_matrix *m, const float *x_dev, double *
 // FP32 CSR path
 // ---------------------------------------------------------------------------
 
-static int launch_spmv_fp32(acc_gpu_matrix *m, const float *x_dev, float *y, hipStream_t st) {
+// Launch shape of fp32_spmv for a matrix.
+struct SpmvShapeH {
+    spmv_fn fn = nullptr;
+    size_t lds = 0;
+    int blocks = 1, RS = 1;  // workgroups; rows per step
+    int64_t steps = 0;
+};
+
+static int spmv_shape(acc_gpu_matrix *m, SpmvShapeH &h) {
     const int B = fp32_step_blocks(m->group, m->rows > 0 ? (double)m->nnz / m->rows : 0.0);
-    spmv_fn k = get_fp32_spmv(m->group, B);
-    if (!k) return fail(ACC_ERR_ARG, "unsupported group size");
-    const int step_rows = B * (64 / m->group);
-    const int64_t steps = ((int64_t)m->rows + step_rows - 1) / step_rows;
+    h.fn = get_fp32_spmv(m->group, B);
+    if (!h.fn) return fail(ACC_ERR_ARG, "unsupported group size");
+    h.RS = B * (64 / m->group);
+    h.steps = ((int64_t)m->rows + h.RS - 1) / h.RS;
     // as many workgroups as run at once (a second wave of workgroups would leave part of the chip idle
     // at the end), fewer for small matrices
-    const size_t lds = fp32_spmv_lds(m->cols, m->group, B);
+    h.lds = fp32_spmv_lds(m->cols, m->group, B);
     int occ = 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *)k, ACC_WG, lds) != hipSuccess || occ < 1)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *)h.fn, ACC_WG, h.lds) != hipSuccess || occ < 1)
         occ = 1;
-    const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((steps + ACC_WAVES - 1) / ACC_WAVES, (int64_t)m->cus * occ));
-    int rc = lds_limit((const void *)k, lds);
-    if (rc != ACC_OK) return rc;
-    LAUNCH(m, 0, k, dim3(blocks), dim3(ACC_WG), lds, st, m->d_ptr, m->d_idx, m->d_val, x_dev, m->rows, m->cols, y);
+    h.blocks = (int)std::max<int64_t>(
+        1, std::min<int64_t>((h.steps + ACC_WAVES - 1) / ACC_WAVES, std::min<int64_t>((int64_t)m->cus * occ, kMaxGroups / ACC_WAVES)));
+    return lds_limit((const void *)h.fn, h.lds);
+}
+
+static int launch_spmv_fp32(acc_gpu_matrix *m, const SpmvShapeH &h, const float *x_dev, float *y, uint64_t *gmax,
+                            hipStream_t st) {
+    LAUNCH(m, 0, h.fn, dim3(h.blocks), dim3(ACC_WG), h.lds, st, m->d_ptr, m->d_idx, m->d_val, x_dev, m->rows, m->cols,
+           y, gmax);
     return check_launch();
+}
+
+// State of an FP32 Top-K query: the handle's or a plan's.
+struct Fp32State {
+    float *y;
+    uint64_t *rsel;  // radix keys, or the groups' largest keys
+    size_t rcap;
+    uint64_t *thr;
+    uint32_t *cnt;
+    uint64_t *cand;
+};
+
+// FP32 Top-K query: SpMV, then the selection from its groups' largest keys
+// where at least K groups hold rows, else the general selection (radix passes,
+// sorted lists above K = 256) over all scores.  between (optional) is recorded
+// after the SpMV.
+static int launch_fp32_topk(acc_gpu_matrix *m, const float *x_dev, int K, const Fp32State &w, acc_element *out,
+                            hipStream_t st, bool prof, hipEvent_t between = nullptr) {
+    SpmvShapeH h;
+    int rc = spmv_shape(m, h);
+    if (rc != ACC_OK) return rc;
+    const int nw = h.blocks * ACC_WAVES;
+    const bool groups = std::min<int64_t>(h.steps, nw) >= K;
+    rc = launch_spmv_fp32(m, h, x_dev, w.y, groups ? w.rsel : nullptr, st);
+    if (rc == ACC_OK && between && hipEventRecord(between, st) != hipSuccess) rc = fail(ACC_ERR_DEVICE, "hipEventRecord failed");
+    if (rc != ACC_OK) return rc;
+    if (!groups)
+        return launch_select(w.y, m->rows, K, m->sel_blocks, m->sel_chunk, w.thr, w.cnt, w.cand, out, st,
+                             prof ? m : nullptr, w.rsel, w.rcap);
+    SelectGroupsArgs a;
+    a.gmax = w.rsel;
+    a.nw = nw;
+    a.gsteps = (int)((h.steps + nw - 1) / nw);
+    a.RS = h.RS;
+    a.y = w.y;
+    a.rows = m->rows;
+    a.K = K;
+    a.out = out;
+    const select_groups_fn f = get_select_groups(nw);
+    if ((rc = lds_limit((const void *)f, select_groups_lds() + 20480)) != ACC_OK) return rc;
+    LAUNCH(prof ? m : nullptr, 1, f, dim3(1), dim3(1024), select_groups_lds(), st, a);
+    return check_launch();
+}
+
+static Fp32State fp32_state(acc_gpu_matrix *m) {
+    return {m->d_y, m->d_rsel, m->rsel_cap, m->d_sthr, m->d_scnt, m->d_scand};
 }
 
 extern "C" int acc_gpu_spmv_fp32(acc_gpu_matrix *m, const float *x_dev, float *y_dev, void *stream) {
     if (!m || !m->has_csr || !x_dev || !y_dev) return fail(ACC_ERR_ARG, "bad arguments");
     HIP_TRY(hipSetDevice(m->device));
-    return launch_spmv_fp32(m, x_dev, y_dev, (hipStream_t)stream);
+    SpmvShapeH h;
+    int rc = spmv_shape(m, h);
+    return rc == ACC_OK ? launch_spmv_fp32(m, h, x_dev, y_dev, nullptr, (hipStream_t)stream) : rc;
 }
 
 extern "C" int acc_gpu_topk_fp32(acc_gpu_matrix *m, const float *x_dev, int k, acc_element *out_dev, void *stream) {
     if (!m || !m->has_csr) return fail(ACC_ERR_ARG, "matrix was uploaded without the FP32 CSR");
     if (!x_dev || !out_dev || k < 1 || k > kMaxK) return fail(ACC_ERR_ARG, "k must be in [1, 960]");
     HIP_TRY(hipSetDevice(m->device));
-    hipStream_t st = (hipStream_t)stream;
-    int rc = launch_spmv_fp32(m, x_dev, m->d_y, st);
-    if (rc != ACC_OK) return rc;
-    return launch_select(m->d_y, m->rows, k, m->sel_blocks, m->sel_chunk, m->d_sthr, m->d_scnt, m->d_scand,
-                         out_dev, st, m, m->d_rsel, m->rsel_cap);
+    return launch_fp32_topk(m, x_dev, k, fp32_state(m), out_dev, (hipStream_t)stream, true);
 }
 
 extern "C" int acc_gpu_set_profiling(acc_gpu_matrix *m, int enable) {
@@ -1354,7 +1415,7 @@ static int plan_enqueue(acc_plan *p, bool upload_k, hipStream_t st) {
         case ACC_PLAN_LOWBIT_BATCH:
             return run_batch(m, p->ws, p->x, p->nq, p->k.data(), upload_k, p->kmax, p->ck, p->out, p->out_stride, st);
         case ACC_PLAN_FP32: {
-            const size_t rcap = radix_select_keys(m->rows, 256);
+            const size_t rcap = fp32_sel_keys(m->rows);
             BatchWs &w = p->ws;
             const bool fresh = w.sthr == nullptr;
             int rc = ws_grow(w, &w.y, &w.y_n, (size_t)m->rows);
@@ -1369,10 +1430,8 @@ static int plan_enqueue(acc_plan *p, bool upload_k, hipStream_t st) {
                 hipLaunchKernelGGL(get_select_reset(), dim3(1), dim3(64), 0, st, w.sthr, w.scnt);
                 rc = check_launch();
             }
-            if (rc == ACC_OK) rc = launch_spmv_fp32(m, p->x, w.y, st);
             if (rc != ACC_OK) return rc;
-            return launch_select(w.y, m->rows, p->kmax, m->sel_blocks, m->sel_chunk, w.sthr, w.scnt, w.scand, p->out,
-                                 st, nullptr, w.rsel, rcap);
+            return launch_fp32_topk(m, p->x, p->kmax, {w.y, w.rsel, rcap, w.sthr, w.scnt, w.scand}, p->out, st, false);
         }
         default:
             return fail(ACC_ERR_ARG, "unknown plan kind");
@@ -1505,11 +1564,7 @@ extern "C" int acc_top_k_spmv(acc_gpu_matrix *A, int row, int col, int k, int nu
             rc = fail(ACC_ERR_DEVICE, "query upload failed");
             break;
         }
-        rc = launch_spmv_fp32(A, A->d_xstage, A->d_y, nullptr);
-        if (rc == ACC_OK && hipEventRecord(ev[1], nullptr) != hipSuccess) rc = fail(ACC_ERR_DEVICE, "hipEventRecord failed");
-        if (rc == ACC_OK)
-            rc = launch_select(A->d_y, A->rows, k, A->sel_blocks, A->sel_chunk, A->d_sthr, A->d_scnt, A->d_scand,
-                               A->d_ostage, nullptr, nullptr, A->d_rsel, A->rsel_cap);
+        rc = launch_fp32_topk(A, A->d_xstage, k, fp32_state(A), A->d_ostage, nullptr, false, ev[1]);
         if (rc != ACC_OK) break;
         float a = 0.f, b = 0.f;
         if (hipEventRecord(ev[2], nullptr) != hipSuccess || hipEventSynchronize(ev[2]) != hipSuccess ||

@@ -1,10 +1,14 @@
 // k_fp32.hip -- plain FP32 CSR path and FP64 exact scores:
 //   fp32_spmv       FP32 CSR SpMV (cpu_mkl_baseline.cpp:261);
+//   fp32_select_groups
+//                   Top-K of its scores (cpu_mkl_baseline.cpp:128-149) from
+//                   the two best keys of each wavefront's rows; together they
+//                   are the plain FP32 CSR Top-K path
+//                   (host_spmv_topk_csr_gpu.cu:171-231 is the GPU spec);
 //   select_radix_pass / select_radix_final (K <= 256),
 //   select_blocks / select_final (any K <= 960)
-//                   Top-K of a score vector (cpu_mkl_baseline.cpp:128-149);
-//                   with fp32_spmv it is the plain FP32 CSR Top-K path
-//                   (host_spmv_topk_csr_gpu.cu:171-231 is the GPU spec);
+//                   Top-K of any score vector, and of a matrix with fewer
+//                   than K wavefronts' worth of rows;
 //   spmv_fp64       FP64 exact scores for precision/recall reporting.
 #include "kernels_common.hpp"
 
@@ -86,18 +90,20 @@ struct SpmvShape {
 // B of a matrix of this mean row length: a mean step fills at most 85% of the
 // staging area (row lengths vary; 75% and 95%, i.e. two and four blocks
 // instead of three, were slower at 2,000,000 x 900: 145 and 188 against 141
-// us), at most 4 blocks (6 of the two-row blocks of G = 32) so that a step's
+// us), at most 4 blocks, so that a step's
 // registers leave five wavefronts per SIMD.
 int fp32_step_blocks(int G, double mean_row) {
     const double per_block = std::max(mean_row, 1.0) * (64 / G);
-    const int fit = (int)std::min(6.0, 0.85 * kFp32Stage / per_block);
-    if (G == 32 && fit >= 6) return 6;
-    return fit >= 4 ? 4 : fit >= 3 ? 3 : fit >= 2 ? 2 : 1;
+    return std::max(1, (int)std::min(4.0, 0.85 * kFp32Stage / per_block));
 }
 
+// With gmax, wavefront w also leaves the two largest ranking keys of its rows
+// (gmax[w] and gmax[wavefronts + w], 0 without such a row) for
+// fp32_select_groups.  A key of 1 stands for a score whose order is 0 or 1 (a
+// NaN of all ones).
 template <int G, int B>
 __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const colx_t *idx, const float *val,
-                                                   const float *x, int rows, int cols, float *y) {
+                                                   const float *x, int rows, int cols, float *y, uint64_t *gmax) {
     using S = SpmvShape<G, B>;
     constexpr int RPI = S::RPI, RS = S::RS, NP = S::NP, U = S::U, kTail = S::kTail;
     static_assert(U * G <= kFp32Slack, "a batch stays in the slack");
@@ -124,7 +130,12 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
     __syncthreads();
     const int nsteps = (int)(((int64_t)rows + RS - 1) / RS);
     const int gw = blockIdx.x * ACC_WAVES + wave, nw = gridDim.x * ACC_WAVES;
-    if (gw >= nsteps) return;
+    if (gw >= nsteps) {
+        if (gmax && lane < 2) gmax[(size_t)lane * nw + gw] = 0ull;
+        return;
+    }
+    // the two best scores (ordered) and their rows of this lane so far
+    uint32_t top = 0u, toprow = 0u, sec = 0u, secrow = 0u;
 
     typedef uint32_t v4 __attribute__((ext_vector_type(4)));
     constexpr int NV = (kFp32Stage + 255) / 256, NC = (kFp32Stage + 511) / 512;
@@ -272,6 +283,12 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
             p[t] = butterfly<G>(p[t]);
             const int64_t r = (int64_t)s * RS + t * RPI + grp;
             if (g == 0 && r < rows) y[r] = p[t];
+            // rows ascend, so an equal score keeps the lower row
+            const uint32_t o = g == 0 && r < rows ? max(dordered_f32(p[t]), 1u) : 0u;
+            secrow = o > top ? toprow : o > sec ? (uint32_t)r : secrow;
+            sec = max(sec, min(top, o));
+            toprow = o > top ? (uint32_t)r : toprow;
+            top = max(top, o);
         }
         if (!more) break;
         s += nw;
@@ -282,7 +299,221 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
             pn[i] = pf[i];
         }
     }
+    if (gmax) {
+        uint64_t best[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t m = wave_umax(top);
+            const uint32_t lo = wave_umax(top == m ? 0xFFFFFFFFu - toprow : 0u);
+            best[i] = m <= 1u ? (uint64_t)m : ((uint64_t)m << 32) | lo;
+            if (top == m && 0xFFFFFFFFu - toprow == lo) {  // one lane: rows are distinct
+                top = sec;
+                toprow = secrow;
+            }
+        }
+        if (lane < 2) gmax[(size_t)lane * nw + gw] = lane == 0 ? best[0] : best[1];
+    }
 }
+
+// Top-K (K <= 960) of the scores y from the two largest keys of each
+// wavefront's rows (a group; one workgroup): T, the K-th largest of the groups'
+// best keys, is reached by K distinct rows, so every row of the Top-K has a
+// key >= T and lies in one of the K groups whose best reaches it.  Their best
+// keys, and their second ones that reach T, are listed in LDS; only a group
+// whose second key reaches T can hold more such rows and is read from y (the
+// steps are dealt in turn, so neighbouring rows lie in different groups and
+// few groups are read).  The listed keys are ranked.  A list that does not fit
+// (an order of rows that puts most of the best ones into the same groups) is
+// cut by a radix selection over the rows of the K groups.
+//
+// Bound: latency, and what one CU reads: at 2,000,000 rows and K = 100 it
+// takes 20 us, reading all K groups' rows took 53 (12 GB/s of scattered rows).
+// Before it, two radix passes over all scores and a final one took 32 us, and
+// above K = 256 the sorted lists of select_blocks and select_final 827 us
+// (4,999,999 rows, K = 500; 22 us here).
+static constexpr int kSelList = 4096;  // keys listed in LDS
+
+template <int V>
+__global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ uint32_t hist[512];
+    __shared__ uint64_t s_t[2];
+    __shared__ int s_need[2], s_n, s_m, s_scans;
+    __shared__ uint32_t s_group[1024], s_scan[1024];  // groups that reach T; those to read
+    __shared__ uint64_t s_below[1024];                // and the key below which their rows are not listed yet
+    uint64_t *s_key = (uint64_t *)smem, *s_top = s_key + kSelList;  // kSelList, then 1024 keys
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const uint32_t nw = (uint32_t)a.nw, RS = (uint32_t)a.RS, rows = (uint32_t)a.rows;
+    uint64_t k[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) k[u] = a.gmax[min((uint32_t)(tid + u * 1024), nw - 1u)];
+#pragma unroll
+    for (int u = 0; u < V; ++u)
+        if ((uint32_t)(tid + u * 1024) >= nw) k[u] = 0ull;
+    if (tid == 0) {
+        s_n = 0;
+        s_m = 0;
+        s_scans = 0;
+    }
+    const uint64_t T = wg_radix_kth<uint64_t>(
+        [&](auto fn) {
+#pragma unroll
+            for (int u = 0; u < V; ++u) fn(k[u]);
+        },
+        a.K, hist, s_t, s_need);
+    // fewer than K groups with rows, or keys of 1 among the best: every group is read
+    const bool all = T <= 1ull;
+    auto append = [&](uint64_t key) {
+        const int j = atomicAdd(&s_n, 1);
+        if (j < kSelList) s_key[j] = key;
+    };
+    if (!all) {
+#pragma unroll
+        for (int u = 0; u < V; ++u)
+            if (k[u] >= T) {
+                append(k[u]);
+                const int j = atomicAdd(&s_m, 1);
+                if (j < 1024) s_group[j] = (uint32_t)(tid + u * 1024);  // K of them: the keys are distinct
+            }
+        __syncthreads();
+        if (tid < min(s_m, 1024)) {
+            const uint32_t w = s_group[tid];
+            const uint64_t second = a.gmax[nw + w];
+            if (second >= T) {
+                append(second);
+                const int j = atomicAdd(&s_scans, 1);
+                s_scan[j] = w;
+                s_below[j] = second;
+            }
+        }
+    }
+    __syncthreads();
+    // fn(key) for every row of groups group(0 .. nl-1) (0: no row).  A
+    // wavefront reads C groups together, U rows per lane and group; the rows'
+    // places in a group are the same for all groups.
+    const uint32_t L = (uint32_t)a.gsteps * RS;  // rows of a group
+    auto scan_by = [&](auto uu, auto cc, int nl, auto group, auto fn) {
+        constexpr int U = decltype(uu)::value, C = decltype(cc)::value;
+        for (uint32_t j0 = 0; j0 < L; j0 += 64 * U) {
+            uint32_t off[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t j = j0 + u * 64 + lane, st = j / RS;
+                off[u] = j < L ? st * nw * RS + (j - st * RS) : 0xFFFFFFFFu;
+            }
+            for (int c0 = wave * C; c0 < nl; c0 += 16 * C) {
+                float v[C][U];
+                uint32_t row[C][U];
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const uint32_t b = group(min(c0 + c, nl - 1)) * RS;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        row[c][u] = c0 + c < nl && off[u] != 0xFFFFFFFFu ? b + off[u] : 0xFFFFFFFFu;
+                        v[c][u] = a.y[min(row[c][u], rows - 1u)];
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        fn(row[c][u] < rows ? dkey_f32(v[c][u], (int32_t)row[c][u]) : 0ull, min(c0 + c, nl - 1));
+            }
+        }
+    };
+    auto scan = [&](int nl, auto group, auto fn) {
+        if (L <= 64) scan_by(std::integral_constant<int, 1>(), std::integral_constant<int, 8>(), nl, group, fn);
+        else scan_by(std::integral_constant<int, 8>(), std::integral_constant<int, 2>(), nl, group, fn);
+    };
+    if (!all)
+        scan(
+            s_scans, [&](int i) { return s_scan[i]; },
+            [&](uint64_t key, int i) {
+                if (key >= T && key < s_below[i]) append(key);
+            });
+    __syncthreads();
+    if (all || s_n > kSelList) {
+        // all rows of the groups that reach T (of every group): their K best
+        const int nl = all ? (int)nw : min(s_m, 1024);
+        auto group = [&](int i) { return all ? (uint32_t)i : s_group[i]; };
+        __syncthreads();
+        if (tid == 0) s_n = 0;
+        const uint64_t cut = wg_radix_kth<uint64_t>(
+            [&](auto fn) { scan(nl, group, [&](uint64_t key, int) { fn(key); }); }, a.K, hist, s_t, s_need);
+        scan(nl, group, [&](uint64_t key, int) {
+            if (key != 0ull && key >= cut) append(key);
+        });
+        __syncthreads();
+    }
+    int n = min(s_n, kSelList);
+    if (n > 1024) {  // keep the best K
+        const uint64_t cut = wg_radix_kth<uint64_t>(
+            [&](auto fn) {
+                for (int i = tid; i < n; i += 1024) fn(s_key[i]);
+            },
+            a.K, hist, s_t, s_need);
+        if (tid == 0) s_n = 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += 1024)
+            if (s_key[i] >= cut) {
+                const int j = atomicAdd(&s_n, 1);
+                if (j < 1024) s_top[j] = s_key[i];
+            }
+        __syncthreads();
+        n = min(s_n, 1024);
+        if (tid < n) s_key[tid] = s_top[tid];
+        __syncthreads();
+    }
+    const uint64_t key = tid < n ? s_key[tid] : 0ull;
+    int rank = 0;
+    if (n <= 256) {  // ranks by counting, two keys per read
+        if (tid < 2) s_key[n + tid] = 0ull;
+        __syncthreads();
+        if (tid < n)
+            for (int j = 0; j < n; j += 2) {
+                const ulonglong2 o = *(const ulonglong2 *)(s_key + j);
+                rank += (o.x > key) + (o.y > key);
+            }
+    } else {  // each wavefront sorts its keys; a key's rank: its places in the sorted lists
+        uint64_t v[1] = {key};
+        reg_sort_desc<1>(v);
+        s_top[tid] = v[0];
+        __syncthreads();
+        rank = lane;
+        for (int w = 0; w * 64 < n; ++w) {
+            if (w == wave) continue;
+            int lo = 0, hi = 64;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (s_top[w * 64 + mid] > v[0]) lo = mid + 1;
+                else hi = mid;
+            }
+            rank += lo;
+        }
+        const uint64_t mine = v[0];
+        if (mine != 0ull && rank < a.K) {
+            acc_element e;
+            e.value = dkey_score_f32(mine);
+            e.index = dkey_row(mine);
+            a.out[rank] = e;
+        }
+    }
+    if (n <= 256 && tid < n && rank < a.K) {
+        acc_element e;
+        e.value = dkey_score_f32(key);
+        e.index = dkey_row(key);
+        a.out[rank] = e;
+    }
+    for (int i = n + tid; i < a.K; i += 1024) {
+        acc_element e;
+        e.value = -__builtin_inff();
+        e.index = -1;
+        a.out[i] = e;
+    }
+}
+
+select_groups_fn get_select_groups(int nw) { return nw <= 2048 ? fp32_select_groups<2> : fp32_select_groups<8>; }
+size_t select_groups_lds() { return (size_t)(kSelList + 1024) * 8; }
 
 
 template <int R>
@@ -430,7 +661,6 @@ static spmv_fn spmv_for(int B) {
         case 2: return fp32_spmv<G, 2>;
         case 3: return fp32_spmv<G, 3>;
         case 4: return fp32_spmv<G, 4>;
-        case 6: return fp32_spmv<G, G == 32 ? 6 : 4>;
         default: return nullptr;
     }
 }

@@ -554,6 +554,18 @@ struct SelectArgs {
     acc_element *out;
 };
 
+// Top-K of the scores an fp32_spmv launch of nw wavefronts has just written,
+// from the two largest keys of each wavefront's rows (steps w, w + nw, ... of
+// wavefront w, at most gsteps, of RS rows each).
+static constexpr int kMaxGroups = 8192;
+struct SelectGroupsArgs {
+    const uint64_t *gmax;  // 2 * nw keys
+    int nw, gsteps, RS;
+    const float *y;
+    int rows, K;
+    acc_element *out;
+};
+
 // ---------------------------------------------------------------------------
 // batched low-bit path: a block of QB queries per matrix pass
 // ---------------------------------------------------------------------------
@@ -674,7 +686,8 @@ typedef void (*lowbit_fn)(LowbitArgs);
 typedef void (*scores_fn)(ScoresArgs);
 typedef void (*select_fn)(SelectArgs);
 typedef void (*batch_fn)(BatchArgs);
-typedef void (*spmv_fn)(const uint32_t *, const colx_t *, const float *, const float *, int, int, float *);
+typedef void (*spmv_fn)(const uint32_t *, const colx_t *, const float *, const float *, int, int, float *, uint64_t *);
+typedef void (*select_groups_fn)(SelectGroupsArgs);
 typedef void (*reset_fn)(uint64_t *, uint32_t *);
 typedef void (*radix_pass_fn)(const void *, int64_t, int, uint64_t *);
 typedef void (*radix_final_fn)(const uint64_t *, int, int, acc_element *);
@@ -688,6 +701,8 @@ scores_fn get_lowbit_scores(int E, bool is_signed);
 spmv_fn get_fp32_spmv(int G, int B);                  // k_fp32.hip
 int fp32_step_blocks(int G, double mean_row);          // B of a matrix
 size_t fp32_spmv_lds(int cols, int G, int B);
+select_groups_fn get_select_groups(int nw);
+size_t select_groups_lds();
 select_fn get_select_blocks(int R);
 select_fn get_select_final(int R);
 radix_pass_fn get_select_radix_pass(bool keys, int V);  // k_fp32.hip

@@ -718,7 +718,7 @@ def main():
         f"; {sc_kernel} {bs_gbs:.0f} GB/s, {bs_tops:.1f} TOP/s int8")
     log(f"[bench] single: slicemax {lb_ms[0] * 1e3:.1f}us ({s1_gbs:.0f} GB/s), select {lb_ms[1] * 1e3:.1f}us, "
         f"final {lb_ms[2] * 1e3:.1f}us; fp32 spmv {fp_ms[0] * 1e3:.1f}us ({fp32_spmv_gbs:.0f} GB/s), "
-        f"select {fp_ms[1] * 1e3:.1f}us + {fp_ms[2] * 1e3:.1f}us")
+        f"select {' + '.join(f'{v * 1e3:.1f}us' for v in fp_ms[1:])}")
 
     # ---- accuracy vs FP64 exact Top-K ----
     y64 = acc.DeviceBuffer((a.rows,), np.float64)

@@ -274,8 +274,8 @@ int acc_gpu_matrix_info(const acc_gpu_matrix *m, acc_gpu_info_t *info);
  * kernel's own start and end); acc_gpu_stage_times waits for the last query
  * and returns up to n kernel durations in ms (low-bit: slice maxima, select
  * + rescoring, final Top-K; batched packets: scores, select, final; batched
- * matrix cores: prep, scores, select + rescoring, final; FP32: SpMV, select,
- * final select) and their count. */
+ * matrix cores: prep, scores, select + rescoring, final; FP32: SpMV, then one
+ * select, or two where fewer wavefronts than k have rows) and their count. */
 int acc_gpu_set_profiling(acc_gpu_matrix *m, int enable);
 int acc_gpu_stage_times(acc_gpu_matrix *m, float *ms, int n, int *count);
 

@@ -48,3 +48,46 @@ def test_spmv_bitexact(acc, gpu, kind, cols):
     g.spmv_fp32(acc.DeviceBuffer.from_numpy(x), y)
     acc.synchronize()
     np.testing.assert_array_equal(y.numpy(), O.spmv_f32(ptr, idx, val, x, g.info.group))
+
+
+def topk_both(acc, csr, ptr, idx, val, x, k):
+    g = acc.GpuMatrix(csr)
+    got = g.topk_fp32_host(x, k)
+    rows, vals = O.topk(O.spmv_f32(ptr, idx, val, x, g.info.group), k)
+    m = min(k, csr.rows)
+    np.testing.assert_array_equal(got["index"][:m], rows[:m])
+    np.testing.assert_array_equal(got["value"][:m], np.asarray(vals[:m], np.float32))
+    assert (got["index"][m:] == -1).all() and np.isneginf(got["value"][m:]).all()
+
+
+# one row per step and group, groups of a few rows, of several steps; K below, at and above the ranking by counting
+@pytest.mark.parametrize("rows,deg", [(977, (50, 90)), (20011, (50, 90)), (130001, (10, 30)), (700001, (1, 6))])
+@pytest.mark.parametrize("k", [1, 100, 256, 257, 960])
+def test_topk_from_groups(acc, gpu, rows, deg, k):
+    csr = acc.CSRMatrix.generate(rows, 300, deg=deg, val_kind=acc.VAL_NORMAL, seed=rows + k)
+    topk_both(acc, csr, *csr.arrays(), acc.generate_queries(1, 300, seed=k)[0], k)
+
+
+# "zeros": every score ties; "same_group": the best rows lie in the same groups (more than the LDS list holds);
+# "levels": a handful of score levels
+@pytest.mark.parametrize("kind", ["zeros", "levels", "same_group", "infinite"])
+@pytest.mark.parametrize("k", [3, 100, 700])
+def test_topk_ties_and_clusters(acc, gpu, kind, k):
+    rows, cols = 400000, 64
+    rng = np.random.default_rng(k)
+    ptr = np.arange(rows + 1, dtype=np.int64)
+    idx = rng.integers(0, cols, rows).astype(np.int32)
+    val = np.ones(rows, np.float32)
+    x = np.ones(cols, np.float32)
+    if kind == "zeros":
+        x[:] = 0.0
+    elif kind == "levels":
+        val = rng.integers(-3, 3, rows).astype(np.float32)
+    elif kind == "same_group":
+        # steps of 128 rows (two lanes per row, four blocks): every 16th step scores high
+        val = np.where(np.arange(rows) // 128 % 16 == 5, rng.random(rows) + 10, rng.random(rows)).astype(np.float32)
+    else:
+        val[rng.integers(0, rows, 50)] = np.inf
+        val[rng.integers(0, rows, 50)] = -np.inf
+    csr = acc.CSRMatrix.from_arrays(rows, cols, ptr, idx, val)
+    topk_both(acc, csr, ptr, idx, val, x, k)
