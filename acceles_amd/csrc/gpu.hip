@@ -10,7 +10,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -761,8 +760,13 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         TRY(dalloc(m, &m->d_y, (size_t)m->rows));
         COPY(m->d_ptr, p32.data(), p32.size() * 4);
         {
-            const std::unique_ptr<uint16_t[]> cx = acc::column_offsets(csr);
-            COPY(m->d_idx, cx.get(), (size_t)nnz * sizeof(colx_t));
+            // converted and copied a piece at a time: the piece stays in the cache and its pages are touched once
+            std::vector<uint16_t> cx((size_t)std::min<int64_t>(nnz, 1 << 20));
+            for (int64_t b = 0; b < nnz; b += (int64_t)cx.size()) {
+                const int64_t n = std::min<int64_t>(nnz - b, (int64_t)cx.size());
+                acc::column_offsets(csr->idx.data() + b, n, cx.data());
+                COPY(m->d_idx + b, cx.data(), (size_t)n * sizeof(colx_t));
+            }
         }
         COPY(m->d_val, csr->val.data(), (size_t)nnz * 4);
         ZERO(m->d_idx + nnz, 8 * sizeof(colx_t));

@@ -355,14 +355,9 @@ extern "C" int acc_csr_create(int32_t rows, int32_t cols, int64_t nnz, const int
     return ACC_OK;
 }
 
-std::unique_ptr<uint16_t[]> acc::column_offsets(const acc_csr *csr) {
-    const int64_t n = csr->nnz();
-    std::unique_ptr<uint16_t[]> out(new uint16_t[(size_t)std::max<int64_t>(n, 1)]);
-    const int32_t *idx = csr->idx.data();
-    uint16_t *o = out.get();
-#pragma omp parallel for schedule(static)
-    for (int64_t i = 0; i < n; ++i) o[i] = (uint16_t)(idx[i] * 4);
-    return out;
+void acc::column_offsets(const int32_t *idx, int64_t n, uint16_t *out) {
+#pragma omp parallel for schedule(static) if (n > (1 << 18))
+    for (int64_t i = 0; i < n; ++i) out[i] = (uint16_t)(idx[i] * 4);
 }
 
 extern "C" int acc_csr_info(const acc_csr *m, int32_t *rows, int32_t *cols, int64_t *nnz) {

@@ -4,7 +4,6 @@
 #include "../../include/acceles.h"
 
 #include <cstdint>
-#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -63,8 +62,8 @@ inline uint32_t ordered_f32(float f) {
 
 int bits_for(int32_t n);  // ceil(log2(n)), at least 1
 
-// 4 * column of every entry (cols <= 8192): the columns as the device reads them.
-std::unique_ptr<uint16_t[]> column_offsets(const acc_csr *csr);
+// 4 * column of n entries (cols <= 8192): the columns as the device reads them.
+void column_offsets(const int32_t *idx, int64_t n, uint16_t *out);
 
 // Batched low-bit queries with a workspace of the caller's (acc_gpu_topk_
 // lowbit_batch uses the handle's own, so one handle runs one batch at a
