@@ -71,6 +71,23 @@ __device__ __forceinline__ int32_t wave_max_lane63(int32_t v) {
     return v;
 }
 
+// Inclusive prefix sum over the wavefront (DPP row shifts, then the row 15 /
+// row 31 broadcasts: eight VALU steps against six LDS shuffles).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_add_step(uint32_t v) {
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t v) {
+    // shifts by 1, 2, 4 and 8 inside the 16-lane rows (lanes without a source add 0)
+    v = dpp_add_step<0x111, 0xF>(v);
+    v = dpp_add_step<0x112, 0xF>(v);
+    v = dpp_add_step<0x114, 0xF>(v);
+    v = dpp_add_step<0x118, 0xF>(v);
+    v = dpp_add_step<0x142, 0xA>(v);
+    v = dpp_add_step<0x143, 0xC>(v);
+    return v;
+}
+
 // The m-th largest (m >= 1, with repeats) of the U values per lane of the
 // wavefront (0 = no value; returns 0 when fewer than m are nonzero), by
 // sorting each lane's values in registers and then extracting the wavefront

@@ -290,7 +290,7 @@ int launch_lowbit_stage(acc_gpu_matrix *m, const LowbitArgs &a, int stage, hipSt
         if (rc != ACC_OK) return rc;
         LAUNCH(m, 1, ksel, dim3(m->split), dim3(SEL_WG), lds_sel, st, a);
     } else if (a.K <= 256 && m->split * a.M <= 4 * SEL_WG) {
-        LAUNCH(m, 2, get_lowbit_final_radix(), dim3(1), dim3(SEL_WG), 0, st, a);
+        LAUNCH(m, 2, get_lowbit_final_radix((m->split * a.M + SEL_WG - 1) / SEL_WG), dim3(1), dim3(SEL_WG), 0, st, a);
     } else {
         const int R = pow2_at_least((m->split * a.M + ACC_WG - 1) / ACC_WG);  // split*M <= kMaxCK = 4*64*16
         lowbit_fn f = get_lowbit_final(R);

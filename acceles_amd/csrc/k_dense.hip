@@ -547,7 +547,7 @@ __global__ __launch_bounds__(ACC_WG) void batch_topk(DenseArgs a) {
 // key, then ranks by counting.
 template <int V>
 __global__ __launch_bounds__(ACC_WG) void batch_topk_radix(DenseArgs a) {
-    __shared__ __align__(16) uint32_t lds[1032];
+    __shared__ __align__(16) uint32_t lds[1036];
     const int q = blockIdx.x;
     const int total = a.split * a.M;
     topk_radix<V>(a.resc + (size_t)q * total, total, a.K[q], a.out + (size_t)q * a.out_stride, lds);

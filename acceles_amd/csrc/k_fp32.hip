@@ -327,10 +327,10 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
 // cut by a radix selection over the rows of the K groups.
 //
 // Bound: latency, and what one CU reads: at 2,000,000 rows and K = 100 it
-// takes 20 us, reading all K groups' rows took 53 (12 GB/s of scattered rows).
+// takes 17 us, reading all K groups' rows took 53 (12 GB/s of scattered rows).
 // Before it, two radix passes over all scores and a final one took 32 us, and
 // above K = 256 the sorted lists of select_blocks and select_final 827 us
-// (4,999,999 rows, K = 500; 22 us here).
+// (4,999,999 rows, K = 500; 20 us here).
 static constexpr int kSelList = 4096;  // keys listed in LDS
 
 template <int V>
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(ACC_WG) void select_radix_pass(const void *in, int6
 
 template <int V>
 __global__ __launch_bounds__(1024) void select_radix_final(const uint64_t *cand, int total, int K, acc_element *out) {
-    __shared__ __align__(16) uint32_t lds[1032];
+    __shared__ __align__(16) uint32_t lds[1036];
     topk_radix<V>(cand, total, K, out, lds);
 }
 

@@ -416,10 +416,11 @@ __global__ __launch_bounds__(ACC_WG) void lowbit_final(LowbitArgs a) {
     topk_by_rank<R>(a.resc, a.split * a.M, a.K, a.out, (uint64_t *)smem, s_nz);
 }
 
-// The same for K <= 256 by radix selection (split*M <= 4*SEL_WG).
+// The same for K <= 256 by radix selection (split*M <= V*SEL_WG).
+template <int V>
 __global__ __launch_bounds__(SEL_WG) void lowbit_final_radix(LowbitArgs a) {
-    __shared__ __align__(16) uint32_t lds[1032];
-    topk_radix<4>(a.resc, a.split * a.M, a.K, a.out, lds);
+    __shared__ __align__(16) uint32_t lds[1036];
+    topk_radix<V>(a.resc, a.split * a.M, a.K, a.out, lds);
 }
 
 // INT32 scores of every row (one work item per wavefront).
@@ -485,7 +486,9 @@ lowbit_fn get_lowbit_slicemax(int E, bool is_signed) {
     return is_signed ? slicemax_for<true>(E) : slicemax_for<false>(E);
 }
 lowbit_fn get_lowbit_select(int E, bool is_signed) { return is_signed ? select_for<true>(E) : select_for<false>(E); }
-lowbit_fn get_lowbit_final_radix() { return lowbit_final_radix; }
+lowbit_fn get_lowbit_final_radix(int V) {
+    return V <= 1 ? lowbit_final_radix<1> : V <= 2 ? lowbit_final_radix<2> : lowbit_final_radix<4>;
+}
 lowbit_fn get_lowbit_final(int R) {
     switch (R) {
         case 1: return lowbit_final<1>;

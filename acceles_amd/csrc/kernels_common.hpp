@@ -348,6 +348,9 @@ __device__ inline void topk_by_rank(const uint64_t *keys, int total, int K, acc_
 
 // The need-th largest of the nonzero keys the workgroup's threads offer
 // (each thread calls fn(key) for its keys through for_each(fn); 0 = no key).
+// Bound: latency (barriers and LDS round trips): wavefront reductions by DPP
+// instead of LDS shuffles took lowbit_final_radix (512 keys) from 6.2 to 4.4
+// us and batch_topk_radix from 5.6 to 4.5.
 // First the keys' range: the bits above the highest bit in which the
 // smallest and largest key differ are common to all keys.  Then digit by
 // digit (8 bits) below them: an LDS histogram of the keys that share the
@@ -364,39 +367,33 @@ __device__ T wg_radix_kth(F for_each, int need, uint32_t *hist, T *s_t, int *s_n
     constexpr int NB = 8 * (int)sizeof(T);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     for (int i = tid; i < 256; i += blockDim.x) hist[i] = 0u;
-    if (tid == 0) {
-        s_t[0] = ~(T)0;
-        s_t[1] = (T)0;
-    }
-    T lo = ~(T)0, hi = 0;
+    // range of the keys' high words (DPP maxima; a 64-bit range would take 24
+    // LDS shuffles): of 64-bit keys that share it, all low bits count
+    uint32_t *s_range = (uint32_t *)s_t;  // ~smallest, largest
+    if (tid < 2) s_range[tid] = 0u;
+    uint32_t nlo = 0u, hi32 = 0u;  // both stay 0 without a key
     for_each([&](T k) {
         if (k != 0) {
-            lo = k < lo ? k : lo;
-            hi = k > hi ? k : hi;
+            const uint32_t h = sizeof(T) == 8 ? (uint32_t)((uint64_t)k >> 32) : (uint32_t)k;
+            nlo = max(nlo, ~h);
+            hi32 = max(hi32, h);
         }
     });
-    for (int o = 32; o > 0; o >>= 1) {
-        T ol, oh;
-        if constexpr (sizeof(T) == 8) {
-            ol = shfl_xor_u64(lo, o);
-            oh = shfl_xor_u64(hi, o);
-        } else {
-            ol = (T)__shfl_xor((int)lo, o);
-            oh = (T)__shfl_xor((int)hi, o);
-        }
-        lo = ol < lo ? ol : lo;
-        hi = oh > hi ? oh : hi;
+    nlo = wave_umax(nlo);
+    hi32 = wave_umax(hi32);
+    __syncthreads();
+    if (lane == 0 && (nlo | hi32) != 0u) {
+        atomicMax(&s_range[0], nlo);
+        atomicMax(&s_range[1], hi32);
     }
     __syncthreads();
-    if (lane == 0 && hi != 0) {
-        atomicMin(&s_t[0], lo);
-        atomicMax(&s_t[1], hi);
-    }
-    __syncthreads();
-    lo = s_t[0];
-    hi = s_t[1];
-    if (hi == 0) return (T)0;
-    int bits = lo == hi ? 1 : NB - (sizeof(T) == 8 ? __builtin_clzll((uint64_t)(lo ^ hi)) : __builtin_clz((uint32_t)(lo ^ hi)));
+    nlo = s_range[0];
+    hi32 = s_range[1];
+    if ((nlo | hi32) == 0u) return (T)0;
+    const uint32_t diff = ~nlo ^ hi32;
+    int bits = diff ? 32 - __builtin_clz(diff) : sizeof(T) == 8 ? 0 : 1;
+    if (sizeof(T) == 8) bits += 32;
+    const T hi = sizeof(T) == 8 ? (T)((uint64_t)hi32 << 32) : (T)hi32;
     T prefix = bits >= NB ? (T)0 : (T)(hi >> bits);  // the common high bits
     int rem = need;
     for (int pass = 0; bits > 0; ++pass) {
@@ -413,12 +410,7 @@ __device__ T wg_radix_kth(F for_each, int need, uint32_t *hist, T *s_t, int *s_n
 #pragma unroll
             for (int j = 0; j < 4; ++j) c[j] = h[255 - 4 * lane - j];  // lane 0 holds the top bins
             const uint32_t sum = c[0] + c[1] + c[2] + c[3];
-            uint32_t inc = sum;
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t t = __shfl_up(inc, o);
-                if (lane >= o) inc += t;
-            }
-            uint32_t above = inc - sum;
+            uint32_t above = wave_prefix_sum(sum) - sum;
             if (lane == 0) s_need[0] = -1;  // stays when fewer than rem keys share the prefix
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -445,7 +437,7 @@ __device__ T wg_radix_kth(F for_each, int need, uint32_t *hist, T *s_t, int *s_n
 // The K <= 256 best of total <= V * blockDim.x ranking keys (0 = empty)
 // into out[0, K), then (value -inf, index -1) past the nonzero keys: radix
 // selection of the K-th key, then each selected key's rank by counting the
-// selected keys above it.  lds: 4128 bytes (histogram, state, 256 keys).
+// selected keys above it.  lds: 4144 bytes (histogram, state, 257 keys).
 template <int V>
 __device__ inline void topk_radix(const uint64_t *keys, int total, int K, acc_element *out, uint32_t *lds) {
     uint32_t *hist = lds;
@@ -457,9 +449,12 @@ __device__ inline void topk_radix(const uint64_t *keys, int total, int K, acc_el
     uint64_t k[V];
 #pragma unroll
     for (int u = 0; u < V; ++u) {
-        const int i = tid + u * (int)blockDim.x;
-        k[u] = i < total ? keys[i] : 0ull;
+        // clamped, masked after: the loads issue together (total >= 1)
+        k[u] = keys[min(tid + u * (int)blockDim.x, total - 1)];
     }
+#pragma unroll
+    for (int u = 0; u < V; ++u)
+        if (tid + u * (int)blockDim.x >= total) k[u] = 0ull;
     if (tid == 0) *s_n = 0;
     const uint64_t T = wg_radix_kth<uint64_t>(
         [&](auto fn) {
@@ -480,10 +475,15 @@ __device__ inline void topk_radix(const uint64_t *keys, int total, int K, acc_el
     }
     __syncthreads();
     const int n = min(*s_n, 256);  // min(K, nonzero keys)
+    if (tid == 0) s_sel[n] = 0ull;  // the list is read two keys at a time
+    __syncthreads();
     if (tid < n) {
         const uint64_t key = s_sel[tid];
         int rank = 0;
-        for (int j = 0; j < n; ++j) rank += s_sel[j] > key;
+        for (int j = 0; j < n; j += 2) {
+            const ulonglong2 o = *(const ulonglong2 *)(s_sel + j);
+            rank += (o.x > key) + (o.y > key);
+        }
         acc_element e;
         e.value = dkey_score_f32(key);
         e.index = dkey_row(key);
@@ -696,7 +696,7 @@ typedef void (*fp64_fn)(const uint32_t *, const colx_t *, const float *, const f
 lowbit_fn get_lowbit_slicemax(int E, bool is_signed);  // k_lowbit.hip
 lowbit_fn get_lowbit_select(int E, bool is_signed);
 lowbit_fn get_lowbit_final(int R);
-lowbit_fn get_lowbit_final_radix();
+lowbit_fn get_lowbit_final_radix(int V);  // V = 1, 2, 4
 scores_fn get_lowbit_scores(int E, bool is_signed);
 spmv_fn get_fp32_spmv(int G, int B);                  // k_fp32.hip
 int fp32_step_blocks(int G, double mean_row);          // B of a matrix
