@@ -41,6 +41,15 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// Workgroup barrier for LDS only: waits for this wavefront's LDS operations,
+// not for its global loads (a full barrier would also wait for the packet
+// loads issued for the slices ahead).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Maximum over the wavefront, valid in lane 63 (DPP steps: quad swaps,
 // half-row and row mirrors, then the row 15 / row 31 broadcasts).
 template <int CTRL, int ROWS>

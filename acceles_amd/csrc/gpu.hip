@@ -27,6 +27,11 @@ static constexpr int kMaxM = 64;     // rows kept per partition
 static constexpr int kMaxK = 960;    // Top-K limit of the FP32 path (collector cap 1024)
 static constexpr int kMaxCK = 4096;  // candidates of the low-bit path
 static constexpr size_t kWordPad = 32 * 64;  // dwords past the packets (>= widest group of 32 entries)
+// Single queries keep three scores per slice up to this many slices: they cost
+// the streaming pass 12 us at 312,500 slices (20,000,000 rows: 146 -> 159 us)
+// and save the selection about 5 us whatever the size (400,000 rows: 15.1 ->
+// 10.0 us), so they pay up to some 100,000 slices.
+static constexpr int64_t kTop3Slices = 65536;
 static constexpr int kPkMaxCols = 1024;  // matrix-core scores: B operands of 32 column blocks in registers
 static constexpr int kPkMinE = 18, kPkMaxE = 23;  // image-packet entry widths instantiated for them
 static constexpr size_t kPkLdsMax = 160 * 1024;  // LDS of a pk_scores workgroup at most
@@ -51,8 +56,8 @@ struct BatchWs {
     size_t corr_n = 0;
     uint32_t *tk = nullptr;      // four-key slice lists
     size_t tk_n = 0;
-    int32_t *smax = nullptr;     // single-query passes: slice maxima
-    size_t smax_n = 0;
+    int4 *stop = nullptr;        // single-query passes: slices' largest scores
+    size_t stop_n = 0;
     float *y = nullptr;          // FP32 plans: scores
     size_t y_n = 0;
     uint64_t *rsel = nullptr;    // FP32 plans: radix selection keys
@@ -93,7 +98,7 @@ struct acc_gpu_matrix {
     int4 *d_items = nullptr;         // per workgroup
     int nitems = 0;
     std::vector<int32_t> part_row_begin;
-    int32_t *d_smax = nullptr;       // per slice: largest INT32 score of the last query
+    int4 *d_stop = nullptr;          // per slice: the largest INT32 scores of the last query
     uint64_t *d_resc = nullptr;      // split * kMaxM
     int32_t *d_crow = nullptr, *d_cscore = nullptr;  // split * kMaxM (candidate outputs)
     int64_t *d_part_slice = nullptr;                 // split + 1
@@ -247,7 +252,7 @@ int lds_limit(const void *fn, size_t bytes);
 // Top-K into out (K > 0) and/or the per-partition candidates into
 // crow/cscore (p*M + i).
 LowbitArgs lowbit_args(acc_gpu_matrix *m, const float *x, int M, int K, acc_element *out, int32_t *crow,
-                       int32_t *cscore, int32_t *smax = nullptr, uint64_t *resc = nullptr) {
+                       int32_t *cscore, int4 *stop = nullptr, uint64_t *resc = nullptr) {
     LowbitArgs a;
     a.words = m->d_words;
     a.slices = m->d_slices;
@@ -255,7 +260,8 @@ LowbitArgs lowbit_args(acc_gpu_matrix *m, const float *x, int M, int K, acc_elem
     a.items = m->d_items;
     a.part_slice = m->d_part_slice;
     a.nvalid = m->d_nvalid;
-    a.smax = smax ? smax : m->d_smax;
+    a.stop = stop ? stop : m->d_stop;
+    a.top3 = m->nslices <= kTop3Slices ? 1 : 0;
     a.x = x;
     a.cols = m->cols;
     a.col_bits = m->col_bits;
@@ -277,16 +283,15 @@ LowbitArgs lowbit_args(acc_gpu_matrix *m, const float *x, int M, int K, acc_elem
 // Launches stage i of a low-bit query: 0 slice maxima, 1 per-partition
 // select + rescoring, 2 final Top-K (a.K > 0).
 int launch_lowbit_stage(acc_gpu_matrix *m, const LowbitArgs &a, int stage, hipStream_t st) {
-    const size_t qlds = (size_t)((m->cols + 15) & ~15);
     if (stage == 0) {
         lowbit_fn k = get_lowbit_slicemax(m->entry_bits, m->is_signed != 0);
         if (!k) return fail(ACC_ERR_ARG, "unsupported entry width");
-        LAUNCH(m, 0, k, dim3(m->nitems), dim3(LB_WG), 64 + qlds, st, a);
+        LAUNCH(m, 0, k, dim3(m->nitems), dim3(LB_WG), 0, st, a);
     } else if (stage == 1) {
         lowbit_fn ksel = get_lowbit_select(m->entry_bits, m->is_signed != 0);
         if (!ksel) return fail(ACC_ERR_ARG, "unsupported entry width");
-        const size_t lds_sel = 64 + 8 * 4096 + 5 * qlds;         // key list, int8 and FP32 query
-        int rc = lds_limit((const void *)ksel, lds_sel + 40960);  // plus about 36 KB static
+        const size_t lds_sel = 64 + 8 * 4096 + 4 * (size_t)((m->cols + 15) & ~15);  // key list, FP32 query
+        int rc = lds_limit((const void *)ksel, lds_sel + 49152);                    // plus about 44 KB static
         if (rc != ACC_OK) return rc;
         LAUNCH(m, 1, ksel, dim3(m->split), dim3(SEL_WG), lds_sel, st, a);
     } else if (a.K <= 256 && m->split * a.M <= 4 * SEL_WG) {
@@ -305,11 +310,11 @@ int launch_lowbit_stage(acc_gpu_matrix *m, const LowbitArgs &a, int stage, hipSt
 int launch_lowbit(acc_gpu_matrix *m, const float *x, int M, int K, acc_element *out, int32_t *crow, int32_t *cscore,
                   hipStream_t st, BatchWs *ws = nullptr) {
     if (ws) {
-        int rc = ws_grow(*ws, &ws->smax, &ws->smax_n, (size_t)m->nslices);
+        int rc = ws_grow(*ws, &ws->stop, &ws->stop_n, (size_t)m->nslices);
         if (rc == ACC_OK) rc = ws_grow(*ws, &ws->resc, &ws->resc_n, (size_t)m->split * kMaxM);
         if (rc != ACC_OK) return rc;
     }
-    const LowbitArgs a = lowbit_args(m, x, M, K, out, crow, cscore, ws ? ws->smax : nullptr, ws ? ws->resc : nullptr);
+    const LowbitArgs a = lowbit_args(m, x, M, K, out, crow, cscore, ws ? ws->stop : nullptr, ws ? ws->resc : nullptr);
     int rc = launch_lowbit_stage(m, a, 0, st);
     if (rc == ACC_OK) rc = launch_lowbit_stage(m, a, 1, st);
     if (rc == ACC_OK && K > 0) rc = launch_lowbit_stage(m, a, 2, st);
@@ -802,7 +807,7 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         TRY(dalloc(m, &m->d_slices, sl.size()));
         TRY(dalloc(m, &m->d_perm, pk->perm.size()));
         TRY(dalloc(m, &m->d_items, items.size()));
-        TRY(dalloc(m, &m->d_smax, (size_t)m->nslices));
+        TRY(dalloc(m, &m->d_stop, (size_t)m->nslices));
         TRY(dalloc(m, &m->d_resc, (size_t)m->split * kMaxM));
         TRY(dalloc(m, &m->d_crow, (size_t)m->split * kMaxM));
         TRY(dalloc(m, &m->d_cscore, (size_t)m->split * kMaxM));
@@ -1035,7 +1040,7 @@ extern "C" int acc_gpu_scores_lowbit(acc_gpu_matrix *m, const float *x_dev, int3
     scores_fn k = get_lowbit_scores(m->entry_bits, m->is_signed != 0);
     if (!k) return fail(ACC_ERR_ARG, "unsupported entry width");
     int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((m->nslices + ACC_WAVES - 1) / ACC_WAVES, m->cus * 8));
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(ACC_WG), 64 + (size_t)((m->cols + 15) & ~15), (hipStream_t)stream, a);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(ACC_WG), 0, (hipStream_t)stream, a);
     return check_launch();
 }
 

@@ -2,11 +2,13 @@
 //   lowbit_slicemax  query quantization (quantify_util.py:31-49, 259) and the
 //                    INT32 scores of the sliced packets (quantify_util.py:5-6,
 //                    173-196; spmv_ucsr_top_k_multicore.hpp:195-355 on the
-//                    FPGA); only the maximum of each 64-row slice is written;
-//   lowbit_select    per partition: threshold = its M-th best slice maximum
-//                    (M distinct rows reach it, so no row below it can be in
-//                    the partition's Top-M), exact rescan of the slices whose
-//                    maximum reaches it, Top-M (quantify_util.py:173-196,
+//                    FPGA); only the three largest of each 64-row slice (with
+//                    many slices: the largest) are written;
+//   lowbit_select    per partition: threshold = about its M-th best slice
+//                    maximum (M distinct rows reach it, so no row below it can
+//                    be in the partition's Top-M), the listed rows that reach
+//                    it, exact rescan of the slices whose list may have
+//                    dropped one, Top-M (quantify_util.py:173-196,
 //                    host_spmv_ucsr.cpp:691-748) and FP32 rescoring of those
 //                    rows (quantify_util.py:354-367);
 //   lowbit_final_radix / lowbit_final
@@ -16,34 +18,63 @@
 // occupancy with nothing but loads, decode and one wavefront max per slice.
 #include "kernels_common.hpp"
 
+#include <type_traits>
+
 template <int E, bool SIGNED>
-__device__ __forceinline__ int32_t slice_score(const LowbitArgs &a, const uint2 sl, const int8_t *qx, uint32_t cmask) {
+__device__ __forceinline__ int32_t slice_score(const LowbitArgs &a, const uint2 sl, const int8_t *qx) {
     const __amdgpu_buffer_rsrc_t rs = slice_rsrc(a.words, sl);
     int32_t acc = 0;
     for (int g0 = 0; g0 < (int)sl.y; g0 += E) {
         uint32_t w[E];
         load_group<E>(w, rs, g0);
-        acc = decode_group<E, SIGNED>(w, min(E, (int)sl.y - g0), qx, a.col_bits, a.val_bits, cmask, acc);
+        acc = decode_group<E, SIGNED>(w, min(E, (int)sl.y - g0), qx, a.col_bits, a.val_bits, acc);
     }
     return acc;
 }
 
-// Work item blockIdx.x (a slice range of one partition): smax[s] = the
-// largest INT32 score over the 64 lanes of slice s.  Padding lanes of a
-// partition's last slice score 0, so that slice's maximum may be too high;
-// lowbit_select only uses full slices for its threshold.
+// The three largest of the lanes' scores and the lanes of the first two:
+// (first, second, third, lane of first | lane of second << 8), in every lane.
+__device__ __forceinline__ int4 top3(int32_t v) {
+    const int lane = lane_id();
+    int32_t m[3];
+    int l[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        m[i] = __builtin_amdgcn_readlane(wave_max_lane63(v), 63);
+        if (i < 2) {
+            l[i] = __builtin_ctzll(__ballot(v == m[i]));
+            v = lane == l[i] ? INT32_MIN : v;
+        }
+    }
+    return make_int4(m[0], m[1], m[2], l[0] | (l[1] << 8));
+}
+
+// Work item blockIdx.x (a slice range of one partition): stop[s] = the three
+// largest INT32 scores over the 64 lanes of slice s and the first two's
+// lanes.  Padding lanes of a partition's last slice score 0, so that slice's
+// may be too high; lowbit_select rescans it.  Without top3 only the largest
+// is known, and lowbit_select rescans every slice that it needs.
+//
+// Bound: HBM (20,000,000 x 1024: 146 us, 6.4 TB/s of packets; 159 before the
+// decode took four instructions per entry instead of six and the loads stayed
+// in flight).  Small matrices: latency (400,000 x 500: 12.4 us, 13.4 before
+// the first packets were loaded ahead of the query's quantization).
 template <int E, bool SIGNED>
 __global__ __launch_bounds__(LB_WG) void lowbit_slicemax(LowbitArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ __align__(16) int8_t qx[kMaxCols];
     __shared__ uint2 s_meta[LB_MAX_ITEM];
-    float *red = (float *)smem;
-    int8_t *qx = (int8_t *)(smem + 64);
+    __shared__ float red[LB_WAVES];
     const int4 item = a.items[blockIdx.x];
-    for (int i = threadIdx.x; i < item.z - item.y; i += LB_WG) s_meta[i] = a.slices[item.y + i];
-    quantize_query_lds(a.x, a.cols, qx, red);  // its barriers also publish s_meta
-
-    const int wave = threadIdx.x >> 6, lane = lane_id();
-    const uint32_t cmask = (1u << a.col_bits) - 1u;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
+    // in order of use: the slices' metadata (into LDS) and the query, then the
+    // first packets, whose latency covers the query's quantization (they
+    // need the metadata of the wave's first two slices only, read here)
+    const int nit = item.z - item.y;
+    const uint2 m0 = a.slices[item.y + min((int)threadIdx.x, nit - 1)];
+    float xr[kQueryRegs];
+    load_query(a.x, a.cols, xr);
+    const uint2 sl0 = a.slices[min(item.y + wave, item.z - 1)], sl1 = a.slices[min(item.y + wave + LB_WAVES, item.z - 1)];
+    __builtin_amdgcn_sched_barrier(0);
     // Groups (E dwords per lane) of the wave's slices item.y + wave,
     // + LB_WAVES, ... stream through a ring of three register slots, two
     // groups ahead of the decoder.  Every load of the loop is unconditional
@@ -57,8 +88,10 @@ __global__ __launch_bounds__(LB_WG) void lowbit_slicemax(LowbitArgs a) {
     int ds[RING], dnd[RING];
     bool dend[RING], dval[RING];
     int ls = item.y + wave, lg = 0;  // load cursor
-    uint2 lsl = ls < item.z ? s_meta[ls - item.y] : make_uint2(0u, 0u);
-    auto issue = [&](int slot) {
+    uint2 lsl = ls < item.z ? sl0 : make_uint2(0u, 0u);
+    // metadata of slice ls (head: before s_meta is published, at most the wave's second slice)
+    auto meta = [&](bool head) { return ls >= item.z ? make_uint2(0u, 0u) : head ? sl1 : s_meta[ls - item.y]; };
+    auto issue = [&](int slot, bool head) {
         const bool valid = ls < item.z;
         load_group<E>(w[slot], slice_rsrc(a.words, lsl), lg);
         __builtin_amdgcn_sched_barrier(0);  // keep the loads here: the scheduler would sink them to their use
@@ -70,14 +103,19 @@ __global__ __launch_bounds__(LB_WG) void lowbit_slicemax(LowbitArgs a) {
             if (dend[slot]) {
                 ls += LB_WAVES;
                 lg = 0;
-                lsl = ls < item.z ? s_meta[ls - item.y] : make_uint2(0u, 0u);
+                lsl = meta(head);
             } else {
                 lg += E;
             }
         }
     };
-    issue(0);
-    issue(1);
+    issue(0, true);
+    issue(1, true);
+    if ((int)threadIdx.x < nit) s_meta[threadIdx.x] = m0;
+    for (int i = threadIdx.x + LB_WG; i < nit; i += LB_WG) s_meta[i] = a.slices[item.y + i];
+    quantize_query_lds(a.x, a.cols, qx, red, nullptr, xr);  // its barriers also publish s_meta
+    // the second issue may have moved on to the third slice
+    if (ls >= item.y + wave + 2 * LB_WAVES) lsl = meta(false);
     int32_t acc = 0;
     bool done = false;
     while (!done) {
@@ -88,41 +126,42 @@ __global__ __launch_bounds__(LB_WG) void lowbit_slicemax(LowbitArgs a) {
                 done = true;
                 break;
             }
-            // Every loaded dword is read here, also on paths that skip
-            // blocks: a load result that is dead on some path lets its
-            // register be reused while the load is in flight, and the reuse
-            // then waits for all outstanding loads.
-            const int nd = dnd[j];
-            uint32_t wm[E];
-#pragma unroll
-            for (int i = 0; i < E; ++i) wm[i] = i < nd ? w[j][i] : 0u;
-            acc = decode_group<E, SIGNED>(wm, nd, qx, a.col_bits, a.val_bits, cmask, acc);
+            hold_group(w[j]);
+            acc = decode_group<E, SIGNED>(w[j], dnd[j], qx, a.col_bits, a.val_bits, acc);
             if (dend[j]) {
-                const int32_t m = wave_max_lane63(acc);
-                if (lane == 63) a.smax[ds[j]] = m;
+                // without the top three: second and third unknown
+                const int4 t = a.top3 ? top3(acc)
+                                      : make_int4(__builtin_amdgcn_readlane(wave_max_lane63(acc), 63), INT32_MAX, INT32_MAX, 0);
+                if (lane == 0) a.stop[ds[j]] = t;
                 acc = 0;
             }
-            issue((j + 2) % RING);
+            issue((j + 2) % RING, false);
         }
     }
 }
 
 // One workgroup of SEL_WG threads per partition p = blockIdx.x, after
 // lowbit_slicemax.
-// 1. ts = the M-th largest maximum among the partition's full slices (radix
-//    selection): each of those M slices holds a distinct row scoring >= ts,
-//    so every row of the partition's Top-M scores >= ts and lies in a slice
-//    whose maximum is >= ts.
-// 2. The slices whose maximum reaches ts are listed in LDS and rescanned
-//    exactly, CS at a time: their groups are spread over all wavefronts
-//    (kU loads in flight per wavefront) and the partial scores added into
-//    per-slice LDS sums, so long slices do not serialize on one wavefront.
-//    Rows >= ts are appended to an LDS key list, which is cut back to its
-//    best M whenever another chunk might not fit.
-// 3. The list's best M by radix selection, ranked by counting.  Past kList
-//    candidate slices (heavy ties) each wavefront instead rescans its share
-//    slice by slice into a wavefront Top-M collector.
+// 1. ts: a score that M distinct rows reach, about the M-th largest of the
+//    full slices' listed scores (radix selection that stops when at most kSlack
+//    more reach it): every row of the partition's Top-M scores >= ts and lies
+//    in a slice whose largest score is >= ts.
+// 2. Of such a slice the two listed rows that reach ts go to an LDS key list.
+//    If the third score reaches ts too (or the slice is not full), the slice
+//    is rescanned exactly instead, CS slices at a time: their groups are
+//    spread over all wavefronts (kU loads in flight per wavefront) and the
+//    partial scores added into per-slice LDS sums, so long slices do not
+//    serialize on one wavefront; rows >= ts are appended to the key list,
+//    which is cut back to its best M whenever another chunk might not fit.
+// 3. The list's best M (by radix selection past 64), ranked by counting.  Past
+//    kList slices to rescan or KCAP keys (heavy ties) each wavefront instead
+//    rescans its share slice by slice into a wavefront Top-M collector.
 // 4. Optional candidate output and the FP32 rescoring of the M rows.
+//
+// Bound: latency.  400,000 x 500 (196 slices, M = 16 per partition): 9.9 us;
+// 15.1 when every slice that reaches ts was rescanned (16 slices, 5 us of
+// decoding on one CU) after an exact threshold (3.6 us).  999,983 x 250: 9.1
+// (before: 11.9), 20,000 x 500: 11.5 (17.2).
 template <int E, bool SIGNED>
 __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
     constexpr int V = 8;         // slice maxima per thread held in registers
@@ -130,117 +169,116 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
     constexpr int CS = 32;       // candidate slices per rescan chunk
     constexpr int kU = E <= 16 ? 3 : 2;  // groups in flight per wavefront (128 VGPRs at 16 waves)
     constexpr int KCAP = 4096;   // LDS key list (rows >= ts)
+    constexpr int kSlack = 16;   // rows beyond M that may reach ts
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ uint32_t s_hist[512];
+    __shared__ __align__(16) int8_t qx[kMaxCols];
+    __shared__ __align__(16) uint32_t s_hist[512];
     __shared__ int32_t s_list[kList];
-    __shared__ uint2 s_lmeta[kList];
+    __shared__ uint2 s_lmeta[CS];
     __shared__ int32_t s_sum[CS * 64];
     __shared__ int s_ustart[CS + 1];
     __shared__ int s_n[SEL_WAVES];
     __shared__ int s_m, s_cnt, s_kn, s_tn, s_need[2];
     __shared__ uint32_t s_t32[2];
     __shared__ uint64_t s_t64[2];
-    __shared__ uint64_t s_tmp[64], s_top[64];
+    __shared__ __align__(16) uint64_t s_tmp[66], s_top[64];
+    __shared__ uint2 s_rng[64];  // entry ranges of the rows in s_top
     float *red = (float *)smem;
     uint64_t *keys = (uint64_t *)(smem + 64);  // KCAP keys; the slow path's collectors reuse it
-    int8_t *qx = (int8_t *)(smem + 64 + 8 * KCAP);
-    float *xs = (float *)(smem + 64 + 8 * KCAP + ((a.cols + 15) & ~15));  // FP32 query (rescoring)
+    float *xs = (float *)(smem + 64 + 8 * KCAP);  // FP32 query (rescoring)
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int p = blockIdx.x;
     const int64_t s0 = a.part_slice[p];
     const int nsl = (int)(a.part_slice[p + 1] - s0);
-    const int32_t *smax = a.smax + s0;
-    const uint8_t *nvalid = a.nvalid + s0;
-    const uint32_t cmask = (1u << a.col_bits) - 1u;
-    const bool regs = nsl <= V * SEL_WG;
-    int32_t sm[V];
-    bool full[V];
-    if (regs) {
-        // one uniform test around loads with clamped indices: they issue
-        // together (a per-element condition would wait for each load)
-        if (nsl > 0) {
+    const int4 *stop = a.stop + s0;
+    const int32_t *perm = a.perm + s0 * 64;
+    const bool regs = nsl <= V * SEL_WG, one = nsl <= SEL_WG;
+    // the query and the thread's slices; one uniform test around loads with
+    // clamped indices: they issue together (a per-element condition would
+    // wait for each load)
+    float xr[kQueryRegs];
+    load_query(a.x, a.cols, xr);
+    int4 st[V];
+    int32_t r1 = -1, r2 = -1;  // one: the rows of the slice's two best scores
+    auto load = [&](auto n) {
 #pragma unroll
-            for (int u = 0; u < V; ++u) {
-                const int i = min(tid + u * SEL_WG, nsl - 1);
-                sm[u] = smax[i];
-                full[u] = nvalid[i] == 64;
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < V; ++u) {
-                sm[u] = 0;
-                full[u] = false;
-            }
-        }
-    }
+        for (int u = 0; u < V; ++u)
+            st[u] = u < decltype(n)::value ? stop[min(tid + u * SEL_WG, nsl - 1)] : make_int4(0, 0, 0, 0);
+    };
+    if (nsl <= 0 || !regs) load(std::integral_constant<int, 0>());
+    else if (one) load(std::integral_constant<int, 1>());
+    else load(std::integral_constant<int, V>());
+    // every slice is full except a partition's last one
+    const int nfull = nsl <= 0 || a.nvalid[s0 + nsl - 1] == 64 ? nsl : nsl - 1;
     if (tid == 0) {
         s_cnt = 0;
         s_kn = 0;
         s_tn = 0;
     }
-    quantize_query_lds(a.x, a.cols, qx, red, xs);
-
-    // 1. threshold (unsigned order: score ^ 2^31; key 0 = not a full slice):
-    //    up to 256 slices and M <= 32 by maximum extraction in wavefront 0,
-    //    otherwise by radix selection over the workgroup
-    auto mkey = [](int32_t v, bool ok) -> uint32_t { return ok ? ((uint32_t)v ^ 0x80000000u) : 0u; };
-    uint32_t T;
-    if (nsl <= 256 && a.M <= 32) {
-        if (tid < 256) s_hist[tid] = tid < nsl ? mkey(sm[0], full[0]) : 0u;  // regs holds slice tid in sm[0]
-        __syncthreads();
-        if (wave == 0) {
-            uint32_t v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = s_hist[u * 64 + lane];
-            const uint32_t t = wave_kth_u32<4>(v, a.M);
-            if (lane == 0) s_t32[0] = t;
-        }
-        __syncthreads();
-        T = s_t32[0];
-    } else {
-        T = wg_radix_kth<uint32_t>(
-            [&](auto fn) {
-                if (regs) {
-#pragma unroll
-                    for (int u = 0; u < V; ++u) fn(tid + u * SEL_WG < nsl ? mkey(sm[u], full[u]) : 0u);
-                } else {
-                    for (int i = tid; i < nsl; i += SEL_WG) fn(mkey(smax[i], nvalid[i] == 64));
-                }
-            },
-            a.M, s_hist, s_t32, s_need);
+    for (int u = 0; u < kQueryRegs; ++u)
+        if (tid + u * SEL_WG < a.cols) xs[tid + u * SEL_WG] = xr[u];
+    for (int c = tid + kQueryRegs * SEL_WG; c < a.cols; c += SEL_WG) xs[c] = a.x[c];
+    if (one && nsl > 0) {  // in flight while the threshold is computed
+        const int32_t *pr = perm + (size_t)min(tid, nsl - 1) * 64;
+        r1 = pr[st[0].w & 63];
+        r2 = pr[(st[0].w >> 8) & 63];
     }
+
+    // 1. threshold (unsigned order: score ^ 2^31; key 0 = not a full slice).
+    //    Up to SEL_WG slices: their three scores each (a partition of fewer
+    //    than M slices has a threshold too), more: their largest.
+    auto mkey = [](int32_t v, bool ok) -> uint32_t { return ok ? ((uint32_t)v ^ 0x80000000u) : 0u; };
+    const uint32_t T = wg_radix_kth<uint32_t>(
+        [&](auto fn) {
+            if (one) {
+                fn(mkey(st[0].x, tid < nfull));
+                fn(mkey(st[0].y, a.top3 && tid < nfull));
+                fn(mkey(st[0].z, a.top3 && tid < nfull));
+            } else if (regs) {
+#pragma unroll
+                for (int u = 0; u < V; ++u) fn(mkey(st[u].x, tid + u * SEL_WG < nfull));
+            } else {
+                for (int i = tid; i < nsl; i += SEL_WG) fn(mkey(stop[i].x, i < nfull));
+            }
+        },
+        a.M, s_hist, s_t32, s_need, kSlack);
     const int32_t ts = T == 0u ? INT32_MIN : (int32_t)(T ^ 0x80000000u);
 
-    // 2. candidate slices, listed with their metadata
-    auto offer = [&](int i, bool cand) {
-        const uint64_t m = __ballot(cand);
-        if (m == 0) return;
-        const uint2 meta = cand ? a.slices[s0 + i] : make_uint2(0u, 0u);  // in flight during the append
+    // 2. keys of the listed rows, slices to rescan
+    auto slot = [&](int *count, bool ok) -> int {  // places in a list, for the lanes that are ok
+        const uint64_t m = __ballot(ok);
         int base = 0;
-        if (lane == 0) base = atomicAdd(&s_cnt, __popcll(m));
-        base = __shfl(base, 0);
-        const int j = base + mbcnt64(m);
-        if (cand && j < kList) {
-            s_list[j] = i;
-            s_lmeta[j] = meta;
+        if (m != 0ull && lane == 0) base = atomicAdd(count, __popcll(m));
+        return __builtin_amdgcn_readfirstlane(base) + mbcnt64(m);
+    };
+    auto offer = [&](int i, const int4 &t) {
+        const bool cand = i < nsl && t.x >= ts;
+        if (!__any(cand)) return;
+        const bool again = cand && (i >= nfull || t.z >= ts), first = cand && !again, second = first && t.y >= ts;
+        if (__any(again)) {
+            const int j = slot(&s_cnt, again);
+            if (again && j < kList) s_list[j] = i;
         }
+        const int32_t *pr = perm + (size_t)i * 64;
+        const int j1 = slot(&s_kn, first);
+        if (first && j1 < KCAP) keys[j1] = dkey_i32(t.x, one ? r1 : pr[t.w & 63]);
+        if (!__any(second)) return;
+        const int j2 = slot(&s_kn, second);
+        if (second && j2 < KCAP) keys[j2] = dkey_i32(t.y, one ? r2 : pr[(t.w >> 8) & 63]);
     };
     if (regs) {
 #pragma unroll
-        for (int u = 0; u < V; ++u) {
-            const int i = tid + u * SEL_WG;
-            offer(i, i < nsl && sm[u] >= ts);
-        }
+        for (int u = 0; u < V; ++u)
+            if (u * SEL_WG < nsl) offer(tid + u * SEL_WG, st[u]);
     } else {
-        for (int b = 0; b < nsl; b += SEL_WG) {
-            const int i = b + tid;
-            offer(i, i < nsl && smax[min(i, nsl - 1)] >= ts);
-        }
+        for (int b = 0; b < nsl; b += SEL_WG) offer(b + tid, stop[min(b + tid, nsl - 1)]);
     }
-    __syncthreads();
+    lds_barrier();
     const int ncand = s_cnt;
     int mcount = 0;
-    if (ncand <= kList) {
+    if (ncand > 0 || s_kn > KCAP) quantize_query_lds(a.x, a.cols, qx, red, nullptr, xr);
+    if (ncand <= kList && s_kn <= KCAP) {
         // keeps the best M of the key list (all threads; the list is published)
         auto cut = [&](int n) -> int {
             const uint64_t Tk = wg_radix_kth<uint64_t>(
@@ -260,29 +298,27 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
                 const int j = base + mbcnt64(m);
                 if (sel && j < 64) s_tmp[j] = k;  // j < M for distinct keys
             }
-            __syncthreads();
+            lds_barrier();
             const int m = min(s_tn, a.M);
-            __syncthreads();
+            lds_barrier();
             if (tid == 0) s_tn = 0;
             return m;
         };
         for (int cb = 0; cb < ncand; cb += CS) {
             const int cn = min(CS, ncand - cb);
-            __syncthreads();  // metadata listed; the previous chunk's sums and keys in place
+            lds_barrier();  // metadata listed; the previous chunk's sums and keys in place
             if (s_kn > KCAP - CS * 64) {  // the next chunk might not fit: keep the best M
                 const int m = cut(s_kn);
                 if (tid < m) keys[tid] = s_tmp[tid];
                 if (tid == 0) s_kn = m;
-                __syncthreads();
+                lds_barrier();
             }
             for (int i = tid; i < CS * 64; i += SEL_WG) s_sum[i] = 0;
             if (wave == 0) {
-                const int ng = lane < cn ? ((int)s_lmeta[cb + lane].y + E - 1) / E : 0;
-                int inc = ng;
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int t = __shfl_up(inc, o);
-                    if (lane >= o) inc += t;
-                }
+                const uint2 sl = a.slices[s0 + s_list[cb + min(lane, cn - 1)]];
+                if (lane < cn) s_lmeta[lane] = sl;
+                const int ng = lane < cn ? ((int)sl.y + E - 1) / E : 0;
+                const int inc = (int)wave_prefix_sum((uint32_t)ng);
                 if (lane < CS) s_ustart[lane + 1] = inc;
                 if (lane == 0) s_ustart[0] = 0;
             }
@@ -291,10 +327,10 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
 #pragma unroll
             for (int r = 0; r < PR; ++r) {  // unconditional (clamped) lookups, masked after
                 const int c = wave + r * SEL_WAVES;
-                const int32_t v = a.perm[(s0 + s_list[cb + min(c, cn - 1)]) * 64 + lane];
+                const int32_t v = perm[(size_t)s_list[cb + min(c, cn - 1)] * 64 + lane];
                 prow[r] = c < cn ? v : -1;
             }
-            __syncthreads();
+            lds_barrier();
             const int nu = s_ustart[cn];
             for (int u0 = wave * kU; u0 < nu; u0 += SEL_WAVES * kU) {
                 uint32_t w[kU][E];
@@ -313,7 +349,7 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
                         }
                         c = lo;
                         g0 = (u - s_ustart[c]) * E;
-                        sl = s_lmeta[cb + c];
+                        sl = s_lmeta[c];
                     }
                     load_group<E>(w[t], slice_rsrc(a.words, sl), g0);
                     cu[t] = c;
@@ -322,11 +358,11 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
 #pragma unroll
                 for (int t = 0; t < kU; ++t) {
                     if (cu[t] < 0) continue;
-                    const int32_t part = decode_group<E, SIGNED>(w[t], nd[t], qx, a.col_bits, a.val_bits, cmask, 0);
+                    const int32_t part = decode_group<E, SIGNED>(w[t], nd[t], qx, a.col_bits, a.val_bits, 0);
                     atomicAdd(&s_sum[cu[t] * 64 + lane], part);
                 }
             }
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int r = 0; r < PR; ++r) {
                 const int c = wave + r * SEL_WAVES;
@@ -342,49 +378,65 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
         const int nk = s_kn;
-        if (nk <= 64) {  // one wavefront sorts the list (keys are distinct; 0 sorts last)
-            if (wave == 0) {
-                uint64_t w[1] = {lane < nk ? keys[lane] : 0ull};
-                reg_sort_desc<1>(w);
-                if (lane < a.M) s_top[lane] = w[0];
+        const uint64_t *src = keys;  // nk <= 64 keys, or the best M of more
+        int n = nk;
+        if (nk > 64) {
+            n = cut(nk);
+            src = s_tmp;
+        }
+        mcount = min(n, a.M);
+        // rank by counting (keys are distinct), two keys per read; the rows'
+        // entry ranges are in flight meanwhile
+        uint64_t k = 0ull;
+        uint2 rg = make_uint2(0u, 0u);
+        if (tid < n) {
+            k = src[tid];
+            if (a.K > 0) rg = make_uint2(a.ptr[dkey_row(k)], a.ptr[dkey_row(k) + 1]);
+        }
+        if (tid == n) (nk > 64 ? s_tmp : keys)[n] = 0ull;
+        lds_barrier();
+        if (tid < n) {
+            int rank = 0;
+            for (int j = 0; j < n; j += 2) {
+                const ulonglong2 o = *(const ulonglong2 *)(src + j);
+                rank += (o.x > k) + (o.y > k);
             }
-            mcount = min(nk, a.M);
-        } else {
-            mcount = cut(nk);
-            if (tid < mcount) {  // rank by counting (keys are distinct)
-                const uint64_t k = s_tmp[tid];
-                int rank = 0;
-                for (int j = 0; j < mcount; ++j) rank += s_tmp[j] > k;
+            if (rank < a.M) {
                 s_top[rank] = k;
+                s_rng[rank] = rg;
             }
         }
-        __syncthreads();
+        lds_barrier();
     } else {
         uint64_t *colbuf = keys;
         WaveTopM<2> col;
         col.init(colbuf + wave * WaveTopM<2>::cap, a.M);
         for (int b = wave * 64; b < nsl; b += SEL_WG) {
-            uint64_t mask = __ballot(b + lane < nsl && smax[min(b + lane, nsl - 1)] >= ts);
+            uint64_t mask = __ballot(b + lane < nsl && stop[min(b + lane, nsl - 1)].x >= ts);
             while (mask) {
                 const int l = __builtin_ctzll(mask);
                 mask &= mask - 1;
                 const int64_t s = s0 + b + l;
-                const int32_t sc = slice_score<E, SIGNED>(a, a.slices[s], qx, cmask);
+                const int32_t sc = slice_score<E, SIGNED>(a, a.slices[s], qx);
                 const int32_t row = a.perm[s * 64 + lane];
                 col.push(row >= 0 && sc >= ts, dkey_i32(sc, row));
             }
         }
         col.compact();
         if (lane == 0) s_n[wave] = col.n;
-        __syncthreads();
+        lds_barrier();
         if (wave == 0) {
             wg_merge(col, colbuf, s_n, SEL_WAVES);
-            if (lane < col.n) s_top[lane] = col.buf[lane];  // col.n <= M <= 64, sorted
+            if (lane < col.n) {  // col.n <= M <= 64, sorted
+                const uint64_t k = col.buf[lane];
+                s_top[lane] = k;
+                if (a.K > 0) s_rng[lane] = make_uint2(a.ptr[dkey_row(k)], a.ptr[dkey_row(k) + 1]);
+            }
             if (lane == 0) s_m = col.n;
         }
-        __syncthreads();
+        lds_barrier();
         mcount = s_m;
     }
     const uint64_t *top = s_top;
@@ -396,14 +448,15 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
     }
     if (a.K <= 0) return;
 
-    // 4. FP32 rescoring of the partition's candidates (16 entries per lane in
-    //    flight; the query from LDS)
+    // 4. FP32 rescoring of the partition's candidates (8 entries per lane in
+    //    flight: a row has two to four per lane on average; the query from LDS)
     for (int base = 0; base < a.M; base += SEL_WG / a.G) {
         const int i = base + (int)threadIdx.x / a.G;
         const bool valid = i < mcount;
-        const int32_t r = valid ? dkey_row(top[i]) : 0;
-        const float sc = group_dot_rt<16>(a.ptr, a.idx, a.val, xs, r, valid, a.G);
-        if ((threadIdx.x & (a.G - 1)) == 0 && i < a.M) a.resc[(size_t)p * a.M + i] = valid ? dkey_f32(sc, r) : 0ull;
+        const uint2 rg = valid ? s_rng[i] : make_uint2(0u, 0u);
+        const float sc = group_dot_range<8>(a.idx, a.val, xs, rg.x, rg.y, a.G);
+        if ((threadIdx.x & (a.G - 1)) == 0 && i < a.M)
+            a.resc[(size_t)p * a.M + i] = valid ? dkey_f32(sc, dkey_row(top[i])) : 0ull;
     }
 }
 
@@ -427,12 +480,10 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_final_radix(LowbitArgs a) {
 
 template <int E, bool SIGNED>
 __global__ __launch_bounds__(ACC_WG) void lowbit_scores(ScoresArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    float *red = (float *)smem;
-    int8_t *qx = (int8_t *)(smem + 64);
+    __shared__ __align__(16) int8_t qx[kMaxCols];
+    __shared__ float red[ACC_WAVES];
     quantize_query_lds(a.x, a.cols, qx, red);
     const int lane = lane_id();
-    const uint32_t cmask = (1u << a.col_bits) - 1u;
     for (int64_t s = (int64_t)blockIdx.x * ACC_WAVES + (threadIdx.x >> 6); s < a.nslices;
          s += (int64_t)gridDim.x * ACC_WAVES) {
         const uint2 sl = a.slices[s];
@@ -441,7 +492,7 @@ __global__ __launch_bounds__(ACC_WG) void lowbit_scores(ScoresArgs a) {
         for (int g0 = 0; g0 < (int)sl.y; g0 += E) {
             uint32_t w[E];
             load_group<E>(w, rs, g0);
-            acc = decode_group<E, SIGNED>(w, min(E, (int)sl.y - g0), qx, a.col_bits, a.val_bits, cmask, acc);
+            acc = decode_group<E, SIGNED>(w, min(E, (int)sl.y - g0), qx, a.col_bits, a.val_bits, acc);
         }
         const int32_t row = a.perm[s * 64 + lane];
         if (row >= 0) a.y[row] = acc;

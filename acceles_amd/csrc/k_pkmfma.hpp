@@ -64,15 +64,6 @@ __device__ __forceinline__ int32_t pk_prekey(int32_t v, int rt, int rr) {
     return (int32_t)(((uint32_t)v << 6) | (uint32_t)(rt * 32 + (rr >> 2) * 8 + (rr & 3)));
 }
 
-// Workgroup barrier for LDS only: waits for this wavefront's LDS operations,
-// not for its global loads (a full barrier would also wait for the packet
-// loads issued for the slices ahead).
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Value modes of the image bytes: the value field as is (unsigned below 8
 // bits, and signed 8-bit whose field is the two's-complement byte), unsigned
 // 8-bit stored as v - 128 (the image background is -128 and 128 * sum(query)

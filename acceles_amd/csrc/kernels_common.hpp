@@ -35,23 +35,35 @@
 
 // Quantize the FP32 query into LDS: q = clip(rint(127 * (x / max|x|)), -128, 127)
 // (quantify_vector with B=8, symmetric; float32 division and product, half-even).
-// The first 4*blockDim.x values are read once, with loads issued together
-// (clamped indices, masked after), and kept in registers for both passes.
+// The first kQueryRegs*blockDim.x values are read once, with loads issued
+// together (clamped indices, masked after), and kept in registers for both
+// passes; load_query issues them ahead of what else is to be in flight.  The
+// barriers wait for LDS only.
 // xs (optional): the FP32 query is also copied there (LDS, cols floats).
-__device__ inline void quantize_query_lds(const float *x, int cols, int8_t *qx, float *red, float *xs = nullptr) {
-    constexpr int XR = 4;
-    const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
-    float xr[XR];
+static constexpr int kQueryRegs = 4;
+__device__ __forceinline__ void load_query(const float *x, int cols, float (&xr)[kQueryRegs]) {
+    if (cols <= (int)blockDim.x) {  // one load instead of four
+        xr[0] = x[min((int)threadIdx.x, cols - 1)];
 #pragma unroll
-    for (int u = 0; u < XR; ++u) xr[u] = x[min(tid + u * nt, cols - 1)];
+        for (int u = 1; u < kQueryRegs; ++u) xr[u] = 0.f;
+    } else {
+#pragma unroll
+        for (int u = 0; u < kQueryRegs; ++u) xr[u] = x[min((int)threadIdx.x + u * (int)blockDim.x, cols - 1)];
+    }
+}
+__device__ inline void quantize_query_lds(const float *x, int cols, int8_t *qx, float *red, float *xs,
+                                          const float (&xr)[kQueryRegs]) {
+    constexpr int XR = kQueryRegs;
+    const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
     float m = 0.f;
 #pragma unroll
     for (int u = 0; u < XR; ++u)
         if (tid + u * nt < cols) m = fmaxf(m, fabsf(xr[u]));
     for (int c = tid + XR * nt; c < cols; c += nt) m = fmaxf(m, fabsf(x[c]));
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    // |values| order like their bits (a DPP maximum, not six LDS shuffles)
+    m = __uint_as_float(wave_umax(__float_as_uint(m)));
     if (lane_id() == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
+    lds_barrier();
     float s = red[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); ++w) s = fmaxf(s, red[w]);
     for (int c = tid, it = 0; c < cols; c += nt, ++it) {
@@ -70,7 +82,12 @@ __device__ inline void quantize_query_lds(const float *x, int cols, int8_t *qx, 
         }
         qx[c] = (int8_t)q;
     }
-    __syncthreads();
+    lds_barrier();
+}
+__device__ inline void quantize_query_lds(const float *x, int cols, int8_t *qx, float *red, float *xs = nullptr) {
+    float xr[kQueryRegs];
+    load_query(x, cols, xr);
+    quantize_query_lds(x, cols, qx, red, xs, xr);
 }
 
 // ---------------------------------------------------------------------------
@@ -96,26 +113,47 @@ __device__ __forceinline__ void load_group(uint32_t (&w)[E], __amdgpu_buffer_rsr
     for (int i = 0; i < E; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(rs, ((g0 + i) * 64 + lane) * 4, 0, 2 /* nt */);
 }
 
+// Largest query in LDS (cols <= 8192).  A static array: its address is a
+// constant, which the byte loads take as their offset (a dynamic array's
+// address costs an addition per entry).
+static constexpr int kMaxCols = 8192;
+
+// Reads every dword of a loaded group: what is not used on some path would
+// otherwise be loaded into a register that is reused while the load is in
+// flight, and the reuse waits for all outstanding loads.
+template <int E>
+__device__ __forceinline__ void hold_group(uint32_t (&w)[E]) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) asm volatile("" : "+v"(w[i]));
+}
+
 // Accumulates value * q[col] over the entries of one group.  Padding entries
-// are all-zero bits (value 0), so only whole blocks of 8 padding entries are
-// skipped.
+// are all-zero bits (value 0; load_group leaves zeros past the slice), so only
+// whole blocks of 8 padding entries are skipped.  Four vector instructions and
+// one byte load per entry that lies in one dword: two bit-field extracts and
+// a 24-bit multiply-add (|value|, |q| < 2^8; a 32-bit multiply is quarter
+// rate), plus the joining shift of one that straddles two.
 template <int E, bool SIGNED>
 __device__ __forceinline__ int32_t decode_group(const uint32_t (&w)[E], int nd, const int8_t *qx, int cb, int vb,
-                                                uint32_t cmask, int32_t acc) {
+                                                int32_t acc) {
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
         if (((blk * 8 * E) >> 5) >= nd) continue;  // whole block is padding (wave-uniform)
+        int32_t q[8], v[8];
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj) {
             const int pos = (blk * 8 + jj) * E;
             const int wi = pos >> 5;
             const int sh = pos & 31;
             const uint32_t hi = (wi + 1 < E) ? w[wi + 1] : 0u;
-            const uint32_t bits = (sh + E <= 32) ? (w[wi] >> sh) : __builtin_amdgcn_alignbit(hi, w[wi], sh);
-            const int col = (int)(bits & cmask);
-            const int val = SIGNED ? __builtin_amdgcn_sbfe(bits, cb, vb) : (int)__builtin_amdgcn_ubfe(bits, cb, vb);
-            acc += __mul24(val, (int)qx[col]);  // |val|, |q| < 2^8: v_mul_i32_i24 (a full-rate op; a 32-bit multiply is quarter rate)
+            const bool one = sh + E <= 32;
+            const uint32_t bits = one ? w[wi] : __builtin_amdgcn_alignbit(hi, w[wi], sh);
+            const int at = one ? sh : 0;
+            q[jj] = qx[__builtin_amdgcn_ubfe(bits, at, cb)];
+            v[jj] = SIGNED ? __builtin_amdgcn_sbfe(bits, at + cb, vb) : (int)__builtin_amdgcn_ubfe(bits, at + cb, vb);
         }
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) asm("v_mad_i32_i24 %0, %1, %2, %0" : "+v"(acc) : "v"(v[jj]), "v"(q[jj]));
     }
     return acc;
 }
@@ -208,6 +246,30 @@ __device__ __forceinline__ float group_dot_rt(const uint32_t *ptr, const colx_t 
             for (int u = 0; u < U; ++u)
                 if (j + u * G < e) p = __builtin_fmaf(v[u], xv[u], p);
         }
+    }
+    for (int s = G >> 1; s >= 1; s >>= 1) p = p + __shfl_xor(p, s);
+    return p;
+}
+
+// group_dot_rt for a row given its entry range [b, e) (b = e: empty).
+template <int U>
+__device__ __forceinline__ float group_dot_range(const colx_t *idx, const float *val, const float *x, uint32_t b, uint32_t e,
+                                                 int G) {
+    float p = 0.f;
+    for (uint32_t j = b + (lane_id() & (G - 1)); j < e; j += U * G) {
+        float v[U], xv[U];
+        uint32_t c[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t jj = min(j + u * G, e - 1);
+            v[u] = val[jj];
+            c[u] = idx[jj];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = x_at(x, c[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (j + u * G < e) p = __builtin_fmaf(v[u], xv[u], p);
     }
     for (int s = G >> 1; s >= 1; s >>= 1) p = p + __shfl_xor(p, s);
     return p;
@@ -360,10 +422,12 @@ __device__ inline void topk_by_rank(const uint64_t *keys, int total, int K, acc_
 // Returns T with at least need keys >= T; when a bin is taken whole it
 // returns its lower end, so exactly need keys are >= T when the keys are
 // distinct.  Returns 0 when fewer than need keys are offered.
+// With slack, a bin's lower end is also returned when at most need + slack keys
+// are >= it (a bound for a filter, one or two digits cheaper).
 // hist: 512 LDS words; s_t: 2 LDS keys; s_need: 2 LDS ints.  Called by
 // every thread of the workgroup.
 template <typename T, class F>
-__device__ T wg_radix_kth(F for_each, int need, uint32_t *hist, T *s_t, int *s_need) {
+__device__ T wg_radix_kth(F for_each, int need, uint32_t *hist, T *s_t, int *s_need, int slack = 0) {
     constexpr int NB = 8 * (int)sizeof(T);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     for (int i = tid; i < 256; i += blockDim.x) hist[i] = 0u;
@@ -417,7 +481,7 @@ __device__ T wg_radix_kth(F for_each, int need, uint32_t *hist, T *s_t, int *s_n
                 if (above < (uint32_t)rem && (uint32_t)rem <= above + c[j]) {
                     s_t[0] = (T)((prefix << d) | (T)(255 - 4 * lane - j));
                     s_need[0] = rem - (int)above;
-                    s_need[1] = c[j] == (uint32_t)rem - above;
+                    s_need[1] = c[j] <= (uint32_t)(rem + slack) - above;
                 }
                 above += c[j];
             }
@@ -515,7 +579,8 @@ struct LowbitArgs {
     const int4 *items;          // per workgroup: (partition, first slice, end slice, 0)
     const int64_t *part_slice;  // split + 1 slice offsets
     const uint8_t *nvalid;      // rows per slice (64 except a partition's last)
-    int32_t *smax;              // per slice: largest INT32 score of its lanes
+    int4 *stop;                 // per slice: its three largest INT32 scores, the lanes of the first two
+    int top3;                   // stop holds three scores (0: the largest only)
     const float *x;             // FP32 query (cols)
     int cols, col_bits, val_bits;
     int split, M;               // partitions, rows kept per partition
