@@ -97,35 +97,68 @@ __device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t v) {
     return v;
 }
 
-// The m-th largest (m >= 1, with repeats) of the U values per lane of the
-// wavefront (0 = no value; returns 0 when fewer than m are nonzero), by
-// sorting each lane's values in registers and then extracting the wavefront
-// maximum m times: about 15 instructions per extracted value, against the 36
-// shuffle stages of a 256-key bitonic sort.
-template <int U>
-__device__ __forceinline__ uint32_t wave_kth_u32(uint32_t (&v)[U], int m) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-        for (int j = 0; j + 1 < U - i; ++j) {
-            const uint32_t x = v[j], y = v[j + 1];
-            v[j] = max(x, y);
-            v[j + 1] = min(x, y);
-        }
-    uint32_t t = 0u;
-    for (int it = 0; it < m; ++it) {
-        const uint32_t mx = wave_umax(v[0]);
-        if (mx == 0u) return 0u;
-        const int l = __builtin_ctzll(__ballot(v[0] == mx));
-        if (lane == l) {
-#pragma unroll
-            for (int j = 0; j + 1 < U; ++j) v[j] = v[j + 1];
-            v[U - 1] = 0u;
-        }
-        t = mx;
+// p + the value of lane ^ S, S a power of two below 32: the rounding of p +
+// __shfl_xor(p, S) without the LDS crossbar.  Lane ^ 4 is the quad reversal
+// of the half-row mirror; lane ^ 16 comes from v_permlane16_swap, whose two
+// results hold the even and the odd 16-lane rows.
+template <int S>
+__device__ __forceinline__ float xor_add(float p) {
+    const int v = __float_as_int(p);
+    if constexpr (S == 1) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+    if constexpr (S == 2) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+    if constexpr (S == 4) {
+        const int t = __builtin_amdgcn_update_dpp(v, v, 0x1B, 0xF, 0xF, false);
+        return p + __int_as_float(__builtin_amdgcn_update_dpp(t, t, 0x141, 0xF, 0xF, false));
     }
-    return t;
+    if constexpr (S == 8) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));
+    if constexpr (S == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return p;
+}
+template <int G>
+__device__ __forceinline__ float butterfly(float p) {
+    if constexpr (G > 16) p = xor_add<16>(p);
+    if constexpr (G > 8) p = xor_add<8>(p);
+    if constexpr (G > 4) p = xor_add<4>(p);
+    if constexpr (G > 2) p = xor_add<2>(p);
+    return xor_add<1>(p);
+}
+// A bound that at least need of the U values per lane of the wavefront reach,
+// and at most need + slack unless equal values force more (0 = no value;
+// returns 0 when fewer than need are nonzero): bisection between the smallest
+// lane maximum and the largest value, one comparison and scalar bit count per
+// value and step (no LDS; about 100 cycles a step for U = 4).
+template <int U>
+__device__ __forceinline__ uint32_t wave_bound_u32(const uint32_t (&v)[U], int need, int slack) {
+    uint32_t m = 0u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) m = max(m, v[u]);
+    auto count = [&](uint32_t t) {
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) c += __popcll(__ballot(v[u] >= t));
+        return c;
+    };
+    uint32_t hi = wave_umax(m), lo = max(~wave_umax(~m), 1u);
+    int c = count(lo);
+    if (c < need) {
+        lo = 1u;
+        c = count(lo);
+        if (c < need) return 0u;
+    }
+    while (c > need + slack && hi > lo) {
+        const uint32_t mid = lo + (hi - lo + 1u) / 2u;
+        const int cm = count(mid);
+        if (cm >= need) {
+            lo = mid;
+            c = cm;
+        } else {
+            hi = mid - 1u;
+        }
+    }
+    return lo;
 }
 
 __device__ __forceinline__ int mbcnt64(uint64_t mask) {
@@ -140,6 +173,11 @@ __device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int src) {
     uint32_t lo = (uint32_t)__shfl((int)(uint32_t)v, src);
     uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(v >> 32), src);
     return ((uint64_t)hi << 32) | lo;
+}
+
+__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int l) {  // l uniform
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
 }
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {

@@ -509,10 +509,9 @@ int launch_dense(acc_gpu_matrix *m, BatchWs &ws, const float *X, int nq, int M, 
     if ((rc = check_launch()) != ACC_OK) return rc;
     // per wavefront: two key buffers, the int8 query (rescans), the FP32 query (rescoring)
     const size_t lds_sel = (size_t)ACC_WAVES * 256 * 8 + (size_t)ACC_WAVES * m->cols_pad * 5;
-    // partitions past the register path (more than 256 slices, or M > 32):
-    // the variant that also holds up to 1024 slices' lists in registers (more
-    // registers, fewer wavefronts per SIMD)
-    const dense_fn fsel = get_dense_select(m->max_part_slices > 256 || M > 32);
+    // up to 1,024 slices per partition and M <= 32: the lists in registers, for
+    // the largest partition (more registers, fewer wavefronts per SIMD)
+    const dense_fn fsel = get_dense_select(m->max_part_slices, M);
     if ((rc = lds_limit((const void *)fsel, lds_sel)) != ACC_OK) return rc;
     LAUNCH(m, 2, fsel, dim3(m->split, (nq + ACC_WAVES - 1) / ACC_WAVES), dim3(ACC_WG), lds_sel, st, a);
     if ((rc = check_launch()) != ACC_OK) return rc;
@@ -760,8 +759,8 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         std::vector<uint32_t> p32(csr->ptr.size());
         for (size_t i = 0; i < p32.size(); ++i) p32[i] = (uint32_t)csr->ptr[i];
         TRY(dalloc(m, &m->d_ptr, p32.size()));
-        TRY(dalloc(m, &m->d_idx, (size_t)nnz + 8));  // 8 entries of padding for fp32_spmv's 16-byte loads
-        TRY(dalloc(m, &m->d_val, (size_t)nnz + 8));
+        TRY(dalloc(m, &m->d_idx, (size_t)nnz + kRowPad));
+        TRY(dalloc(m, &m->d_val, (size_t)nnz + kRowPad));
         TRY(dalloc(m, &m->d_y, (size_t)m->rows));
         COPY(m->d_ptr, p32.data(), p32.size() * 4);
         {
@@ -774,8 +773,8 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
             }
         }
         COPY(m->d_val, csr->val.data(), (size_t)nnz * 4);
-        ZERO(m->d_idx + nnz, 8 * sizeof(colx_t));
-        ZERO(m->d_val + nnz, 32);
+        ZERO(m->d_idx + nnz, kRowPad * sizeof(colx_t));
+        ZERO(m->d_val + nnz, kRowPad * 4);
         select_geometry(m->rows, m->cus, m->sel_blocks, m->sel_chunk);
         TRY(dalloc(m, &m->d_sthr, 1));
         TRY(dalloc(m, &m->d_scnt, 1));

@@ -115,63 +115,7 @@ __global__ __launch_bounds__(ACC_WG) void dense_prep(DenseArgs a) {
     }
 }
 
-// Bitonic sort, descending, of 64*R 32-bit keys in registers (element
-// i = r*64 + lane in v[r] of that lane).
-template <int R>
-__device__ __forceinline__ void reg_sort_desc_u32(uint32_t (&v)[R]) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int k = 2; k <= 64 * R; k <<= 1) {
-#pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            if (j >= 64) {
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int rp = r ^ (j >> 6);
-                    if (rp > r) {
-                        const bool desc = ((r * 64 + lane) & k) == 0;
-                        const uint32_t x = v[r], y = v[rp];
-                        const bool sw = desc ? (x < y) : (x > y);
-                        v[r] = sw ? y : x;
-                        v[rp] = sw ? x : y;
-                    }
-                }
-            } else {
-                const bool lower = (lane & j) == 0;
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const uint32_t o = (uint32_t)__shfl_xor((int)v[r], j);
-                    const bool desc = ((r * 64 + lane) & k) == 0;
-                    v[r] = (lower == desc) ? max(v[r], o) : min(v[r], o);
-                }
-            }
-        }
-    }
-}
-
-// Global rows of the listed keys of 64*U slices (k4[u] = the list of slice
-// s0 + b + u*64 + lane); -1 for keys of padding rows (row_in_slice >= nv[u],
-// nv[u] = 0 past the partition).  Issued before the threshold is known, so
-// the lookups are in flight while it is computed.
-template <int U>
-__device__ __forceinline__ void list_rows(const DenseArgs &a, const uint4 (&k4)[U], const int (&nv)[U], int64_t s0,
-                                          int b, int32_t (&row)[U][4]) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int64_t s = s0 + b + u * 64 + lane;
-        const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            // loaded for every key (slices past the matrix clamped into it) so
-            // that the loads issue together; the row is kept for real rows
-            const int32_t r = a.perm[min(s, a.nslices - 1) * 64 + tk_rho(ke[e])];
-            row[u][e] = tk_rho(ke[e]) < nv[u] ? r : -1;
-        }
-    }
-}
-
-// Offers the listed keys of those slices scoring >= ts to the collector; a
+// Offers the listed keys (k4[u] = the list of slice s0 + b + u*64 + lane) scoring >= ts to the collector; a
 // slice whose list may have dropped such a row is rescanned exactly (from its
 // packets).  Keys of padding rows are discarded, and since they may have
 // displaced real rows from a list, every list whose fourth key scores >= ts
@@ -235,10 +179,9 @@ __device__ __forceinline__ void stage_query(float *xs, const float *xq, int cols
 // order (LDS); slot i of the candidate list is keys[i] or empty past nn.
 // Each group of G lanes rescores C candidates at once in the declared order
 // (strided fmaf, then the butterfly), so the scores equal those of every
-// other rescoring path; xs is the FP32 query, staged in LDS; ranges
-// (optional, LDS): the candidates' CSR entry ranges, already loaded.
+// other rescoring path; xs is the FP32 query, staged in LDS.
 __device__ __forceinline__ void emit_candidates(const DenseArgs &a, const uint64_t *keys, int nn, size_t base,
-                                                const float *xs, const uint2 *ranges) {
+                                                const float *xs) {
     const int lane = lane_id(), M = a.M;
     if (a.cand_rows_out)
         for (int i = lane; i < M; i += 64) {
@@ -261,18 +204,7 @@ __device__ __forceinline__ void emit_candidates(const DenseArgs &a, const uint64
             r[c] = valid[c] ? dkey_row(key) : 0;
         }
         float sc[C];
-        if (ranges) {
-            uint32_t lo[C], hi[C];
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const uint2 rg = ranges[min(i0 + c * groups + grp, 63)];
-                lo[c] = valid[c] ? rg.x : 0u;
-                hi[c] = valid[c] ? rg.y : 0u;
-            }
-            group_dot_ranges_multi<C, 4>(a.idx, a.val, xs, lo, hi, G, sc);
-        } else {
-            group_dot_rt_multi<C, 4>(a.ptr, a.idx, a.val, xs, r, valid, G, sc);
-        }
+        group_dot_rt_multi<C, 4>(a.ptr, a.idx, a.val, xs, r, valid, G, sc);
         if ((lane & (G - 1)) == 0)
 #pragma unroll
             for (int c = 0; c < C; ++c) {
@@ -282,26 +214,247 @@ __device__ __forceinline__ void emit_candidates(const DenseArgs &a, const uint64
     }
 }
 
-// One wavefront per (partition p = blockIdx.x, query q = blockIdx.y*4 + wave):
-//  1. ts = a score that M distinct rows of the partition reach: the M-th best
-//     of the lanes' largest full-slice maxima on the register path, the M-th
-//     best full-slice maximum otherwise (INT32_MIN when there are not M).  The
-//     partition's M-th best score is >= ts, so no row below ts can be in its
-//     Top-M.
+// FP32 rescoring of keys[0, nn) (ranking order, LDS) with their entry ranges
+// (LDS) in the declared order, G lanes per row: a lane's U entries are at
+// constant distances, so a row takes two addresses, and C rows per lane group
+// are in flight (16 rows per round of loads: at G = 32 two rounds of eight
+// rows took 5.7 us of the selection).  Loads past a row's end are
+// masked; idx and val hold kRowPad entries past nnz.
+template <int G>
+__device__ __forceinline__ void rescore_rows(const DenseArgs &a, const uint64_t *keys, const uint2 *ranges, int nn,
+                                             size_t base, const float *xs) {
+    constexpr int groups = 64 / G, C = G >= 4 ? G / 4 : 1, U = G == 32 ? 3 : 6;
+    static_assert(U * G <= kRowPad, "reads past the last row stay in the padding");
+    const int lane = lane_id(), g = lane & (G - 1), grp = lane / G, M = a.M;
+    for (int i0 = 0; i0 < M; i0 += groups * C) {
+        uint32_t b[C], e[C];
+        float out[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int i = i0 + c * groups + grp;
+            const uint2 rg = ranges[min(i, 63)];
+            b[c] = i < nn ? rg.x + g : 0u;
+            e[c] = i < nn ? rg.y : 0u;
+            out[c] = 0.f;
+        }
+        for (;;) {
+            bool any = false;
+#pragma unroll
+            for (int c = 0; c < C; ++c) any |= b[c] < e[c];
+            if (!__any(any)) break;
+            float v[C][U];
+            uint32_t x[C][U];
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const uint32_t at = min(b[c], e[c]);
+                const float *pv = a.val + at;
+                const colx_t *pc = a.idx + at;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    v[c][u] = pv[u * G];
+                    x[c][u] = pc[u * G];
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const float f = __builtin_fmaf(v[c][u], x_at(xs, x[c][u]), out[c]);
+                    out[c] = b[c] + u * G < e[c] ? f : out[c];
+                }
+                b[c] += U * G;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const float sc = butterfly<G>(out[c]);
+            const int i = i0 + c * groups + grp;
+            if (g == 0 && i < M) a.resc[base + i] = i < nn ? dkey_f32(sc, dkey_row(keys[min(i, 63)])) : 0ull;
+        }
+    }
+}
+
+// One wavefront per (partition p = blockIdx.x, query q = blockIdx.y*4 + wave),
+// for partitions of at most 64*U slices and M <= 32:
+//  1. ts = a score that M distinct rows of the partition reach (INT32_MIN when
+//     there are not M): at least M and, equal scores aside, at most M + kSlack
+//     of the full slices' maxima reach it.  The partition's M-th best score is
+//     >= ts, so no row below ts can be in its Top-M.
 //  2. Every listed key of a real row scoring >= ts is a candidate.  A list
 //     whose fourth key still scores >= ts may have dropped a qualifying row:
 //     that slice is rescanned exactly (all 64 rows, one dot4 pass) instead.
-//     Slice maxima of partial slices (padding rows score 0) are left out of
-//     step 1; the maxima of the full slices still give M distinct real rows
-//     >= ts.
+//     Maxima of the partial slice (padding rows score 0) are left out of step
+//     1, and its padding rows' keys, which may have displaced real rows from
+//     its list, of step 2.
 //  3. Top-M of the candidates by (score, row) (quantify_util.py:173-196 with
 //     the lower-row tie rule), then their FP32 rescoring (out != null).
-// Partitions of at most 256 slices (M <= 32, at most 64 candidates) keep
-// their lists in registers: one prefix sum appends the candidates, a count
-// ranks them.  In the WIDE variant, up to 1024 slices the lists are still
-// read once into registers and offered to a collector; anything else streams
-// them twice (threshold, then offers).
-template <bool WIDE>
+// One prefix sum appends the candidates' slots, one gather finds their rows, a
+// count ranks them.  More than 64 candidates (heavy ties): every slice that
+// reaches ts is rescanned and merged into a sorted list of one key per lane.
+//
+// Bound: the memory requests of the rescoring (rows of a few cache lines each,
+// anywhere in the CSR), about 0.4 ns per row.  400,000 x 500, 100 queries:
+// 18.5 us; 22.9 when the rows of every listed key were looked up (784 per
+// partition; now about 18), the threshold came from a 64-key sort through LDS
+// and eight rows were rescored at a time.  1,000,000 x 500, 41 queries: 11.1
+// us (26.2); 2,000,000 x 900, 256 queries: 65 (111).
+template <int U>
+__global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
+    constexpr int kSlack = 8, kRescans = 128;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int wave = threadIdx.x >> 6, lane = lane_id();
+    const int p = blockIdx.x, q = blockIdx.y * ACC_WAVES + wave;
+    if (q >= a.nq) return;  // whole wavefront; no workgroup barrier below
+    // per wavefront: 64 ranked keys and their entry ranges, 64 candidates, the slices to rescan
+    uint64_t *keys = (uint64_t *)smem + wave * 256, *cand = keys + 128;
+    uint2 *ranges = (uint2 *)(keys + 64);
+    uint32_t *rl = (uint32_t *)(keys + 192);
+    int8_t *qx = (int8_t *)(smem + ACC_WAVES * 256 * 8) + (size_t)wave * a.cols_pad;
+    float *xs = (float *)(smem + ACC_WAVES * 256 * 8 + (size_t)ACC_WAVES * a.cols_pad) + (size_t)wave * a.cols_pad;
+    const int64_t s0 = a.part_slice[p];
+    const int nsl = (int)(a.part_slice[p + 1] - s0);
+    const uint4 *L = (const uint4 *)a.tk + (size_t)q * a.nslices + s0;
+    const int32_t *perm = a.perm + s0 * 64;
+    const int M = a.M;
+    const size_t base = ((size_t)q * a.split + p) * M;
+
+    int nn = 0;          // candidates kept, ranked in keys
+    if (nsl > 0) {
+        // unconditional loads (clamped into the partition, masked after) so
+        // that the lists and the query for the rescoring arrive in one round
+        // trip; a conditional load would be waited for on its own
+        uint4 k4[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) k4[u] = L[min(u * 64 + lane, nsl - 1)];
+        const int nvl = (int)a.nvalid[s0 + nsl - 1];  // every slice is full except a partition's last one
+        if (a.out) stage_query(xs, a.X + (size_t)q * a.cols, a.cols);
+        uint32_t v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = u * 64 + lane;
+            if (i >= nsl) k4[u] = make_uint4(0u, 0u, 0u, 0u);
+            v[u] = i < nsl - 1 || nvl == 64 ? k4[u].x : 0u;
+        }
+        // tk: the smallest list key of a score that reaches the bound (keys of
+        // one score differ in the row)
+        const uint32_t t = wave_bound_u32<U>(v, M, kSlack), tk = t & ~63u;
+        const int32_t ts = t != 0u ? tk_score(t) : INT32_MIN;
+        auto again = [&](int u) { return u * 64 + lane < nsl && k4[u].w >= tk; };       // to rescan
+        auto rows_of = [&](int u) {                                                   // real rows of a list to take
+            const int i = u * 64 + lane;
+            return again(u) || i >= nsl ? 0 : i == nsl - 1 ? nvl : 64;
+        };
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int nv = rows_of(u);
+            const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c += tk_rho(ke[e]) < nv && ke[e] >= tk ? 1 : 0;
+        }
+        const int incl = (int)wave_prefix_sum((uint32_t)c);
+        const int nl = __builtin_amdgcn_readlane(incl, 63);  // listed candidates
+        int n = nl, nr = 0;
+        uint64_t k = 0ull;
+        if (nl <= 64) {
+            int pos = incl - c;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int nv = rows_of(u);
+                const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (tk_rho(ke[e]) < nv && ke[e] >= tk)
+                        cand[pos++] = ((uint64_t)ke[e] << 32) | (uint32_t)((u * 64 + lane) * 64 + tk_rho(ke[e]));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {  // slices to rescan, listed so that one loop serves them all
+                const bool r = again(u);
+                const uint64_t m = __ballot(r);
+                const int j = nr + mbcnt64(m);
+                if (r && j < kRescans) rl[j] = (uint32_t)(u * 64 + lane);
+                nr += __popcll(m);
+            }
+            wave_sync();
+            if (lane < nl) {
+                const uint64_t e = cand[lane];
+                k = dkey_i32(tk_score((uint32_t)(e >> 32)), perm[(uint32_t)e]);
+            }
+        }
+        const bool many = nl > 64 || nr > kRescans;
+        if (nr > 0 || many) {
+            const int8_t *src = a.qplain + (size_t)q * a.cols_pad;
+            for (int cc = lane; cc < a.cols_pad; cc += 64) qx[cc] = src[cc];
+            wave_sync();
+        }
+        if (!many) {
+            for (int j = 0; j < nr && n <= 64; ++j) {
+                const int64_t s = s0 + __builtin_amdgcn_readfirstlane((int)rl[j]);
+                const int32_t sc = slice_dot_packets(a, s, qx);
+                const int32_t r = a.perm[s * 64 + lane];
+                const bool pr = r >= 0 && sc >= ts;
+                const uint64_t bm = __ballot(pr);
+                if (n + __popcll(bm) <= 64 && pr) cand[n + mbcnt64(bm)] = dkey_i32(sc, r);
+                n += __popcll(bm);
+            }
+            wave_sync();
+            if (n <= 64 && lane >= nl && lane < n) k = cand[lane];
+        }
+        int rank = lane;
+        if (many || n > 64) {
+            // lane i: the i-th best key so far
+            k = 0ull;
+            for (int b = 0; b < nsl; b += 64) {
+                const int i = b + lane;
+                uint64_t mask = __ballot(i < nsl && L[min(i, nsl - 1)].x >= tk);
+                while (mask) {
+                    const int64_t s = s0 + b + __builtin_ctzll(mask);
+                    mask &= mask - 1;
+                    const int32_t sc = slice_dot_packets(a, s, qx);
+                    const int32_t r = a.perm[s * 64 + lane];
+                    const uint64_t nk = r >= 0 ? dkey_i32(sc, r) : 0ull, least = shfl_u64(k, M - 1);
+                    if (!__any(nk > least)) continue;
+                    uint64_t w[2] = {k, nk};
+                    reg_sort_desc<2>(w);
+                    k = w[0];
+                }
+            }
+            n = __popcll(__ballot(k != 0ull));
+        }
+        // the candidates' CSR entry ranges, in flight while the ranks are
+        // counted (out set: the CSR is present)
+        uint2 rg = make_uint2(0u, 0u);
+        if (a.out) {
+            const int32_t r = lane < n ? dkey_row(k) : 0;
+            rg = make_uint2(a.ptr[r], a.ptr[r + 1]);
+        }
+        rank = 0;
+        for (int j = 0; j < n; ++j) rank += readlane_u64(k, j) > k;  // distinct: one per row
+        nn = min(n, M);
+        if (lane < n && rank < nn) {
+            keys[rank] = k;
+            ranges[rank] = rg;
+        }
+        wave_sync();
+    }
+    if (a.cand_rows_out)
+        for (int i = lane; i < M; i += 64) {
+            a.cand_rows_out[base + i] = i < nn ? dkey_row(keys[i]) : -1;
+            a.cand_scores_out[base + i] = i < nn ? dkey_score_i32(keys[i]) : 0;
+        }
+    if (!a.out) return;
+    switch (a.G) {
+        case 2: return rescore_rows<2>(a, keys, ranges, nn, base, xs);
+        case 4: return rescore_rows<4>(a, keys, ranges, nn, base, xs);
+        case 8: return rescore_rows<8>(a, keys, ranges, nn, base, xs);
+        case 16: return rescore_rows<16>(a, keys, ranges, nn, base, xs);
+        default: return rescore_rows<32>(a, keys, ranges, nn, base, xs);
+    }
+}
+
+// The same for any partition and M <= 64, by a collector of the offered keys:
+// the lists are streamed twice (threshold = the M-th best full-slice maximum,
+// then offers).
 __global__ __launch_bounds__(ACC_WG) void dense_select(DenseArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = threadIdx.x >> 6, lane = lane_id();
@@ -318,185 +471,12 @@ __global__ __launch_bounds__(ACC_WG) void dense_select(DenseArgs a) {
     const size_t base = ((size_t)q * a.split + p) * M;
     bool have_qx = false;
 
-    if (nsl > 0 && nsl <= 256 && M <= 32) {
-        // unconditional loads (clamped into the partition, masked after) so
-        // that the lists and the query for the rescoring arrive in one round
-        // trip; a conditional load would be waited for on its own
-        const bool narrow = a.cols <= 512;
-        float xt[8];
-        if (a.out && narrow)
-#pragma unroll
-            for (int u = 0; u < 8; ++u) xt[u] = xq[min(u * 64 + lane, a.cols - 1)];
-        uint4 k4[4];
-        int nv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = min(u * 64 + lane, nsl - 1);
-            k4[u] = L[i];
-            nv[u] = (int)a.nvalid[s0 + i];
-        }
-        if (a.out && narrow) {
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (u * 64 + lane < a.cols) xs[u * 64 + lane] = xt[u];
-        } else if (a.out) {
-            stage_query(xs, xq, a.cols);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (u * 64 + lane >= nsl) {
-                k4[u] = make_uint4(0u, 0u, 0u, 0u);
-                nv[u] = 0;
-            }
-        int32_t row[4][4];
-        list_rows<4>(a, k4, nv, s0, 0, row);
-        int32_t ts = INT32_MIN;
-        {
-            uint32_t v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = nv[u] == 64 ? k4[u].x : 0u;
-            // the M-th largest of the lanes' largest full-slice maxima: M lanes
-            // hold a maximum >= it, i.e. M distinct rows score >= it -- a
-            // valid threshold, found with one 64-key register sort
-            uint32_t h[1] = {max(max(v[0], v[1]), max(v[2], v[3]))};
-            reg_sort_desc_u32<1>(h);
-            const uint32_t t = (uint32_t)__shfl((int)h[0], M - 1);
-            if (t != 0u) ts = tk_score(t);
-        }
-        bool rescan[4], pass[16];
-        int c = 0;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            rescan[u] = nv[u] > 0 && tk_score(k4[u].w) >= ts;
-            const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                pass[u * 4 + e] = !rescan[u] && row[u][e] >= 0 && tk_score(ke[e]) >= ts;
-                c += pass[u * 4 + e] ? 1 : 0;
-            }
-        }
-        int incl = c;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(incl, o);
-            if (lane >= o) incl += t;
-        }
-        int n = __builtin_amdgcn_readlane(incl, 63);
-        if (n <= 64) {
-            int pos = incl - c;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (pass[u * 4 + e]) bufB[pos++] = dkey_i32(tk_score(ke[e]), row[u][e]);
-            }
-            // slices to rescan, listed in LDS so that one loop serves them all
-            uint32_t *rl = (uint32_t *)bufA;
-            int nr = 0;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint64_t m = __ballot(rescan[u]);
-                if (rescan[u]) rl[nr + mbcnt64(m)] = (uint32_t)(u * 64 + lane);
-                nr += __popcll(m);
-            }
-            wave_sync();
-            for (int k = 0; k < nr && n <= 64; ++k) {
-                const int64_t s = s0 + rl[k];
-                if (!have_qx) {
-                    const int8_t *src = a.qplain + (size_t)q * a.cols_pad;
-                    for (int cc = lane; cc < a.cols_pad; cc += 64) qx[cc] = src[cc];
-                    wave_sync();
-                    have_qx = true;
-                }
-                const int32_t sc = slice_dot_packets(a, s, qx);
-                const int32_t r = a.perm[s * 64 + lane];
-                const bool pr = r >= 0 && sc >= ts;
-                const uint64_t bm = __ballot(pr);
-                if (n + __popcll(bm) <= 64 && pr) bufB[n + mbcnt64(bm)] = dkey_i32(sc, r);
-                n += __popcll(bm);
-            }
-            if (n <= 64) {
-                wave_sync();
-                const uint64_t k = lane < n ? bufB[lane] : 0ull;
-                // the candidates' CSR entry ranges, in flight while the ranks
-                // are counted (out set: the CSR is present)
-                uint2 rg = make_uint2(0u, 0u);
-                if (a.out) {
-                    const int32_t r = lane < n ? dkey_row(k) : 0;
-                    rg = make_uint2(a.ptr[r], a.ptr[r + 1]);
-                }
-                const uint32_t klo = (uint32_t)k, khi = (uint32_t)(k >> 32);
-                int rank = 0;
-                for (int j = 0; j < n; ++j) {
-                    const uint64_t kj = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)khi, j) << 32) |
-                                        (uint32_t)__builtin_amdgcn_readlane((int)klo, j);
-                    rank += (kj > k || (kj == k && j < lane)) ? 1 : 0;
-                }
-                const int nn = n < M ? n : M;
-                uint2 *ranges = (uint2 *)(bufA + 64);
-                if (lane < n && rank < nn) {
-                    bufA[rank] = k;
-                    ranges[rank] = rg;
-                }
-                wave_sync();
-                emit_candidates(a, bufA, nn, base, xs, ranges);
-                return;
-            }
-        }
-    }
-
-    // General path: a collector of the offered keys.
     if (a.out) stage_query(xs, xq, a.cols);
     WaveTopM<2> cb;
     cb.init(bufB, M);
     constexpr int U = 4;
     int32_t ts = INT32_MIN;
-    if (WIDE && nsl <= 1024 && M <= 32) {
-        // every list in registers (16 per lane, loaded together, clamped into
-        // the partition and masked after); the threshold is the M-th largest
-        // full-slice maximum, then the lists are offered from the registers
-        uint4 k4[4][U];
-        int nv[4][U];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = min((j * U + u) * 64 + lane, nsl - 1);
-                k4[j][u] = L[i];
-                nv[j][u] = (int)a.nvalid[s0 + i];
-            }
-        uint32_t v[16];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if ((j * U + u) * 64 + lane >= nsl) {
-                    k4[j][u] = make_uint4(0u, 0u, 0u, 0u);
-                    nv[j][u] = 0;
-                }
-                v[j * U + u] = nv[j][u] == 64 ? k4[j][u].x : 0u;
-            }
-        const uint32_t t = wave_kth_u32<16>(v, M);
-        if (t != 0u) ts = tk_score(t);
-        offer_lists<U>(a, cb, k4[0], nv[0], s0, 0, ts, q, qx, have_qx);
-        if (U * 64 < nsl) offer_lists<U>(a, cb, k4[1], nv[1], s0, U * 64, ts, q, qx, have_qx);
-        if (2 * U * 64 < nsl) offer_lists<U>(a, cb, k4[2], nv[2], s0, 2 * U * 64, ts, q, qx, have_qx);
-        if (3 * U * 64 < nsl) offer_lists<U>(a, cb, k4[3], nv[3], s0, 3 * U * 64, ts, q, qx, have_qx);
-        cb.compact();
-        emit_candidates(a, cb.buf, cb.n, base, xs, nullptr);
-        return;
-    }
-    if (nsl <= 1024 && M <= 32) {  // the M-th largest maximum by extraction, maxima in registers
-        uint32_t v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int i = u * 64 + lane;
-            v[u] = i < nsl && a.nvalid[s0 + i] == 64 ? L[i].x : 0u;
-        }
-        const uint32_t t = wave_kth_u32<16>(v, M);
-        if (t != 0u) ts = tk_score(t);
-    } else {
+    {
         WaveTopM<2> ca;
         ca.init(bufA, M);
         for (int b = 0; b < nsl; b += 64 * U) {
@@ -527,7 +507,7 @@ __global__ __launch_bounds__(ACC_WG) void dense_select(DenseArgs a) {
         offer_lists<U>(a, cb, k4, nv, s0, b, ts, q, qx, have_qx);
     }
     cb.compact();
-    emit_candidates(a, cb.buf, cb.n, base, xs, nullptr);
+    emit_candidates(a, cb.buf, cb.n, base, xs);
 }
 
 // One workgroup per query: each wavefront sorts a quarter of the query's
@@ -554,7 +534,10 @@ __global__ __launch_bounds__(ACC_WG) void batch_topk_radix(DenseArgs a) {
 }
 
 dense_fn get_dense_prep() { return dense_prep; }
-dense_fn get_dense_select(bool wide) { return wide ? dense_select<true> : dense_select<false>; }
+dense_fn get_dense_select(int64_t part_slices, int M) {
+    if (M > 32 || part_slices > 1024) return dense_select;
+    return part_slices <= 256 ? dense_select_regs<4> : part_slices <= 512 ? dense_select_regs<8> : dense_select_regs<16>;
+}
 dense_fn get_batch_topk_radix(int V) {
     switch (V) {
         case 1: return batch_topk_radix<1>;

@@ -19,35 +19,6 @@
 // FP32 CSR path
 // ---------------------------------------------------------------------------
 
-// p + the value of lane ^ S, S a power of two below 32: the rounding of p +
-// __shfl_xor(p, S) without the LDS crossbar.  Lane ^ 4 is the quad reversal
-// of the half-row mirror; lane ^ 16 comes from v_permlane16_swap, whose two
-// results hold the even and the odd 16-lane rows.
-template <int S>
-__device__ __forceinline__ float xor_add(float p) {
-    const int v = __float_as_int(p);
-    if constexpr (S == 1) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
-    if constexpr (S == 2) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
-    if constexpr (S == 4) {
-        const int t = __builtin_amdgcn_update_dpp(v, v, 0x1B, 0xF, 0xF, false);
-        return p + __int_as_float(__builtin_amdgcn_update_dpp(t, t, 0x141, 0xF, 0xF, false));
-    }
-    if constexpr (S == 8) return p + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));
-    if constexpr (S == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    }
-    return p;
-}
-template <int G>
-__device__ __forceinline__ float butterfly(float p) {
-    if constexpr (G > 16) p = xor_add<16>(p);
-    if constexpr (G > 8) p = xor_add<8>(p);
-    if constexpr (G > 4) p = xor_add<4>(p);
-    if constexpr (G > 2) p = xor_add<2>(p);
-    return xor_add<1>(p);
-}
-
 // y = A x with G lanes per row.  Lane g of a row sums its entries
 // g, g+G, g+2G, ... in that order with fmaf, then an xor butterfly of plain
 // adds.

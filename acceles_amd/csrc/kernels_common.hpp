@@ -216,6 +216,7 @@ __device__ inline void publish_and_append(WaveTopM<R> &col, uint64_t *thr, uint3
 // 4 * column (cols <= 8192), so that an entry is 6 bytes instead of 8 and the
 // offset addresses x without a shift.
 typedef uint16_t colx_t;
+static constexpr int kRowPad = 256;  // entries (zeros) past nnz that kernels may read and mask
 __device__ __forceinline__ float x_at(const float *x, uint32_t c) { return *(const float *)((const char *)x + c); }
 
 // Dot product of CSR row r with x by a group of G lanes (runtime G): lane g
@@ -780,7 +781,7 @@ batch_fn get_batch_select();                                   // k_batch.hip
 batch_fn get_batch_final(int R);
 typedef void (*dense_fn)(DenseArgs);
 dense_fn get_dense_prep();                                     // k_dense.hip
-dense_fn get_dense_select(bool wide);
+dense_fn get_dense_select(int64_t part_slices, int M);
 dense_fn get_batch_topk_radix(int V);
 dense_fn get_batch_topk(int R);
 dense_fn get_pk_scores_8(int E);                               // k_pkmfma_a.hip
