@@ -278,8 +278,9 @@ __device__ __forceinline__ void rescore_rows(const DenseArgs &a, const uint64_t 
 // for partitions of at most 64*U slices and M <= 32:
 //  1. ts = a score that M distinct rows of the partition reach (INT32_MIN when
 //     there are not M): at least M and, equal scores aside, at most M + kSlack
-//     of the full slices' maxima reach it.  The partition's M-th best score is
-//     >= ts, so no row below ts can be in its Top-M.
+//     of the full slices' maxima reach it (up to 64 slices: M of their listed
+//     scores).  The partition's M-th best score is >= ts, so no row below ts
+//     can be in its Top-M.
 //  2. Every listed key of a real row scoring >= ts is a candidate.  A list
 //     whose fourth key still scores >= ts may have dropped a qualifying row:
 //     that slice is rescanned exactly (all 64 rows, one dot4 pass) instead.
@@ -328,16 +329,29 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
         for (int u = 0; u < U; ++u) k4[u] = L[min(u * 64 + lane, nsl - 1)];
         const int nvl = (int)a.nvalid[s0 + nsl - 1];  // every slice is full except a partition's last one
         if (a.out) stage_query(xs, a.X + (size_t)q * a.cols, a.cols);
-        uint32_t v[U];
+        uint32_t t;
+        {
+            uint32_t v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = u * 64 + lane;
-            if (i >= nsl) k4[u] = make_uint4(0u, 0u, 0u, 0u);
-            v[u] = i < nsl - 1 || nvl == 64 ? k4[u].x : 0u;
+            for (int u = 0; u < U; ++u) {
+                const int i = u * 64 + lane;
+                if (i >= nsl) k4[u] = make_uint4(0u, 0u, 0u, 0u);
+                v[u] = i < nsl - 1 || nvl == 64 ? k4[u].x : 0u;
+            }
+            if (nsl <= 64) {
+                // few slices: their whole lists (distinct rows), exactly --
+                // fewer than M maxima, or a low one, would make every list
+                // drop rows that qualify
+                const bool full = lane < nsl - 1 || nvl == 64;
+                const uint32_t w[4] = {full ? k4[0].x : 0u, full ? k4[0].y : 0u, full ? k4[0].z : 0u, full ? k4[0].w : 0u};
+                t = wave_bound_u32<4>(w, M, 0);
+            } else {
+                t = wave_bound_u32<U>(v, M, kSlack);
+            }
         }
         // tk: the smallest list key of a score that reaches the bound (keys of
         // one score differ in the row)
-        const uint32_t t = wave_bound_u32<U>(v, M, kSlack), tk = t & ~63u;
+        const uint32_t tk = t & ~63u;
         const int32_t ts = t != 0u ? tk_score(t) : INT32_MIN;
         auto again = [&](int u) { return u * 64 + lane < nsl && k4[u].w >= tk; };       // to rescan
         auto rows_of = [&](int u) {                                                   // real rows of a list to take
