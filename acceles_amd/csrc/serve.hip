@@ -137,7 +137,12 @@ void reap(acc_server *s) {
 }
 
 // Gives free slots to the matrices whose oldest waiting request is oldest.
-void launch(acc_server *s) {
+// The lock (lk, held on entry and on return) is dropped while a batch is
+// enqueued: with it held, every submission waited for the launches of the
+// batch before it, so that a burst of requests ran as batches of one (200
+// requests at 400,000 x 500: 4.0 ms, now 1.24).  The slot is marked busy first; only
+// this thread changes slots, and a matrix is destroyed only after it has ended.
+void launch(acc_server *s, std::unique_lock<std::mutex> &lk) {
     for (int i = 0; i < s->o.slots; ++i) {
         Slot &sl = s->slots[i];
         if (sl.busy) continue;
@@ -168,15 +173,21 @@ void launch(acc_server *s) {
         }
         sl.stride = kmax;
         sl.matrix = best;
-        int rc = hipMemcpyAsync(sl.x_dev, sl.x_pin, (size_t)nq * mx.cols * 4, hipMemcpyHostToDevice, sl.st) == hipSuccess
-                     ? ACC_OK : ACC_ERR_DEVICE;
+        sl.busy = true;
+        acc_gpu_matrix *m = mx.m;  // s->mats may grow meanwhile
+        const size_t x_bytes = (size_t)nq * mx.cols * 4;
+        lk.unlock();
+        int rc = hipMemcpyAsync(sl.x_dev, sl.x_pin, x_bytes, hipMemcpyHostToDevice, sl.st) == hipSuccess ? ACC_OK
+                                                                                                        : ACC_ERR_DEVICE;
         if (rc == ACC_OK)
-            rc = acc::topk_lowbit_batch_ws(mx.m, sl.ws, sl.x_dev, nq, sl.ks.data(), s->o.ck, sl.o_dev, kmax, sl.st);
+            rc = acc::topk_lowbit_batch_ws(m, sl.ws, sl.x_dev, nq, sl.ks.data(), s->o.ck, sl.o_dev, kmax, sl.st);
         if (rc == ACC_OK &&
             hipMemcpyAsync(sl.o_pin, sl.o_dev, (size_t)nq * kmax * sizeof(acc_element), hipMemcpyDeviceToHost, sl.st) != hipSuccess)
             rc = ACC_ERR_DEVICE;
         if (rc == ACC_OK && hipEventRecord(sl.ev, sl.st) != hipSuccess) rc = ACC_ERR_DEVICE;
-        if (rc != ACC_OK) {  // fail these requests; the slot stays free
+        lk.lock();
+        if (rc != ACC_OK) {  // fail these requests; the slot is free again
+            sl.busy = false;
             const auto now = Clock::now();
             for (uint64_t id : sl.ids) {
                 auto it = s->reqs.find(id);
@@ -192,9 +203,9 @@ void launch(acc_server *s) {
             s->cv_done.notify_all();
             continue;
         }
-        ++mx.inflight;
-        s->peak_inflight = std::max<int64_t>(s->peak_inflight, mx.inflight);
-        sl.busy = true;
+        Matrix &launched = s->mats[(size_t)best];
+        ++launched.inflight;
+        s->peak_inflight = std::max<int64_t>(s->peak_inflight, launched.inflight);
         ++s->batches;
         s->batched += nq;
     }
@@ -207,7 +218,7 @@ void worker_main(acc_server *s) {
         const int64_t before = s->completed;
         reap(s);
         if (s->completed != before) s->cv_done.notify_all();
-        launch(s);
+        launch(s, lk);
         bool busy = false;
         for (int i = 0; i < s->o.slots; ++i) busy |= s->slots[i].busy;
         if (busy)
