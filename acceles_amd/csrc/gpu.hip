@@ -113,7 +113,7 @@ struct acc_gpu_matrix {
     bool dense_ok = false;           // the matrix cores can score this matrix exactly
     std::string dense_why;           // why not, otherwise
     int batch_mode = ACC_BATCH_AUTO;
-    int dense_min_nq = 16;           // ACC_BATCH_AUTO, untuned: matrix cores from this batch size on
+    int dense_min_nq = 0;            // ACC_BATCH_AUTO, untuned: matrix cores from this batch size on (0: by estimate)
     // ACC_BATCH_AUTO after acc_gpu_autotune: the layout measured fastest at
     // tune_nq[i], used for batches of tune_nq[i] .. tune_nq[i+1]-1 queries
     int ntune = 0;
@@ -414,7 +414,30 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
     return a;
 }
 
-// Layout of a batch of nq queries: ACC_BATCH_SINGLE, _SPARSE or _DENSE.
+// Estimated time of a batch per layout, in us.  Measured (CK 512, K 100; batch
+// of 8, us single / packets / matrix cores): 20,000 x 500 175 / 70 / 43, 400,000
+// x 500 218 / 103 / 47, 1,000,000 x 250 4-bit 215 / 118 / 71, 2,000,000 x 900
+// 472 / 232 / 198, 5,000,000 x 1024 (20 entries per row) 472 / 302 / 488; one
+// query: 25 / 65 / 41, 31 / 98 / 47, 28 / 110 / 70, 59 / 221 / 201, 61 / 278
+// / 493.  So: a single query pays about 21 us and its packets at 7 TB/s; the
+// packet batch 55 us and 1.5 ns per 1,000 entries and 0.6 ns per slice for
+// every block of 16 or 32 queries; the matrix cores 33 us and per slice 2.4
+// ns up to 16 column blocks, 5.5 above (a 128-query block).
+struct BatchCost {
+    double single, sparse, dense;
+};
+BatchCost batch_cost(const acc_gpu_matrix *m, int nq) {
+    BatchCost c;
+    c.single = nq * (21.0 + (double)m->stream_bytes / 7e6);
+    const int qb = nq <= 16 ? 16 : 32;
+    c.sparse = 55.0 + (1.5e-6 * (double)m->nnz + 0.6e-3 * (double)m->nslices) * (qb / 16) * ((nq + qb - 1) / qb);
+    c.dense = 33.0 + (m->nkb <= 16 ? 2.4e-3 : 5.5e-3) * (double)m->nslices * ((nq + 127) / 128);
+    return c;
+}
+
+// Layout of a batch of nq queries: ACC_BATCH_SINGLE, _SPARSE or _DENSE.  All
+// give the same results; untuned, the one of the lowest estimate, except that
+// a crossover the caller has set decides where the matrix cores are used.
 int batch_layout(const acc_gpu_matrix *m, int nq) {
     if (m->batch_mode != ACC_BATCH_AUTO) return m->batch_mode;
     if (m->ntune > 0) {
@@ -423,7 +446,9 @@ int batch_layout(const acc_gpu_matrix *m, int nq) {
             if (m->tune_nq[i] <= nq) pick = m->tune_layout[i];
         return pick;
     }
-    return m->dense_ok && nq >= m->dense_min_nq ? ACC_BATCH_DENSE : ACC_BATCH_SPARSE;
+    const BatchCost c = batch_cost(m, nq);
+    const bool dense = m->dense_ok && (m->dense_min_nq > 0 ? nq >= m->dense_min_nq : c.dense < std::min(c.single, c.sparse));
+    return dense ? ACC_BATCH_DENSE : c.single < c.sparse ? ACC_BATCH_SINGLE : ACC_BATCH_SPARSE;
 }
 
 // B registers for 8, 16, 24, 30 or 32 column blocks: the smallest that holds
@@ -1002,6 +1027,8 @@ void batch_ws_destroy(BatchWorkspace *w, int device) {
 }
 
 int64_t batch_ws_bytes(const BatchWorkspace *w) { return w ? w->bytes : 0; }
+
+int batch_layout_of(const acc_gpu_matrix *m, int nq) { return batch_layout(m, nq); }
 
 int topk_lowbit_batch_ws(acc_gpu_matrix *m, BatchWorkspace *w, const float *x_dev, int nq, const int32_t *k_host,
                          int ck, acc_element *out_dev, int out_stride, void *stream) {

@@ -328,8 +328,9 @@ extern "C" int acc_server_add_matrix(acc_server *s, const acc_csr *csr, const ac
     if (rc == ACC_OK && s->o.autotune)
         rc = acc_gpu_autotune(m, s->o.ck, std::min(100, std::min(kMaxK, s->o.ck)), s->o.max_batch, nullptr, 0, nullptr);
     // the workspace a slot needs for this matrix: a scratch workspace warmed
-    // with batches of 1, 2, 4, ... max_batch queries (every layout the
-    // handle's batch-size table can pick), then freed
+    // with batches of 1, 2, 4, ... max_batch queries and the largest batch of
+    // every run of sizes with one layout (a layout's workspace grows with the
+    // batch), then freed
     int64_t need = 0;
     {
         acc::BatchWorkspace *w = acc::batch_ws_create();
@@ -340,10 +341,11 @@ extern "C" int acc_server_add_matrix(acc_server *s, const acc_csr *csr, const ac
             rc = fail(ACC_ERR_NOMEM, "warm-up buffers");
         if (rc == ACC_OK && hipMemset(x, 0, (size_t)s->o.max_batch * csr->cols * 4) != hipSuccess) rc = ACC_ERR_DEVICE;
         std::vector<int32_t> ks((size_t)s->o.max_batch, 1);
-        for (int b = 1; rc == ACC_OK; b = std::min(2 * b, s->o.max_batch)) {
+        for (int b = 1; rc == ACC_OK && b <= s->o.max_batch; ++b) {
+            if ((b & (b - 1)) != 0 && b != s->o.max_batch && acc::batch_layout_of(m, b) == acc::batch_layout_of(m, b + 1))
+                continue;
             rc = acc::topk_lowbit_batch_ws(m, w, x, b, ks.data(), s->o.ck, o, 1, nullptr);
             if (rc == ACC_OK && hipDeviceSynchronize() != hipSuccess) rc = fail(ACC_ERR_DEVICE, "warm-up batch failed");
-            if (b == s->o.max_batch) break;
         }
         need = acc::batch_ws_bytes(w);
         acc::batch_ws_destroy(w, s->o.device);
