@@ -33,7 +33,6 @@ static constexpr size_t kWordPad = 32 * 64;  // dwords past the packets (>= wide
 // 10.0 us), so they pay up to some 100,000 slices.
 static constexpr int64_t kTop3Slices = 65536;
 static constexpr int kPkMaxCols = 1024;  // matrix-core scores: B operands of 32 column blocks in registers
-static constexpr int kPkMinE = 18, kPkMaxE = 23;  // image-packet entry widths instantiated for them
 static constexpr size_t kPkLdsMax = 160 * 1024;  // LDS of a pk_scores workgroup at most
 
 // Per-batch device workspace of the batched path.  The handle owns one;
@@ -103,9 +102,8 @@ struct acc_gpu_matrix {
     int32_t *d_crow = nullptr, *d_cscore = nullptr;  // split * kMaxM (candidate outputs)
     int64_t *d_part_slice = nullptr;                 // split + 1
     int64_t max_part_slices = 0;                     // slices of the largest partition
-    uint32_t *d_pwords = nullptr;                    // image packets (matrix-core scores), E = 8 + pcb
+    uint32_t *d_pwords = nullptr;                    // image packets (matrix-core scores)
     uint2 *d_pslices = nullptr;
-    int pcb = 0;
     int64_t pbytes = 0;                              // image-packet bytes read per pass (words + slice table)
     BatchWs ws;                      // batched-path workspace (grown on demand)
     // batched path on the matrix cores (slices expanded from the packets in LDS)
@@ -394,7 +392,6 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
     a.slices = m->d_slices;
     a.pwords = m->d_pwords;
     a.pslices = m->d_pslices;
-    a.pcb = m->pcb;
     a.perm = m->d_perm;
     a.part_slice = m->d_part_slice;
     a.nvalid = m->d_nvalid;
@@ -452,21 +449,19 @@ int batch_layout(const acc_gpu_matrix *m, int nq) {
 }
 
 // B registers for 8, 16, 24, 30 or 32 column blocks: the smallest that holds
-// the matrix (the multiplications run over all of them, zero past nkb); E =
-// the image packets' entry bits.  Up to 16 column blocks the chain runs in
-// half-rounds: with one tile per MFMA wavefront its registers leave room for
+// the matrix (the multiplications run over all of them, zero past nkb).  Up to
+// 16 column blocks the chain runs in half-rounds: with one tile per MFMA wavefront its registers leave room for
 // two workgroups per CU (k_pkmfma_{a,b}), with two tiles (tpw = 2) each A
 // read feeds both (k_pkmfma_{f,g}).  Above 16 column blocks, a batch of more
 // than four tiles runs eight MFMA wavefronts per workgroup, two per SIMD
 // (wide, k_pkmfma_h): one decode of each slice for up to 256 queries.
 dense_fn pk_kernel(const acc_gpu_matrix *m, int tpw, bool wide) {
-    const int E = 8 + m->pcb;
-    if (tpw == 2) return m->nkb > 8 ? get_pk2_scores_16(E) : get_pk2_scores_8(E);
-    if (wide) return m->nkb > 30 ? get_pk3_scores_32(E) : m->nkb > 24 ? get_pk3_scores_30(E) : get_pk3_scores_24(E);
-    if (m->nkb > 30) return get_pk_scores_32(E);
-    if (m->nkb > 24) return get_pk_scores_30(E);
-    if (m->nkb > 16) return get_pk_scores_24(E);
-    return m->nkb > 8 ? get_pk_scores_16(E) : get_pk_scores_8(E);
+    if (tpw == 2) return m->nkb > 8 ? get_pk2_scores_16() : get_pk2_scores_8();
+    if (wide) return m->nkb > 30 ? get_pk3_scores_32() : m->nkb > 24 ? get_pk3_scores_30() : get_pk3_scores_24();
+    if (m->nkb > 30) return get_pk_scores_32();
+    if (m->nkb > 24) return get_pk_scores_30();
+    if (m->nkb > 16) return get_pk_scores_24();
+    return m->nkb > 8 ? get_pk_scores_16() : get_pk_scores_8();
 }
 
 // Batched low-bit queries on the matrix cores: dense_prep, pk_scores (slices
@@ -879,14 +874,9 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
             // their offsets in a decode wavefront's 16 image rows, repeated
             // columns merged (k_pkmfma.hpp)
             const uint32_t stride = (uint32_t)m->cols_pad + 16u;
-            m->pcb = acc::bits_for((int32_t)(16u * stride));
-            if (8 + m->pcb < kPkMinE || 8 + m->pcb > kPkMaxE) {
-                rc = fail(ACC_ERR_ARG, "image-packet entry width out of range");
-                goto failed;
-            }
             std::vector<uint32_t> pw;
             std::vector<std::pair<uint32_t, uint32_t>> ps;
-            TRY(acc::image_packets(pk, m->u8off, m->pcb, stride, pw, ps));
+            TRY(acc::image_packets(pk, m->u8off, stride, pw, ps));
             std::vector<uint2> psl(ps.size());
             for (size_t i = 0; i < ps.size(); ++i) psl[i] = make_uint2(ps[i].first, ps[i].second);
             TRY(dalloc(m, &m->d_pwords, pw.size() + kWordPad));

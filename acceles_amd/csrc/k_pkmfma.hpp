@@ -68,16 +68,24 @@ __device__ __forceinline__ int32_t pk_prekey(int32_t v, int rt, int rr) {
 // bits, and signed 8-bit whose field is the two's-complement byte), unsigned
 // 8-bit stored as v - 128 (the image background is -128 and 128 * sum(query)
 // is added back per query), and signed below 8 bits (sign-extended).
-// Entry j of a lane's image-packet chunk (E dwords = 32 entries) stored into
-// the decode wavefront's 16 image rows at wimg: an entry is byte | (o << 8)
-// with o = row * stride + column inside those rows, and its byte is already
-// the image's value.
-template <int E>
-__device__ __forceinline__ void pk_entry(const uint32_t (&w)[E], int j, unsigned char *wimg, int ob) {
-    const int pos = j * E, wi = pos >> 5, sh = pos & 31;
-    const uint32_t hi = (wi + 1 < E) ? w[wi + 1] : 0u;
-    const uint32_t bits = (sh + E <= 32) ? (w[wi] >> sh) : __builtin_amdgcn_alignbit(hi, w[wi], sh);
-    wimg[__builtin_amdgcn_ubfe(bits, 8, ob)] = (unsigned char)bits;
+
+// A lane's group of four image entries: (offset 0 | offset 1 << 16, offset 2 |
+// offset 3 << 16, their bytes), the offsets inside the decode wavefront's 16
+// image rows at wimg.  The decode wavefronts share their SIMD's issue slots with
+// the multiplications and set the pace of a round, so an entry is laid out for
+// few instructions rather than few bits: 5 VALU per four entries (an add that
+// selects the offset's half word each, one shift for bytes 1 and 3, which the
+// stores take from bits 7:0 and 23:16) where bit-packed entries of 18 to 23
+// bits took 12.  pk_scores, with the A operands three column blocks ahead:
+// 1M x 500 signed 6-bit, 41 queries 67.5 -> 62.4 us; 400k x 500, 100 queries
+// 37.6 -> 36.2 us, 8 queries 25.1 -> 24.6 us; 2M x 900, 256 queries level.
+typedef uint32_t pv3u __attribute__((ext_vector_type(3)));
+__device__ __forceinline__ void pk_group(const pv3u &w, unsigned char *wimg) {
+    const uint32_t odd = w.z >> 8;
+    wimg[w.x & 0xFFFFu] = (unsigned char)w.z;
+    wimg[w.x >> 16] = (unsigned char)odd;
+    wimg[w.y & 0xFFFFu] = (unsigned char)(w.z >> 16);
+    wimg[w.y >> 16] = (unsigned char)(odd >> 16);
 }
 
 // Wavefront roles: up to kPkMfmaWaves MFMA wavefronts (one or two 32-query
@@ -112,7 +120,6 @@ struct PkCtx {
     int64_t end;  // one past this workgroup's last slice
     uint32_t cols_pad, stride, img_bytes, fill, a_base;
     uint32_t wrow;                // decode wavefronts: offset of their 16 rows in an image (16 * dw * stride)
-    int ob;                       // offset bits of the image-packet entries
     __amdgpu_buffer_rsrc_t meta;  // a.pslices
 };
 
@@ -261,7 +268,10 @@ struct PkMRegsH {
 
 template <int KB, int NTL, int RT, bool LISTS, int kb>
 __device__ __forceinline__ void pk_hstep(PkMRegsH<NTL> &r, const pv4i (&B)[NTL][KB], const pv4i *A) {
-    constexpr int RING = 4, DIST = 2;
+    // the A operand three column blocks ahead, the ring's last free slot: two
+    // ahead, a wavefront waits for LDS while decode stores fill its queue
+    // (1M x 500, 41 queries: 66.2 -> 62.4 us; 400k x 500, 100: 36.6 -> 36.2)
+    constexpr int RING = 4, DIST = 3;
     if constexpr (kb + DIST < KB) r.ar[(kb + DIST) % RING] = A[(kb + DIST) * 2];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -298,6 +308,7 @@ __device__ __forceinline__ void pk_hround(const PkCtx &c, PkMRegsH<NTL> &r, cons
     const pv4i *A = (const pv4i *)(c.smem + img * c.img_bytes + c.a_base + (uint32_t)RT * 32u * c.stride);
     r.ar[0] = A[0];
     r.ar[1] = A[2];
+    r.ar[2] = A[4];
     pk_hchain<KB, NTL, RT, LISTS>(std::make_integer_sequence<int, KB>(), r, B, A);
 }
 
@@ -412,44 +423,42 @@ __device__ __forceinline__ void pk_mmains(const PkCtx &c, int qb, int tile, int6
 
 // Decode wavefront dw owns rows 16*dw .. 16*dw + 15 of every image.  Its
 // stream of a slice holds the entries of those rows split among its lanes,
-// consecutive ones per lane, n per lane (n a multiple of 4, the same for
+// consecutive ones per lane, in groups of four per lane (the same number for
 // every lane; a lane's last slots repeat entries of the next lanes), so the
-// entries are spread evenly over the lanes whatever the rows' lengths.  Every byte of those rows is written
-// by this wavefront only, in program order, so clearing an image and
-// expanding the next slice into it need no barrier between them.
-template <int E>
+// entries are spread evenly over the lanes whatever the rows' lengths.  Every
+// byte of those rows is written by this wavefront only, in program order, so
+// clearing an image and expanding the next slice into it need no barrier
+// between them.
+static constexpr int kPkChunk = 8;  // groups of a chunk (32 entries per lane)
 struct PkDRegs {
-    uint32_t w[2][E];       // the first chunk of the next slice, by round parity
+    pv3u w[2][kPkChunk];    // the first chunk of the next slice, by round parity
 };
 
-// This wavefront's stream of the slice with metadata m (offset in units of
-// 64 dwords; n/4 of wavefront w in byte w): a buffer over its dwords (loads
-// past its end return zeros and fetch nothing) and n.
+// This wavefront's stream of the slice with metadata m (offset in groups;
+// groups of wavefront w in byte w): a buffer over its groups (loads past its
+// end return zeros and fetch nothing) and their number.
 struct PkStream {
     __amdgpu_buffer_rsrc_t rs;
     int n;
 };
 
-template <int E>
 __device__ __forceinline__ PkStream pk_stream(const PkCtx &c, uint2 m, int dw) {
     const uint32_t off = __builtin_amdgcn_readfirstlane(m.x), cnt = __builtin_amdgcn_readfirstlane(m.y);
     dw = __builtin_amdgcn_readfirstlane(dw);  // uniform: the buffer descriptor stays scalar
-    uint32_t woff = 0;
-    for (int w = 0; w < dw; ++w) woff += (((cnt >> (8 * w)) & 255u) * 4u * E + 31u) / 32u;
-    const uint32_t n = ((cnt >> (8 * dw)) & 255u) * 4u;
+    uint32_t before = 0;
+    for (int w = 0; w < dw; ++w) before += (cnt >> (8 * w)) & 255u;
     PkStream st;
-    st.rs = __builtin_amdgcn_make_buffer_rsrc((void *)(c.a->pwords + ((size_t)off + woff) * 64), (short)0,
-                                              (int)((n * E + 31u) / 32u * 256u), 0x00020000 /* 32-bit data format */);
-    st.n = (int)n;
+    st.n = (int)((cnt >> (8 * dw)) & 255u);
+    st.rs = __builtin_amdgcn_make_buffer_rsrc((void *)(c.a->pwords + ((size_t)off + before) * 192), (short)0, st.n * 768,
+                                              0x00020000 /* 32-bit data format */);
     return st;
 }
 
-// The E dwords of chunk k (entries 32k .. 32k+31) of the lane's stream.
-template <int E>
-__device__ __forceinline__ void pk_load_chunk(uint32_t (&w)[E], __amdgpu_buffer_rsrc_t rs, const PkCtx &c, int k) {
+// Chunk k of the lane's stream (groups 8k .. 8k+7), 12-byte loads.
+__device__ __forceinline__ void pk_load_chunk(pv3u (&w)[kPkChunk], __amdgpu_buffer_rsrc_t rs, const PkCtx &c, int k) {
 #pragma unroll
-    for (int i = 0; i < E; ++i)
-        w[i] = __builtin_amdgcn_raw_buffer_load_b32(rs, ((k * E + i) * 64 + c.lane) * 4, 0, 2 /* nt */);
+    for (int i = 0; i < kPkChunk; ++i)
+        w[i] = __builtin_amdgcn_raw_buffer_load_b96(rs, ((k * kPkChunk + i) * 64 + c.lane) * 12, 0, 2 /* nt */);
 }
 
 // This wavefront's rows of image img back to the background: 16 rows =
@@ -468,29 +477,28 @@ __device__ __forceinline__ void pk_clear(const PkCtx &c, unsigned char *img) {
     for (; i < c.stride; i += 64u) p4[i] = f;
 }
 
-// The first m entries of a chunk (m wave-uniform, a multiple of 4).
-template <int E>
-__device__ __forceinline__ void pk_chunk(const uint32_t (&w)[E], int m, unsigned char *wimg, int ob) {
-    m = __builtin_amdgcn_readfirstlane(m);  // a scalar branch per four entries
+// The first m groups of a chunk (m wave-uniform).
+__device__ __forceinline__ void pk_chunk(const pv3u (&w)[kPkChunk], int m, unsigned char *wimg) {
+    m = __builtin_amdgcn_readfirstlane(m);  // a scalar branch per group
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        if (4 * q >= m) return;
-#pragma unroll
-        for (int j = 4 * q; j < 4 * q + 4; ++j) pk_entry<E>(w, j, wimg, ob);
+    for (int q = 0; q < kPkChunk; ++q) {
+        if (q >= m) return;
+        pk_group(w[q], wimg);
     }
 }
 
 // A slice (stream st, first chunk in w, further chunks loaded here) into
 // image img.
-template <int E>
-__device__ __forceinline__ void pk_expand(const PkCtx &c, const uint32_t (&w)[E], const PkStream &st,
+__device__ __forceinline__ void pk_expand(const PkCtx &c, const pv3u (&w)[kPkChunk], const PkStream &st,
                                           unsigned char *img) {
     unsigned char *wimg = img + c.wrow;
-    pk_chunk<E>(w, st.n, wimg, c.ob);
-    for (int k = 1; 32 * k < st.n; ++k) {
-        uint32_t x[E];
-        pk_load_chunk<E>(x, st.rs, c, k);
-        pk_chunk<E>(x, st.n - 32 * k, wimg, c.ob);
+    pk_chunk(w, st.n, wimg);
+    for (int k = 1; kPkChunk * k < st.n; ++k) {
+        pv3u x[kPkChunk];
+        pk_load_chunk(x, st.rs, c, k);
+#pragma unroll
+        for (int i = 0; i < kPkChunk; ++i) asm volatile("" : "+v"(x[i]));  // all loads issued here, not one per branch
+        pk_chunk(x, st.n - kPkChunk * k, wimg);
     }
 }
 
@@ -510,14 +518,14 @@ __device__ __forceinline__ uint2 pk_slice_meta(const PkCtx &c, int64_t s) {
 // earlier) expanded into image 1 - P after this wavefront's rows of it are
 // cleared; the first chunk of slice s + 2 (sl2) requested into r.w[1-P].
 // sl1, sl2 advance by one slice.
-template <int E, int P>
-__device__ __forceinline__ void pk_dround(const PkCtx &c, PkDRegs<E> &r, int dw, int64_t s, uint2 &sl1, uint2 &sl2) {
+template <int P>
+__device__ __forceinline__ void pk_dround(const PkCtx &c, PkDRegs &r, int dw, int64_t s, uint2 &sl1, uint2 &sl2) {
     unsigned char *nxt = c.smem + (1 - P) * c.img_bytes;
     const int64_t s3 = s + 3;
     const uint2 s3m = pk_slice_meta(c, s3);
-    pk_load_chunk<E>(r.w[1 - P], pk_stream<E>(c, sl2, dw).rs, c, 0);
+    pk_load_chunk(r.w[1 - P], pk_stream(c, sl2, dw).rs, c, 0);
     pk_clear(c, nxt);
-    pk_expand<E>(c, r.w[P], pk_stream<E>(c, sl1, dw), nxt);
+    pk_expand(c, r.w[P], pk_stream(c, sl1, dw), nxt);
     sl1 = sl2;
     sl2 = s3 < c.end ? s3m : make_uint2(0u, 0u);
     lds_barrier();  // the next slice's image complete
@@ -529,9 +537,9 @@ __device__ __forceinline__ void pk_dround(const PkCtx &c, PkDRegs<E> &r, int dw,
 // each round (the MFMA wavefronts wait at its barrier), so their
 // instructions, mostly LDS stores, issue first; with two MFMA wavefronts per
 // SIMD these bound it, and the decode keeps the default priority.
-template <int E, bool RAISE>
+template <bool RAISE>
 __device__ __forceinline__ void pk_dmain(const PkCtx &c, int dw, int64_t s) {
-    PkDRegs<E> r;
+    PkDRegs r;
     if constexpr (RAISE) __builtin_amdgcn_s_setprio(2);
     pk_clear(c, c.smem);  // image 0's rows of this wavefront hold the background
     const uint2 s0m = pk_slice_meta(c, s);
@@ -539,21 +547,21 @@ __device__ __forceinline__ void pk_dmain(const PkCtx &c, int dw, int64_t s) {
     uint2 sl1 = s + 1 < c.end ? s1m : make_uint2(0u, 0u);
     uint2 sl2 = s + 2 < c.end ? s2m : make_uint2(0u, 0u);
     {
-        uint32_t w0[E];
-        const PkStream st0 = pk_stream<E>(c, s0m, dw);
-        pk_load_chunk<E>(w0, st0.rs, c, 0);
-        pk_load_chunk<E>(r.w[0], pk_stream<E>(c, sl1, dw).rs, c, 0);
+        pv3u w0[kPkChunk];
+        const PkStream st0 = pk_stream(c, s0m, dw);
+        pk_load_chunk(w0, st0.rs, c, 0);
+        pk_load_chunk(r.w[0], pk_stream(c, sl1, dw).rs, c, 0);
         lds_barrier();  // (the MFMA wavefronts' first barrier)
-        pk_expand<E>(c, w0, st0, c.smem);
+        pk_expand(c, w0, st0, c.smem);
     }
     lds_barrier();  // the first slice expanded
-    pk_dround<E, 0>(c, r, dw, s, sl1, sl2);
+    pk_dround<0>(c, r, dw, s, sl1, sl2);
     ++s;
     for (;;) {
         if (s >= c.end) return;
-        pk_dround<E, 1>(c, r, dw, s, sl1, sl2);
+        pk_dround<1>(c, r, dw, s, sl1, sl2);
         if (++s >= c.end) return;
-        pk_dround<E, 0>(c, r, dw, s, sl1, sl2);
+        pk_dround<0>(c, r, dw, s, sl1, sl2);
         ++s;
     }
 }
@@ -581,7 +589,7 @@ __device__ __forceinline__ void pk_dmain(const PkCtx &c, int dw, int64_t s) {
 // rt*32 + l%32 at column kb*32 + (l/32)*16: with stride/4 = 8m + 4, any 8
 // consecutive lanes read disjoint banks.  The query table pairs each B byte
 // with the same column.
-template <int E, int KB, int MODE>
+template <int KB, int MODE>
 __global__ __launch_bounds__(PkShape::threads(MODE))
 __attribute__((amdgpu_waves_per_eu(PkShape::waves_per_eu(MODE), PkShape::waves_per_eu(MODE)))) void pk_scores(
     DenseArgs a) {
@@ -607,23 +615,11 @@ __attribute__((amdgpu_waves_per_eu(PkShape::waves_per_eu(MODE), PkShape::waves_p
     const int mw = a.NT / (MODE == 2 ? 2 : 1);                         // MFMA wavefronts
     c.wrow = (uint32_t)(wave - mw) * 16u * c.stride;                   // decode wavefronts' rows
     c.a_base = (uint32_t)(lane & 31) * c.stride + (uint32_t)hi * 16u;  // A operand of row tile 0
-    c.ob = a.pcb;
     c.meta = __builtin_amdgcn_make_buffer_rsrc((void *)a.pslices, (short)0, (int)(a.nslices * 8),
                                                0x00020000 /* 32-bit data format */);
-    if (wave >= mw) pk_dmain<E, MODE != 3>(c, wave - mw, s0);
+    if (wave >= mw) pk_dmain<MODE != 3>(c, wave - mw, s0);
     else if constexpr (MODE == 0) pk_mmain<KB>(c, qb, wave, s0);
     else if constexpr (MODE == 1) pk_mmainh<KB, 1>(c, qb, wave, s0);
     else if constexpr (MODE == 3) pk_mmains<KB>(c, qb, wave, s0);
     else pk_mmainh<KB, 2>(c, qb, 2 * wave, s0);
 }
-
-#define PK_CASES(KB, MODE)                       \
-    switch (E) {                                \
-        case 18: return pk_scores<18, KB, MODE>; \
-        case 19: return pk_scores<19, KB, MODE>; \
-        case 20: return pk_scores<20, KB, MODE>; \
-        case 21: return pk_scores<21, KB, MODE>; \
-        case 22: return pk_scores<22, KB, MODE>; \
-        case 23: return pk_scores<23, KB, MODE>; \
-        default: return nullptr;                \
-    }

@@ -3,4 +3,4 @@
 // one translation unit each, for build parallelism).
 #include "k_pkmfma.hpp"
 
-dense_fn get_pk_scores_8(int E) { PK_CASES(8, 1) }
+dense_fn get_pk_scores_8() { return pk_scores<8, 1>; }

@@ -2,4 +2,4 @@
 // (one translation unit each, for build parallelism).
 #include "k_pkmfma.hpp"
 
-dense_fn get_pk_scores_30(int E) { PK_CASES(30, 0) }
+dense_fn get_pk_scores_30() { return pk_scores<30, 0>; }

@@ -3,4 +3,4 @@
 // parallelism).
 #include "k_pkmfma.hpp"
 
-dense_fn get_pk2_scores_8(int E) { PK_CASES(8, 2) }
+dense_fn get_pk2_scores_8() { return pk_scores<8, 2>; }

@@ -3,4 +3,4 @@
 // parallelism).
 #include "k_pkmfma.hpp"
 
-dense_fn get_pk2_scores_16(int E) { PK_CASES(16, 2) }
+dense_fn get_pk2_scores_16() { return pk_scores<16, 2>; }

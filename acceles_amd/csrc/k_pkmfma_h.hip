@@ -3,6 +3,6 @@
 // translation unit, for build parallelism).
 #include "k_pkmfma.hpp"
 
-dense_fn get_pk3_scores_24(int E) { PK_CASES(24, 3) }
-dense_fn get_pk3_scores_30(int E) { PK_CASES(30, 3) }
-dense_fn get_pk3_scores_32(int E) { PK_CASES(32, 3) }
+dense_fn get_pk3_scores_24() { return pk_scores<24, 3>; }
+dense_fn get_pk3_scores_30() { return pk_scores<30, 3>; }
+dense_fn get_pk3_scores_32() { return pk_scores<32, 3>; }

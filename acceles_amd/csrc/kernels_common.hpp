@@ -716,11 +716,10 @@ static constexpr int kPkDecodeWaves = 4;
 struct DenseArgs {
     const uint32_t *words;       // sliced packets
     const uint2 *slices;
-    const uint32_t *pwords;      // image packets (pk_scores): (byte, offset in a decode wavefront's
-                                 // 16 image rows) entries of pcb + 8 bits, one stream per wavefront
-    const uint2 *pslices;        // per slice: (offset in units of 64 dwords, entries per lane / 4 of
-                                 // decode wavefront w in byte w)
-    int pcb;                     // offset bits
+    const uint32_t *pwords;      // image packets (pk_scores): groups of four (offset in a decode
+                                 // wavefront's 16 image rows, byte) entries per lane, 3 dwords, one
+                                 // stream per wavefront
+    const uint2 *pslices;        // per slice: (offset in groups, groups of decode wavefront w in byte w)
     const int32_t *perm;
     const int64_t *part_slice;   // split + 1
     const uint8_t *nvalid;       // valid rows per slice (a prefix of its lanes)
@@ -784,13 +783,13 @@ dense_fn get_dense_prep();                                     // k_dense.hip
 dense_fn get_dense_select(int64_t part_slices, int M);
 dense_fn get_batch_topk_radix(int V);
 dense_fn get_batch_topk(int R);
-dense_fn get_pk_scores_8(int E);                               // k_pkmfma_a.hip
-dense_fn get_pk_scores_16(int E);                              // k_pkmfma_b.hip
-dense_fn get_pk_scores_32(int E);                              // k_pkmfma_c.hip
-dense_fn get_pk_scores_24(int E);                              // k_pkmfma_d.hip
-dense_fn get_pk_scores_30(int E);                              // k_pkmfma_e.hip
-dense_fn get_pk2_scores_8(int E);                              // k_pkmfma_f.hip
-dense_fn get_pk2_scores_16(int E);                             // k_pkmfma_g.hip
-dense_fn get_pk3_scores_24(int E);                             // k_pkmfma_h.hip
-dense_fn get_pk3_scores_30(int E);
-dense_fn get_pk3_scores_32(int E);
+dense_fn get_pk_scores_8();                               // k_pkmfma_a.hip
+dense_fn get_pk_scores_16();                              // k_pkmfma_b.hip
+dense_fn get_pk_scores_32();                              // k_pkmfma_c.hip
+dense_fn get_pk_scores_24();                              // k_pkmfma_d.hip
+dense_fn get_pk_scores_30();                              // k_pkmfma_e.hip
+dense_fn get_pk2_scores_8();                              // k_pkmfma_f.hip
+dense_fn get_pk2_scores_16();                             // k_pkmfma_g.hip
+dense_fn get_pk3_scores_24();                             // k_pkmfma_h.hip
+dense_fn get_pk3_scores_30();
+dense_fn get_pk3_scores_32();

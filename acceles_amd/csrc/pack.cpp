@@ -269,15 +269,14 @@ bool wave_image_entries(const acc_packed *pk, int64_t s, int w, int u8off, uint3
 
 }  // namespace
 
-int acc::image_packets(const acc_packed *pk, int u8off, int ob, uint32_t stride, std::vector<uint32_t> &words,
+int acc::image_packets(const acc_packed *pk, int u8off, uint32_t stride, std::vector<uint32_t> &words,
                        std::vector<std::pair<uint32_t, uint32_t>> &slices) {
     const int64_t NS = pk->nslices();
-    const int E = ob + 8;
-    if (ob < 1 || E > 32 || (int64_t(16) * stride) > (int64_t(1) << ob) || (int64_t)stride <= pk->cols)
-        return fail(ACC_ERR_ARG, "image packets: offset bits");
+    if (16 * (int64_t)stride > 65536 || (int64_t)stride <= pk->cols)
+        return fail(ACC_ERR_ARG, "image packets: offsets past 16 bits");
     slices.assign((size_t)NS, {0u, 0u});
-    // per slice and wavefront: entries per lane, a multiple of 4 (<= 256)
-    std::vector<uint32_t> n4((size_t)NS * 4, 0);
+    // per slice and wavefront: groups of four entries per lane (<= 64)
+    std::vector<uint32_t> groups((size_t)NS * 4, 0);
     int bad = 0;
 #pragma omp parallel
     {
@@ -288,26 +287,24 @@ int acc::image_packets(const acc_packed *pk, int u8off, int ob, uint32_t stride,
         for (int64_t s = 0; s < NS; ++s)
             for (int w = 0; w < 4; ++w) {
                 if (!wave_image_entries(pk, s, w, u8off, stride, ent, row, out)) bad = 1;
-                const uint64_t n = (out.size() + 63) / 64;
-                n4[(size_t)s * 4 + w] = (uint32_t)((n + 3) / 4 * 4);
+                groups[(size_t)s * 4 + w] = (uint32_t)((out.size() + 255) / 256);
             }
     }
     if (bad) return fail(ACC_ERR_RANGE, "image packets: a row's values in one column sum past one byte");
-    auto ndw_of = [E](uint32_t n) { return (n * (uint32_t)E + 31u) / 32u; };
     uint64_t off = 0;
     for (int64_t s = 0; s < NS; ++s) {
-        uint32_t ndw = 0, packed = 0;
+        uint32_t n = 0, packed = 0;
         for (int w = 0; w < 4; ++w) {
-            const uint32_t n = n4[(size_t)s * 4 + w];
-            if (n > 256) return fail(ACC_ERR_RANGE, "image packets: more than 256 entries per lane");
-            ndw += ndw_of(n);
-            packed |= (n / 4) << (8 * w);
+            const uint32_t g = groups[(size_t)s * 4 + w];
+            if (g > 64) return fail(ACC_ERR_RANGE, "image packets: more than 256 entries per lane");
+            n += g;
+            packed |= g << (8 * w);
         }
-        if (off + ndw > 0xFFFFFFFFull) return fail(ACC_ERR_RANGE, "image packets exceed 2^40 bytes");
+        if (off + n > 0xFFFFFFFFull) return fail(ACC_ERR_RANGE, "image packets exceed 3 * 2^40 bytes");
         slices[(size_t)s] = {(uint32_t)off, packed};
-        off += ndw;
+        off += n;
     }
-    words.assign((size_t)off * 64, 0u);
+    words.assign((size_t)off * 192, 0u);
 #pragma omp parallel
     {
         std::vector<std::pair<int32_t, int32_t>> ent;
@@ -315,26 +312,25 @@ int acc::image_packets(const acc_packed *pk, int u8off, int ob, uint32_t stride,
         std::vector<uint32_t> out;
 #pragma omp for schedule(dynamic, 64)
         for (int64_t s = 0; s < NS; ++s) {
-            uint32_t *base = words.data() + (size_t)slices[(size_t)s].first * 64;
+            uint32_t *base = words.data() + (size_t)slices[(size_t)s].first * 192;
             for (int w = 0; w < 4; ++w) {
-                const uint32_t n = n4[(size_t)s * 4 + w];
+                const uint32_t n = 4 * groups[(size_t)s * 4 + w];
                 if (n == 0) continue;
                 wave_image_entries(pk, s, w, u8off, stride, ent, row, out);
                 // lane l takes entries l*m .. l*m + m-1 of the wavefront's
                 // list, m = ceil(size / 64) (so one store instruction spreads
                 // over the rows); its slots m .. n-1 repeat entries of the next
                 // lanes, wrapping round to the list's start (the same byte to
-                // the same place again, never twice in one instruction)
+                // the same place again)
                 const size_t m = (out.size() + 63) / 64;
                 for (uint32_t j = 0; j < n; ++j)
                     for (int l = 0; l < 64; ++l) {
-                        const size_t i = (size_t)l * m + j;
-                        const uint32_t v = out[i % out.size()];
-                        const uint32_t pos = j * (uint32_t)E, wi = pos >> 5, sh = pos & 31;
-                        base[(size_t)wi * 64 + l] |= v << sh;
-                        if (sh + E > 32) base[(size_t)(wi + 1) * 64 + l] |= v >> (32 - sh);
+                        const uint32_t v = out[((size_t)l * m + j) % out.size()];
+                        uint32_t *g = base + (size_t)(j / 4) * 192 + (size_t)l * 3;
+                        g[(j / 2) & 1] |= (v >> 8) << (16 * (j & 1));
+                        g[2] |= (v & 0xFFu) << (8 * (j & 3));
                     }
-                base += (size_t)ndw_of(n) * 64;
+                base += (size_t)n * 48;
             }
         }
     }

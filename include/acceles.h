@@ -324,7 +324,7 @@ int acc_gpu_topk_lowbit_batch(acc_gpu_matrix *m, const float *x_dev, int nq,
  * v_mfma_i32_32x32x32_i8: each 64-row slice is expanded into an int8 image
  * in LDS, one byte per (row, column), inside the scoring kernel, from the
  * handle's image packets -- the packets re-encoded at upload with each
- * entry's place in the image, 18 to 23 bits per entry,
+ * entry's place in the image, 24 bits per entry,
  * acc_gpu_info_t.dense_bytes).  Both give the same integer
  * scores and the same results.  ACC_BATCH_DENSE fails with a message when
  * the matrix cores cannot score the matrix exactly (a row whose values in one
