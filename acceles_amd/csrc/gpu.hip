@@ -578,7 +578,7 @@ size_t radix_select_keys(int64_t n, int K) {
 
 // Keys of an FP32 query's selection buffer: the radix passes', or the two
 // largest of every wavefront's rows.
-size_t fp32_sel_keys(int64_t rows) { return std::max<size_t>(radix_select_keys(rows, 256), 2 * kMaxGroups); }
+size_t fp32_sel_keys(int64_t rows) { return std::max<size_t>(radix_select_keys(rows, 256), 3 * kMaxGroups); }
 
 // Radix Top-K (K <= 256) of n scores; buf holds radix_select_keys(n, K) keys.
 int launch_select_radix(const float *y, int64_t n, int K, uint64_t *buf, acc_element *out, hipStream_t st,
@@ -1121,9 +1121,9 @@ static int spmv_shape(acc_gpu_matrix *m, SpmvShapeH &h) {
 }
 
 static int launch_spmv_fp32(acc_gpu_matrix *m, const SpmvShapeH &h, const float *x_dev, float *y, uint64_t *gmax,
-                            hipStream_t st) {
+                            bool wg_groups, hipStream_t st) {
     LAUNCH(m, 0, h.fn, dim3(h.blocks), dim3(ACC_WG), h.lds, st, m->d_ptr, m->d_idx, m->d_val, x_dev, m->rows, m->cols,
-           y, gmax);
+           y, gmax, wg_groups ? 1 : 0);
     return check_launch();
 }
 
@@ -1146,9 +1146,15 @@ static int launch_fp32_topk(acc_gpu_matrix *m, const float *x_dev, int K, const 
     SpmvShapeH h;
     int rc = spmv_shape(m, h);
     if (rc != ACC_OK) return rc;
-    const int nw = h.blocks * ACC_WAVES;
-    const bool groups = std::min<int64_t>(h.steps, nw) >= K;
-    rc = launch_spmv_fp32(m, h, x_dev, w.y, groups ? w.rsel : nullptr, st);
+    // Groups of the selection: workgroups where a third row of the Top-K in one
+    // group is rare (K^3 / 6 blocks^2 of them expected), since the selection reads
+    // a quarter of the keys then (2M x 900, K = 100: 9 against 15 us), else
+    // wavefronts (5M power-law rows, K = 500: 16 us, from workgroups 32)
+    const bool wg_groups = (int64_t)K * K * K <= (int64_t)h.blocks * h.blocks &&
+                           std::min<int64_t>((h.steps + ACC_WAVES - 1) / ACC_WAVES, h.blocks) >= K;
+    const int per = wg_groups ? ACC_WAVES : 1, nw = h.blocks * ACC_WAVES / per;
+    const bool groups = wg_groups || std::min<int64_t>(h.steps, nw) >= K;
+    rc = launch_spmv_fp32(m, h, x_dev, w.y, groups ? w.rsel : nullptr, wg_groups, st);
     if (rc == ACC_OK && between && hipEventRecord(between, st) != hipSuccess) rc = fail(ACC_ERR_DEVICE, "hipEventRecord failed");
     if (rc != ACC_OK) return rc;
     if (!groups)
@@ -1157,8 +1163,8 @@ static int launch_fp32_topk(acc_gpu_matrix *m, const float *x_dev, int K, const 
     SelectGroupsArgs a;
     a.gmax = w.rsel;
     a.nw = nw;
-    a.gsteps = (int)((h.steps + nw - 1) / nw);
-    a.RS = h.RS;
+    a.gsteps = (int)((h.steps + (int64_t)nw * per - 1) / ((int64_t)nw * per));
+    a.RS = h.RS * per;
     a.y = w.y;
     a.rows = m->rows;
     a.K = K;
@@ -1178,7 +1184,7 @@ extern "C" int acc_gpu_spmv_fp32(acc_gpu_matrix *m, const float *x_dev, float *y
     HIP_TRY(hipSetDevice(m->device));
     SpmvShapeH h;
     int rc = spmv_shape(m, h);
-    return rc == ACC_OK ? launch_spmv_fp32(m, h, x_dev, y_dev, nullptr, (hipStream_t)stream) : rc;
+    return rc == ACC_OK ? launch_spmv_fp32(m, h, x_dev, y_dev, nullptr, false, (hipStream_t)stream) : rc;
 }
 
 extern "C" int acc_gpu_topk_fp32(acc_gpu_matrix *m, const float *x_dev, int k, acc_element *out_dev, void *stream) {

@@ -68,13 +68,17 @@ int fp32_step_blocks(int G, double mean_row) {
     return std::max(1, (int)std::min(4.0, 0.85 * kFp32Stage / per_block));
 }
 
-// With gmax, wavefront w also leaves the two largest ranking keys of its rows
-// (gmax[w] and gmax[wavefronts + w], 0 without such a row) for
-// fp32_select_groups.  A key of 1 stands for a score whose order is 0 or 1 (a
+// With gmax, group w also leaves the three largest ranking keys of its rows
+// (gmax[w] and the pair at gmax[group_pairs(groups) + 2w], 0 without such a row) for
+// fp32_select_groups; a group is a wavefront, or with wg_groups a workgroup.
+// Each lane of a row's group holds the row's sum, so lane
+// g of the group takes block g's row: one update of a lane's best keys per step
+// instead of one per block.  A key of 1 stands for a score whose order is 0 or 1 (a
 // NaN of all ones).
 template <int G, int B>
 __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const colx_t *idx, const float *val,
-                                                   const float *x, int rows, int cols, float *y, uint64_t *gmax) {
+                                                   const float *x, int rows, int cols, float *y, uint64_t *gmax,
+                                                   int wg_groups) {
     using S = SpmvShape<G, B>;
     constexpr int RPI = S::RPI, RS = S::RS, NP = S::NP, U = S::U, kTail = S::kTail;
     static_assert(U * G <= kFp32Slack, "a batch stays in the slack");
@@ -101,18 +105,14 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
     __syncthreads();
     const int nsteps = (int)(((int64_t)rows + RS - 1) / RS);
     const int gw = blockIdx.x * ACC_WAVES + wave, nw = gridDim.x * ACC_WAVES;
-    if (gw >= nsteps) {
-        if (gmax && lane < 2) gmax[(size_t)lane * nw + gw] = 0ull;
-        return;
-    }
-    // the two best scores (ordered) and their rows of this lane so far
-    uint32_t top = 0u, toprow = 0u, sec = 0u, secrow = 0u;
+    // the three best scores (ordered) and their rows of this lane so far
+    uint32_t top = 0u, toprow = 0u, sec = 0u, secrow = 0u, thd = 0u, thdrow = 0u;
 
     typedef uint32_t v4 __attribute__((ext_vector_type(4)));
     constexpr int NV = (kFp32Stage + 255) / 256, NC = (kFp32Stage + 511) / 512;
     v4 lv[NV], lc[NC];
     auto load_starts = [&](int s, uint32_t (&p)[NP]) {  // row starts of step s (past the matrix: nnz)
-        const int r0 = min(s, nsteps - 1) * RS;
+        const int r0 = max(min(s, nsteps - 1), 0) * RS;
 #pragma unroll
         for (int i = 0; i < NP; ++i) p[i] = ptr[(int)min((int64_t)r0 + i * 64 + lane, (int64_t)rows)];
     };
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
     load_starts(gw, pc);
     load_starts(gw + nw, pn);
     issue(first(pc), last(pc));
-    for (int s = gw;;) {
+    for (int s = gw; s < nsteps;) {  // (none for wavefronts past the last step)
         const uint32_t sa = first(pc) & ~7u;
         const bool staged = fits(first(pc), last(pc));
         stage();
@@ -250,15 +250,24 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
                 for (int k = U * G; __any(n[t] > k); k += kTail * G) batch(one, tail, o + t, n + t, k, p + t);
         }
 #pragma unroll
-        for (int t = 0; t < B; ++t) {
-            p[t] = butterfly<G>(p[t]);
-            const int64_t r = (int64_t)s * RS + t * RPI + grp;
-            if (g == 0 && r < rows) y[r] = p[t];
+        for (int t = 0; t < B; ++t) p[t] = butterfly<G>(p[t]);
+#pragma unroll
+        for (int t0 = 0; t0 < B; t0 += G) {  // lane g of a group: block t0 + g
+            float v = p[t0];
+#pragma unroll
+            for (int t = 1; t < G; ++t)
+                if (t0 + t < B) v = g == t ? p[t0 + t] : v;
+            const int64_t r = (int64_t)s * RS + (t0 + g) * RPI + grp;
+            const bool mine = t0 + g < B && r < rows;
+            if (mine) y[r] = v;
             // rows ascend, so an equal score keeps the lower row
-            const uint32_t o = g == 0 && r < rows ? max(dordered_f32(p[t]), 1u) : 0u;
-            secrow = o > top ? toprow : o > sec ? (uint32_t)r : secrow;
+            const uint32_t o = mine ? max(dordered_f32(v), 1u) : 0u;
+            const bool b1 = o > top, b2 = o > sec, b3 = o > thd;
+            thdrow = b2 ? secrow : b3 ? (uint32_t)r : thdrow;
+            thd = max(thd, min(sec, o));
+            secrow = b1 ? toprow : b2 ? (uint32_t)r : secrow;
             sec = max(sec, min(top, o));
-            toprow = o > top ? (uint32_t)r : toprow;
+            toprow = b1 ? (uint32_t)r : toprow;
             top = max(top, o);
         }
         if (!more) break;
@@ -271,38 +280,59 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
         }
     }
     if (gmax) {
-        uint64_t best[2];
+        uint64_t best[3];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < 3; ++i) {
             const uint32_t m = wave_umax(top);
             const uint32_t lo = wave_umax(top == m ? 0xFFFFFFFFu - toprow : 0u);
             best[i] = m <= 1u ? (uint64_t)m : ((uint64_t)m << 32) | lo;
             if (top == m && 0xFFFFFFFFu - toprow == lo) {  // one lane: rows are distinct
                 top = sec;
                 toprow = secrow;
+                sec = thd;
+                secrow = thdrow;
             }
         }
-        if (lane < 2) gmax[(size_t)lane * nw + gw] = lane == 0 ? best[0] : best[1];
+        int w = gw, n = nw, t = lane;
+        uint64_t key = lane == 0 ? best[0] : lane == 1 ? best[1] : best[2];
+        if (wg_groups) {  // the workgroup's best of its wavefronts' keys, ranked by counting
+            __shared__ uint64_t s_best[3 * ACC_WAVES];
+            if (lane < 3) s_best[wave * 3 + lane] = key;
+            __syncthreads();
+            w = blockIdx.x;
+            n = gridDim.x;
+            t = 3;
+            if (threadIdx.x < 3 * ACC_WAVES) {
+                key = s_best[threadIdx.x];
+                t = 0;
+                for (int i = 0; i < 3 * ACC_WAVES; ++i)
+                    t += s_best[i] > key || (s_best[i] == key && i < (int)threadIdx.x);  // equal: zeros and ones
+            }
+        }
+        if (t < 3) gmax[t == 0 ? (size_t)w : group_pairs(n) + 2 * (size_t)w + t - 1] = key;
     }
 }
 
-// Top-K (K <= 960) of the scores y from the two largest keys of each
-// wavefront's rows (a group; one workgroup): T, the K-th largest of the groups'
-// best keys, is reached by K distinct rows, so every row of the Top-K has a
-// key >= T and lies in one of the K groups whose best reaches it.  Their best
-// keys, and their second ones that reach T, are listed in LDS; only a group
-// whose second key reaches T can hold more such rows and is read from y (the
-// steps are dealt in turn, so neighbouring rows lie in different groups and
-// few groups are read).  The listed keys are ranked.  A list that does not fit
-// (an order of rows that puts most of the best ones into the same groups) is
-// cut by a radix selection over the rows of the K groups.
+// Top-K (K <= 960) of the scores y from the three largest keys of
+// each group's rows (one workgroup): T, at most the K-th largest of
+// the groups' best keys, is reached by K distinct rows, so every row of the
+// Top-K has a key >= T and lies in one of the groups whose best reaches it (at
+// most K + kSelSlack).  Their best keys, and their second ones that reach T, are
+// listed in LDS; only a group whose third key reaches T can hold more such rows
+// and is read from y (the steps are dealt in turn, so neighbouring rows lie in
+// different groups and hardly any is read).  The listed keys are ranked.  A list
+// that does not fit (an order of rows that puts most of the best ones into the
+// same groups) is cut by a radix selection over the rows of those groups.
 //
 // Bound: latency, and what one CU reads: at 2,000,000 rows and K = 100 it
-// takes 17 us, reading all K groups' rows took 53 (12 GB/s of scattered rows).
+// takes 9 us (at 100,000 rows 6), from wavefronts' instead of workgroups' keys
+// 15 (10).  With two keys per wavefront, and some groups read in every call, it
+// took 17 (11), reading all K groups' rows 53 (12 GB/s of scattered rows).
 // Before it, two radix passes over all scores and a final one took 32 us, and
 // above K = 256 the sorted lists of select_blocks and select_final 827 us
-// (4,999,999 rows, K = 500; 20 us here).
+// (4,999,999 rows, K = 500; 16 us here).
 static constexpr int kSelList = 4096;  // keys listed in LDS
+static constexpr int kSelSlack = 16;   // groups listed past the K-th, for one or two radix digits less
 
 template <int V>
 __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
@@ -315,9 +345,14 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
     uint64_t *s_key = (uint64_t *)smem, *s_top = s_key + kSelList;  // kSelList, then 1024 keys
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint32_t nw = (uint32_t)a.nw, RS = (uint32_t)a.RS, rows = (uint32_t)a.rows;
+    // all keys are loaded at once; the second and third ones arrive during the
+    // radix selection of the best ones
     uint64_t k[V];
+    ulonglong2 k23[V];
 #pragma unroll
     for (int u = 0; u < V; ++u) k[u] = a.gmax[min((uint32_t)(tid + u * 1024), nw - 1u)];
+#pragma unroll
+    for (int u = 0; u < V; ++u) k23[u] = ((const ulonglong2 *)(a.gmax + group_pairs(a.nw)))[min((uint32_t)(tid + u * 1024), nw - 1u)];
 #pragma unroll
     for (int u = 0; u < V; ++u)
         if ((uint32_t)(tid + u * 1024) >= nw) k[u] = 0ull;
@@ -331,7 +366,10 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
 #pragma unroll
             for (int u = 0; u < V; ++u) fn(k[u]);
         },
-        a.K, hist, s_t, s_need);
+        a.K, hist, s_t, s_need, kSelSlack);
+#pragma unroll
+    for (int u = 0; u < V; ++u)  // not in the branches below, one wait each
+        asm volatile("" : "+v"(k23[u].x), "+v"(k23[u].y));
     // fewer than K groups with rows, or keys of 1 among the best: every group is read
     const bool all = T <= 1ull;
     auto append = [&](uint64_t key) {
@@ -343,20 +381,18 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
         for (int u = 0; u < V; ++u)
             if (k[u] >= T) {
                 append(k[u]);
+                const uint32_t w = (uint32_t)(tid + u * 1024);
                 const int j = atomicAdd(&s_m, 1);
-                if (j < 1024) s_group[j] = (uint32_t)(tid + u * 1024);  // K of them: the keys are distinct
+                if (j < 1024) s_group[j] = w;  // K + kSelSlack of them at most: the keys are distinct
+                if (k23[u].x >= T) append(k23[u].x);
+                if (k23[u].y >= T) {
+                    const int i = atomicAdd(&s_scans, 1);
+                    if (i < 1024) {
+                        s_scan[i] = w;
+                        s_below[i] = k23[u].x;
+                    }
+                }
             }
-        __syncthreads();
-        if (tid < min(s_m, 1024)) {
-            const uint32_t w = s_group[tid];
-            const uint64_t second = a.gmax[nw + w];
-            if (second >= T) {
-                append(second);
-                const int j = atomicAdd(&s_scans, 1);
-                s_scan[j] = w;
-                s_below[j] = second;
-            }
-        }
     }
     __syncthreads();
     // fn(key) for every row of groups group(0 .. nl-1) (0: no row).  A
@@ -398,7 +434,7 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
     };
     if (!all)
         scan(
-            s_scans, [&](int i) { return s_scan[i]; },
+            min(s_scans, 1024), [&](int i) { return s_scan[i]; },
             [&](uint64_t key, int i) {
                 if (key >= T && key < s_below[i]) append(key);
             });
@@ -435,18 +471,26 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
         if (tid < n) s_key[tid] = s_top[tid];
         __syncthreads();
     }
-    const uint64_t key = tid < n ? s_key[tid] : 0ull;
     int rank = 0;
-    if (n <= 256) {  // ranks by counting, two keys per read
-        if (tid < 2) s_key[n + tid] = 0ull;
+    if (n <= 256) {  // ranks by counting: four lanes per key, two keys per read
+        if (tid < 8) s_key[n + tid] = 0ull;
         __syncthreads();
-        if (tid < n)
-            for (int j = 0; j < n; j += 2) {
-                const ulonglong2 o = *(const ulonglong2 *)(s_key + j);
-                rank += (o.x > key) + (o.y > key);
-            }
+        const int i = tid >> 2;
+        const uint64_t mine = s_key[min(i, n)];
+        for (int j = (tid & 3) * 2; j < n; j += 8) {
+            const ulonglong2 o = *(const ulonglong2 *)(s_key + j);
+            rank += (o.x > mine) + (o.y > mine);
+        }
+        rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+        rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xF, 0xF, false);  // lane ^ 2
+        if ((tid & 3) == 0 && i < n && rank < a.K) {
+            acc_element e;
+            e.value = dkey_score_f32(mine);
+            e.index = dkey_row(mine);
+            a.out[rank] = e;
+        }
     } else {  // each wavefront sorts its keys; a key's rank: its places in the sorted lists
-        uint64_t v[1] = {key};
+        uint64_t v[1] = {tid < n ? s_key[tid] : 0ull};
         reg_sort_desc<1>(v);
         s_top[tid] = v[0];
         __syncthreads();
@@ -468,12 +512,6 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
             e.index = dkey_row(mine);
             a.out[rank] = e;
         }
-    }
-    if (n <= 256 && tid < n && rank < a.K) {
-        acc_element e;
-        e.value = dkey_score_f32(key);
-        e.index = dkey_row(key);
-        a.out[rank] = e;
     }
     for (int i = n + tid; i < a.K; i += 1024) {
         acc_element e;

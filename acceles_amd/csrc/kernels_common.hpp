@@ -620,12 +620,14 @@ struct SelectArgs {
     acc_element *out;
 };
 
-// Top-K of the scores an fp32_spmv launch of nw wavefronts has just written,
-// from the two largest keys of each wavefront's rows (steps w, w + nw, ... of
-// wavefront w, at most gsteps, of RS rows each).
+// Top-K of the scores an fp32_spmv launch has just written, from the three
+// largest keys of the rows of its nw groups, wavefronts or workgroups (group w:
+// steps w, w + nw, ..., at most gsteps, of RS rows each; a workgroup's step is
+// its wavefronts' neighbouring steps).
 static constexpr int kMaxGroups = 8192;
+__host__ __device__ inline size_t group_pairs(int nw) { return ((size_t)nw + 1) & ~(size_t)1; }
 struct SelectGroupsArgs {
-    const uint64_t *gmax;  // 2 * nw keys
+    const uint64_t *gmax;  // nw best keys, then (16-byte aligned) nw pairs of second and third ones
     int nw, gsteps, RS;
     const float *y;
     int rows, K;
@@ -751,7 +753,8 @@ typedef void (*lowbit_fn)(LowbitArgs);
 typedef void (*scores_fn)(ScoresArgs);
 typedef void (*select_fn)(SelectArgs);
 typedef void (*batch_fn)(BatchArgs);
-typedef void (*spmv_fn)(const uint32_t *, const colx_t *, const float *, const float *, int, int, float *, uint64_t *);
+typedef void (*spmv_fn)(const uint32_t *, const colx_t *, const float *, const float *, int, int, float *, uint64_t *,
+                        int);
 typedef void (*select_groups_fn)(SelectGroupsArgs);
 typedef void (*reset_fn)(uint64_t *, uint32_t *);
 typedef void (*radix_pass_fn)(const void *, int64_t, int, uint64_t *);
