@@ -413,13 +413,14 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
 
 // Estimated time of a batch per layout, in us.  Measured (CK 512, K 100; batch
 // of 8, us single / packets / matrix cores): 20,000 x 500 175 / 70 / 43, 400,000
-// x 500 218 / 103 / 47, 1,000,000 x 250 4-bit 215 / 118 / 71, 2,000,000 x 900
-// 472 / 232 / 198, 5,000,000 x 1024 (20 entries per row) 472 / 302 / 488; one
-// query: 25 / 65 / 41, 31 / 98 / 47, 28 / 110 / 70, 59 / 221 / 201, 61 / 278
-// / 493.  So: a single query pays about 21 us and its packets at 7 TB/s; the
+// x 500 218 / 103 / 45, 1,000,000 x 250 4-bit 215 / 118 / 71, 2,000,000 x 900
+// 458 / 230 / 163, 5,000,000 x 1024 (20 entries per row) 468 / 296 / 402; one
+// query: 25 / 65 / 41, 31 / 98 / 47, 28 / 110 / 70, 60 / 215 / 164, 65 / 276
+// / 395.  So: a single query pays about 21 us and its packets at 7 TB/s; the
 // packet batch 55 us and 1.5 ns per 1,000 entries and 0.6 ns per slice for
 // every block of 16 or 32 queries; the matrix cores 33 us and per slice 2.4
-// ns up to 16 column blocks, 5.5 above (a 128-query block).
+// ns up to 16 column blocks, 5.5 above (a 128-query block), 4.6 up to 64 queries
+// (two wavefronts per query tile: 8 queries at 2M x 900: 198 -> 163 us).
 struct BatchCost {
     double single, sparse, dense;
 };
@@ -428,7 +429,7 @@ BatchCost batch_cost(const acc_gpu_matrix *m, int nq) {
     c.single = nq * (21.0 + (double)m->stream_bytes / 7e6);
     const int qb = nq <= 16 ? 16 : 32;
     c.sparse = 55.0 + (1.5e-6 * (double)m->nnz + 0.6e-3 * (double)m->nslices) * (qb / 16) * ((nq + qb - 1) / qb);
-    c.dense = 33.0 + (m->nkb <= 16 ? 2.4e-3 : 5.5e-3) * (double)m->nslices * ((nq + 127) / 128);
+    c.dense = 33.0 + (m->nkb <= 16 ? 2.4e-3 : nq <= 64 ? 4.6e-3 : 5.5e-3) * (double)m->nslices * ((nq + 127) / 128);
     return c;
 }
 
@@ -454,8 +455,15 @@ int batch_layout(const acc_gpu_matrix *m, int nq) {
 // two workgroups per CU (k_pkmfma_{a,b}), with two tiles (tpw = 2) each A
 // read feeds both (k_pkmfma_{f,g}).  Above 16 column blocks, a batch of more
 // than four tiles runs eight MFMA wavefronts per workgroup, two per SIMD
-// (wide, k_pkmfma_h): one decode of each slice for up to 256 queries.
-dense_fn pk_kernel(const acc_gpu_matrix *m, int tpw, bool wide) {
+// (wide, k_pkmfma_h): one decode of each slice for up to 256 queries.  rows: two
+// MFMA wavefronts per tile (k_pkmfma_{i,j}).
+dense_fn pk_kernel(const acc_gpu_matrix *m, int tpw, bool wide, bool rows) {
+    if (rows) {
+        if (m->nkb > 30) return get_pk4_scores_32();
+        if (m->nkb > 24) return get_pk4_scores_30();
+        if (m->nkb > 16) return get_pk4_scores_24();
+        return m->nkb > 8 ? get_pk4_scores_16() : get_pk4_scores_8();
+    }
     if (tpw == 2) return m->nkb > 8 ? get_pk2_scores_16() : get_pk2_scores_8();
     if (wide) return m->nkb > 30 ? get_pk3_scores_32() : m->nkb > 24 ? get_pk3_scores_30() : get_pk3_scores_24();
     if (m->nkb > 30) return get_pk_scores_32();
@@ -485,7 +493,13 @@ int launch_dense(acc_gpu_matrix *m, BatchWs &ws, const float *X, int nq, int M, 
     const int per_block = wide ? kPkMfmaWaves3 : kPkMfmaWaves * tpw;
     const int nqb = (tiles + per_block - 1) / per_block;
     const int NT = ((tiles + nqb - 1) / nqb + tpw - 1) / tpw * tpw, QB = 32 * NT;
-    const int W = NT / tpw + kPkDecodeWaves;
+    // up to two tiles: two MFMA wavefronts per tile, one per row tile (41 queries
+    // at 1M x 500 64.5 -> 57.7 us; up to 15% of a call at other widths).  One
+    // tile at 9 to 16 column blocks gains nothing (the decode bounds it: 47.6
+    // against 48.7 us at 400k x 500).  Three or four tiles above 16 column blocks
+    // on eight such wavefronts, two per SIMD, took 131 us against 123 (1M x 900)
+    const bool rows = tiles == 2 || (tiles == 1 && (m->nkb <= 8 || m->nkb > 16));
+    const int W = (rows ? 2 * NT : NT / tpw) + kPkDecodeWaves;
     const size_t cand = (size_t)nq * m->split * M;
     int rc = ws_grow(ws, &ws.qtab, &ws.qtab_n, (size_t)nqb * m->nkb * NT * 1024);
     if (rc == ACC_OK) rc = ws_grow(ws, &ws.qplain, &ws.qplain_n, (size_t)nq * m->cols_pad);
@@ -512,11 +526,11 @@ int launch_dense(acc_gpu_matrix *m, BatchWs &ws, const float *X, int nq, int M, 
 
     LAUNCH(m, 0, get_dense_prep(), dim3(nqb * QB), dim3(ACC_WG), 0, st, a);
     if ((rc = check_launch()) != ACC_OK) return rc;
-    dense_fn fs = pk_kernel(m, tpw, wide);
+    dense_fn fs = pk_kernel(m, tpw, wide, rows);
     if (!fs) return fail(ACC_ERR_ARG, "unsupported entry width");
     // two slice images (one multiplied while the other is cleared and refilled)
     const size_t img = (size_t)64 * (m->cols_pad + 16);
-    const size_t lds_s = 2 * img + kPkLdsTail;
+    const size_t lds_s = 2 * img + kPkLdsTail + (rows ? (size_t)NT * 2048 : 0);  // and the row tiles' lists
     if ((rc = lds_limit((const void *)fs, lds_s)) != ACC_OK) return rc;
     // workgroups per query block: as many as fit the chip at once, a multiple
     // of 8 (the kernel keeps a slice range's query blocks on one XCD)

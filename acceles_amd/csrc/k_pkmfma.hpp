@@ -98,8 +98,11 @@ struct PkShape {
     // slice, three wavefronts per SIMD
     static constexpr int threads(int mode) { return (mode == 3 ? 12 : kPkMfmaWaves + kPkDecodeWaves) * 64; }
     // two wavefronts per SIMD; four (two workgroups per CU) for the
-    // one-tile half-round chain, whose registers fit 128
-    static constexpr int waves_per_eu(int mode) { return mode == 1 ? 4 : mode == 3 ? 3 : 2; }
+    // one-tile half-round and row-tile chains at up to 16 column blocks, whose
+    // registers fit 128
+    static constexpr int waves_per_eu(int mode, int kb) {
+        return mode == 1 || (mode == 4 && kb <= 16) ? 4 : mode == 3 ? 3 : 2;
+    }
 };
 
 // Registers of an MFMA wavefront (one object, so that the compile-time steps
@@ -421,6 +424,118 @@ __device__ __forceinline__ void pk_mmains(const PkCtx &c, int qb, int tile, int6
     }
 }
 
+// The chain of MODE 4 (up to two query tiles): a tile's two row tiles of 32 rows
+// go to two MFMA wavefronts, so that the chain of a round is half as long: with
+// few tiles one wavefront per tile leaves SIMDs without an MFMA wavefront and
+// the others' chains bound the round.  pk_scores at 1M x 500 (signed 6-bit, 41
+// queries): 64.5 -> 57.7 us; calls of 4 and 64 queries at 1M x 900: 107 -> 94
+// and 117 -> 105, at 600k x 250: 54 -> 46.5 and 57 -> 53.5.  Round P multiplies slice s into acc[P] while it reduces acc[1-P] (slice s - 1) to
+// the list kk.
+struct PkMRegsR {
+    pv4i ar[4];       // A operands in flight (ring)
+    pv16i acc[2];     // [round parity]
+    int32_t kk[4];    // four-pre-key list of the previous slice
+};
+
+template <int KB, int P, bool LISTS, int kb>
+__device__ __forceinline__ void pk_rstep(PkMRegsR &r, const pv4i (&B)[KB], const pv4i *A) {
+    constexpr int RING = 4, DIST = 3;
+    if constexpr (kb + DIST < KB) r.ar[(kb + DIST) % RING] = A[(kb + DIST) * 2];
+    __builtin_amdgcn_sched_barrier(0);
+    r.acc[P] = __builtin_amdgcn_mfma_i32_32x32x32_i8(r.ar[kb % RING], B[kb], r.acc[P], 0, 0, 0);
+    // the previous slice's accumulators into the list, value v at step v*KB/16
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+        if (LISTS && v * KB / 16 == kb)
+            pk_top4s(r.kk[0], r.kk[1], r.kk[2], r.kk[3], pk_prekey(r.acc[1 - P][v], 0, v));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int KB, int P, bool LISTS, int... KBS>
+__device__ __forceinline__ void pk_rchain(std::integer_sequence<int, KBS...>, PkMRegsR &r, const pv4i (&B)[KB],
+                                          const pv4i *A) {
+    (pk_rstep<KB, P, LISTS, KBS>(r, B, A), ...);
+}
+
+// An MFMA wavefront of MODE 4: row tile w % 2 of query tile w / 2 over slices
+// s .. end-1 (the same barriers as pk_mmain, and one more after the last
+// round).  The list of slice j of row tile 1 (its pre-keys offset by 32 rows)
+// goes through LDS: written at the end of round j + 1 into slot j % 2, read by
+// row tile 0's wavefront at the start of round j + 2, which merges and stores it
+// while only one set of accumulators is live.
+template <int KB>
+__device__ __forceinline__ void pk_mmainr(const PkCtx &c, int w, int64_t s) {
+    const DenseArgs &a = *c.a;
+    w = __builtin_amdgcn_readfirstlane(w);
+    const int tile = w >> 1;
+    const bool low = (w & 1) == 0;
+    pv4i B[KB];
+    {
+        const pv4i *q = (const pv4i *)a.qtab + c.lane;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+            B[kb] = kb < a.nkb ? q[((size_t)kb * a.NT + tile) * 64] : (pv4i){0, 0, 0, 0};
+    }
+    const int q = tile * 32 + (c.lane & 31);
+    const uint32_t Dk = ((uint32_t)(a.corr[q] + (1 << 25)) << 6) + (uint32_t)(c.hi * 4);
+    const uint32_t a_base = c.a_base + (uint32_t)(w & 1) * 32u * c.stride;
+    pv4i *x = (pv4i *)(c.smem + 2u * c.img_bytes + kPkLdsTail) + tile * 128 + c.lane;  // slots x[0], x[64]
+    PkMRegsR r;
+    auto merge = [&](int32_t (&k)[4], const pv4i &o, int64_t sx) {  // row tile 1's list o into k, stored
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pk_top4s(k[0], k[1], k[2], k[3], o[i]);
+        pk_store_list(c, Dk, q, k[0], k[1], k[2], k[3], sx);
+    };
+    auto pass = [&](int slot) {
+        pv4i o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = (int32_t)((uint32_t)r.kk[i] + 32u);
+        x[64 * slot] = o;
+    };
+    auto round = [&](auto par, auto lists, bool two) {  // two: a slice before the previous one
+        constexpr int P = decltype(par)::value;
+        constexpr bool LISTS = decltype(lists)::value;
+        const pv4i *A = (const pv4i *)(c.smem + (uint32_t)P * c.img_bytes + a_base);
+        const pv4i o = x[64 * P];
+        r.ar[0] = A[0];
+        r.ar[1] = A[2];
+        r.ar[2] = A[4];
+        if (low && two) merge(r.kk, o, s - 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.kk[i] = INT32_MIN;
+        __builtin_amdgcn_sched_barrier(0);
+        r.acc[P] = (pv16i){0};
+        pk_rchain<KB, P, LISTS>(std::make_integer_sequence<int, KB>(), r, B, A);
+        if (LISTS && !low) pass(1 - P);
+        lds_barrier();  // this slice's image read, the next one written
+    };
+    auto last = [&](auto par, bool two) {  // slice s of parity par was the last
+        constexpr int P = decltype(par)::value;
+        if (low && two) merge(r.kk, x[64 * (1 - P)], s - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.kk[i] = INT32_MIN;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) pk_top4s(r.kk[0], r.kk[1], r.kk[2], r.kk[3], pk_prekey(r.acc[P][v], 0, v));
+        if (!low) pass(P);
+        lds_barrier();
+        if (low) merge(r.kk, x[64 * P], s);
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    const int64_t s0 = s;
+    lds_barrier();  // the images filled
+    lds_barrier();  // the first slice decoded
+    round(even, std::false_type{}, false);
+    for (;;) {
+        if (s + 1 >= c.end) return last(even, s > s0);
+        ++s;
+        round(odd, std::true_type{}, s - s0 >= 2);
+        if (s + 1 >= c.end) return last(odd, true);
+        ++s;
+        round(even, std::true_type{}, true);
+    }
+}
+
 // Decode wavefront dw owns rows 16*dw .. 16*dw + 15 of every image.  Its
 // stream of a slice holds the entries of those rows split among its lanes,
 // consecutive ones per lane, in groups of four per lane (the same number for
@@ -570,7 +685,8 @@ __device__ __forceinline__ void pk_dmain(const PkCtx &c, int dw, int64_t s) {
 // MFMA wavefronts of one tile each, or two, then kPkDecodeWaves decode
 // wavefronts).  MODE 0: one tile per MFMA wavefront, whole-slice rounds; 1:
 // one tile, half-rounds, registers for two workgroups per CU (up to 16
-// column blocks); 2: two tiles, half-rounds (up to 16 column blocks).
+// column blocks); 2: two tiles, half-rounds (up to 16 column blocks); 3: eight
+// wavefronts of one tile; 4: two wavefronts per tile, one row tile each.
 // Grid = nwx * nqb workgroups; the nqb blocks of one slice range
 // wx get workgroup ids 8 apart, hence one XCD, and the second and later
 // blocks find the packets in its L2.  Workgroup wx takes the slices wx*per
@@ -591,7 +707,7 @@ __device__ __forceinline__ void pk_dmain(const PkCtx &c, int dw, int64_t s) {
 // with the same column.
 template <int KB, int MODE>
 __global__ __launch_bounds__(PkShape::threads(MODE))
-__attribute__((amdgpu_waves_per_eu(PkShape::waves_per_eu(MODE), PkShape::waves_per_eu(MODE)))) void pk_scores(
+__attribute__((amdgpu_waves_per_eu(PkShape::waves_per_eu(MODE, KB), PkShape::waves_per_eu(MODE, KB)))) void pk_scores(
     DenseArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = (int)(threadIdx.x >> 6), lane = lane_id(), hi = lane >> 5;
@@ -612,12 +728,15 @@ __attribute__((amdgpu_waves_per_eu(PkShape::waves_per_eu(MODE), PkShape::waves_p
     c.stride = c.cols_pad + 16u;
     c.img_bytes = 64u * c.stride;
     c.fill = a.u8off ? 0x80808080u : 0u;                               // the image byte of an absent entry
-    const int mw = a.NT / (MODE == 2 ? 2 : 1);                         // MFMA wavefronts
+    const int mw = MODE == 4 ? 2 * a.NT : MODE == 2 ? a.NT / 2 : a.NT;  // MFMA wavefronts
     c.wrow = (uint32_t)(wave - mw) * 16u * c.stride;                   // decode wavefronts' rows
     c.a_base = (uint32_t)(lane & 31) * c.stride + (uint32_t)hi * 16u;  // A operand of row tile 0
     c.meta = __builtin_amdgcn_make_buffer_rsrc((void *)a.pslices, (short)0, (int)(a.nslices * 8),
                                                0x00020000 /* 32-bit data format */);
-    if (wave >= mw) pk_dmain<MODE != 3>(c, wave - mw, s0);
+    if (wave >= mw) {
+        pk_dmain<MODE != 3>(c, wave - mw, s0);
+        if constexpr (MODE == 4) lds_barrier();  // (the MFMA wavefronts' last one)
+    } else if constexpr (MODE == 4) pk_mmainr<KB>(c, wave, s0);
     else if constexpr (MODE == 0) pk_mmain<KB>(c, qb, wave, s0);
     else if constexpr (MODE == 1) pk_mmainh<KB, 1>(c, qb, wave, s0);
     else if constexpr (MODE == 3) pk_mmains<KB>(c, qb, wave, s0);

@@ -705,12 +705,13 @@ struct QTable {
 // (absent entries as -128) and 128 * sum(query) is added back per query;
 // other widths are stored as is.  Two images, then kPkLdsTail bytes that the
 // chain's reads of column blocks past nkb (multiplied by zero B operands)
-// may reach.
+// may reach, then with two wavefronts per tile 2 KB per tile for their lists.
 static constexpr int kPkLdsTail = 34 * 32;
 // pk_scores workgroups: up to kPkMfmaWaves MFMA wavefronts (one 32-query tile
 // each, or two where the B operands of two tiles fit the registers: up to 16
-// column blocks), or up to kPkMfmaWaves3 of one tile each (two per SIMD,
-// above 16 column blocks), and kPkDecodeWaves decode wavefronts.
+// column blocks), or two per tile of one row tile each (up to two tiles), or up
+// to kPkMfmaWaves3 of one tile each (two per SIMD, above 16 column blocks), and
+// kPkDecodeWaves decode wavefronts.
 static constexpr int kPkMfmaWaves = 4;
 static constexpr int kPkMfmaWaves3 = 8;
 static constexpr int kPkDecodeWaves = 4;
@@ -793,6 +794,11 @@ dense_fn get_pk_scores_24();                              // k_pkmfma_d.hip
 dense_fn get_pk_scores_30();                              // k_pkmfma_e.hip
 dense_fn get_pk2_scores_8();                              // k_pkmfma_f.hip
 dense_fn get_pk2_scores_16();                             // k_pkmfma_g.hip
+dense_fn get_pk4_scores_8();                              // k_pkmfma_i.hip
+dense_fn get_pk4_scores_16();
+dense_fn get_pk4_scores_24();                             // k_pkmfma_j.hip
+dense_fn get_pk4_scores_30();
+dense_fn get_pk4_scores_32();
 dense_fn get_pk3_scores_24();                             // k_pkmfma_h.hip
 dense_fn get_pk3_scores_30();
 dense_fn get_pk3_scores_32();
