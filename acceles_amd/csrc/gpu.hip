@@ -76,6 +76,7 @@ struct acc_gpu_matrix {
     int64_t nnz = 0;
     // FP32 CSR
     bool has_csr = false;
+    double row_sd = 0.0;  // standard deviation of the FP32 CSR's row lengths
     uint32_t *d_ptr = nullptr;
     colx_t *d_idx = nullptr;         // 4 * column per entry
     float *d_val = nullptr;
@@ -791,7 +792,14 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         m->nnz = nnz;
         m->group = choose_group(m->rows > 0 ? (double)nnz / m->rows : 1.0);
         std::vector<uint32_t> p32(csr->ptr.size());
-        for (size_t i = 0; i < p32.size(); ++i) p32[i] = (uint32_t)csr->ptr[i];
+        double sq = 0.0;
+        for (size_t i = 0; i < p32.size(); ++i) {
+            p32[i] = (uint32_t)csr->ptr[i];
+            const double len = i > 0 ? (double)(csr->ptr[i] - csr->ptr[i - 1]) : 0.0;
+            sq += len * len;
+        }
+        const double mean = m->rows > 0 ? (double)nnz / m->rows : 0.0;
+        m->row_sd = std::sqrt(std::max(0.0, sq / std::max(m->rows, 1) - mean * mean));
         TRY(dalloc(m, &m->d_ptr, p32.size()));
         TRY(dalloc(m, &m->d_idx, (size_t)nnz + kRowPad));
         TRY(dalloc(m, &m->d_val, (size_t)nnz + kRowPad));
@@ -1118,7 +1126,7 @@ struct SpmvShapeH {
 };
 
 static int spmv_shape(acc_gpu_matrix *m, SpmvShapeH &h) {
-    const int B = fp32_step_blocks(m->group, m->rows > 0 ? (double)m->nnz / m->rows : 0.0);
+    const int B = fp32_step_blocks(m->group, m->rows > 0 ? (double)m->nnz / m->rows : 0.0, m->row_sd);
     h.fn = get_fp32_spmv(m->group, B);
     if (!h.fn) return fail(ACC_ERR_ARG, "unsupported group size");
     h.RS = B * (64 / m->group);

@@ -62,10 +62,15 @@ struct SpmvShape {
 // staging area (row lengths vary; 75% and 95%, i.e. two and four blocks
 // instead of three, were slower at 2,000,000 x 900: 145 and 188 against 141
 // us), at most 4 blocks, so that a step's
-// registers leave five wavefronts per SIMD.
-int fp32_step_blocks(int G, double mean_row) {
-    const double per_block = std::max(mean_row, 1.0) * (64 / G);
-    return std::max(1, (int)std::min(4.0, 0.85 * kFp32Stage / per_block));
+// registers leave five wavefronts per SIMD.  One block less of three or four
+// where a step two standard deviations above the mean would not fit: a step that
+// exceeds the area waits for each of its blocks (power-law rows of 20 entries on
+// average, 5M x 1024: three blocks 196 us, four 209, two 215).
+int fp32_step_blocks(int G, double mean_row, double row_sd) {
+    const int RPI = 64 / G;
+    const double per_block = std::max(mean_row, 1.0) * RPI;
+    const int B = std::max(1, (int)std::min(4.0, 0.85 * kFp32Stage / per_block));
+    return B > 2 && B * per_block + 2.0 * row_sd * std::sqrt((double)B * RPI) > kFp32Stage ? B - 1 : B;
 }
 
 // With gmax, group w also leaves the three largest ranking keys of its rows
@@ -140,9 +145,10 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
         for (int i = 0; i < NC; ++i)
             *(v4 *)(sc + (i * 64 + lane) * 8) = lc[i];
     };
-    // Entries k .. of NT rows per lane, U per lane and row, added to p in order
-    // (base: the lane's first entry's place in the area, n: entries of its row
-    // from there on).  All reads are issued before the first is used; the
+    // Entries k .. of NT rows per lane, U per lane and row, added to p in order;
+    // slots past a row's end read x[0], one address for all (power-law rows,
+    // half of whose slots are: 212 -> 209 us) (base: the lane's first entry's
+    // place in the area, n: entries of its row from there on).  All reads are issued before the first is used; the
     // empty asm keeps them out of the branches that the masked additions
     // would otherwise become.
     auto batch = [&](auto nt, auto nu, const uint32_t *base, const int *n, int k, float *p) {
@@ -161,7 +167,7 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int u = 0; u < U; ++u) xv[t][u] = x_at(xs, c[t][u]);
+            for (int u = 0; u < U; ++u) xv[t][u] = x_at(xs, n[t] > k + u * G ? c[t][u] : (uint32_t)0);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll

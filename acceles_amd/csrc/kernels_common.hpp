@@ -768,7 +768,7 @@ lowbit_fn get_lowbit_final(int R);
 lowbit_fn get_lowbit_final_radix(int V);  // V = 1, 2, 4
 scores_fn get_lowbit_scores(int E, bool is_signed);
 spmv_fn get_fp32_spmv(int G, int B);                  // k_fp32.hip
-int fp32_step_blocks(int G, double mean_row);          // B of a matrix
+int fp32_step_blocks(int G, double mean_row, double row_sd);  // B of a matrix
 size_t fp32_spmv_lds(int cols, int G, int B);
 select_groups_fn get_select_groups(int nw);
 size_t select_groups_lds();

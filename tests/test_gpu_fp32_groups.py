@@ -32,3 +32,25 @@ def test_workgroup_groups(acc, gpu, rows, ks, best):
         r, v = O.topk(y, k)
         np.testing.assert_array_equal(got["index"], r)
         np.testing.assert_array_equal(got["value"], np.asarray(v, np.float32))
+
+
+# steps of three or four blocks that become one less: rows of 20, 35 and 60 entries on average, a few of many
+@pytest.mark.parametrize("mean,long", [(20, 0), (20, 100), (35, 0), (35, 300), (60, 0), (60, 280)])
+def test_step_blocks_by_spread(acc, gpu, mean, long):
+    rng = np.random.default_rng(mean + long)
+    lens = rng.integers(mean - 3, mean + 4, 6007)
+    lens = np.where(rng.random(6007) < 0.1, long, lens) if long else lens
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    idx = np.concatenate([np.sort(rng.permutation(310)[:n]) for n in lens]).astype(np.int32)
+    val = rng.standard_normal(len(idx)).astype(np.float32)
+    x = rng.standard_normal(310).astype(np.float32)
+    x[0] = np.inf  # read by slots past a row's end: no row has column 0, so none may sum it
+    keep = idx != 0
+    ptr = np.concatenate([[0], np.cumsum(np.add.reduceat(keep, ptr[:-1]))]).astype(np.int64)
+    idx, val = idx[keep], val[keep]
+    csr = acc.CSRMatrix.from_arrays(6007, 310, ptr, idx, val)
+    g = acc.GpuMatrix(csr)
+    y = acc.DeviceBuffer.from_numpy(np.full(6007, 7, np.float32))
+    g.spmv_fp32(acc.DeviceBuffer.from_numpy(x), y)
+    acc.synchronize()
+    np.testing.assert_array_equal(y.numpy(), O.spmv_f32(ptr, idx, val, x, g.info.group))
