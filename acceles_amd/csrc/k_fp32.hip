@@ -349,7 +349,7 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
     __shared__ uint32_t s_group[1024], s_scan[1024];  // groups that reach T; those to read
     __shared__ uint64_t s_below[1024];                // and the key below which their rows are not listed yet
     uint64_t *s_key = (uint64_t *)smem, *s_top = s_key + kSelList;  // kSelList, then 1024 keys
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const uint32_t nw = (uint32_t)a.nw, RS = (uint32_t)a.RS, rows = (uint32_t)a.rows;
     // all keys are loaded at once; the second and third ones arrive during the
     // radix selection of the best ones
@@ -402,36 +402,42 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
     }
     __syncthreads();
     // fn(key) for every row of groups group(0 .. nl-1) (0: no row).  A
-    // wavefront reads C groups together, U rows per lane and group; the rows'
-    // places in a group are the same for all groups.
+    // wavefront reads U rows per lane of C groups together, and all wavefronts
+    // share a group's rows (20M x 1024: one group of 15,600 rows read by one
+    // wavefront took 36 us, 5 now); the rows' places in a group are the same for
+    // all groups.
     const uint32_t L = (uint32_t)a.gsteps * RS;  // rows of a group
     auto scan_by = [&](auto uu, auto cc, int nl, auto group, auto fn) {
         constexpr int U = decltype(uu)::value, C = decltype(cc)::value;
-        for (uint32_t j0 = 0; j0 < L; j0 += 64 * U) {
-            uint32_t off[U];
+        const uint32_t nc = (uint32_t)(nl + C - 1) / C, items = nc * ((L + 64 * U - 1) / (64 * U));
+        uint32_t off[U], cur = 0xFFFFFFFFu;
+        for (uint32_t it = wave; it < items; it += 16) {
+            const uint32_t jb = it / nc;
+            const int c0 = (int)(it - jb * nc) * C;
+            if (jb != cur) {
+                cur = jb;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t j = j0 + u * 64 + lane, st = j / RS;
-                off[u] = j < L ? st * nw * RS + (j - st * RS) : 0xFFFFFFFFu;
-            }
-            for (int c0 = wave * C; c0 < nl; c0 += 16 * C) {
-                float v[C][U];
-                uint32_t row[C][U];
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const uint32_t b = group(min(c0 + c, nl - 1)) * RS;
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        row[c][u] = c0 + c < nl && off[u] != 0xFFFFFFFFu ? b + off[u] : 0xFFFFFFFFu;
-                        v[c][u] = a.y[min(row[c][u], rows - 1u)];
-                    }
+                for (int u = 0; u < U; ++u) {
+                    const uint32_t j = (jb * U + u) * 64 + lane, st = j / RS;
+                    off[u] = j < L ? st * nw * RS + (j - st * RS) : 0xFFFFFFFFu;
                 }
-#pragma unroll
-                for (int c = 0; c < C; ++c)
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        fn(row[c][u] < rows ? dkey_f32(v[c][u], (int32_t)row[c][u]) : 0ull, min(c0 + c, nl - 1));
             }
+            float v[C][U];
+            uint32_t row[C][U];
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const uint32_t b = group(min(c0 + c, nl - 1)) * RS;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    row[c][u] = c0 + c < nl && off[u] != 0xFFFFFFFFu ? b + off[u] : 0xFFFFFFFFu;
+                    v[c][u] = a.y[min(row[c][u], rows - 1u)];
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    fn(row[c][u] < rows ? dkey_f32(v[c][u], (int32_t)row[c][u]) : 0ull, min(c0 + c, nl - 1));
         }
     };
     auto scan = [&](int nl, auto group, auto fn) {

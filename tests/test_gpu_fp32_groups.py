@@ -54,3 +54,18 @@ def test_step_blocks_by_spread(acc, gpu, mean, long):
     g.spmv_fp32(acc.DeviceBuffer.from_numpy(x), y)
     acc.synchronize()
     np.testing.assert_array_equal(y.numpy(), O.spmv_f32(ptr, idx, val, x, g.info.group))
+
+
+# the best rows in one workgroup's group of several thousand rows, which all wavefronts read together
+@pytest.mark.parametrize("rows,first,count,k", [(2000003, 1000, 300, 100), (2000003, 1999900, 103, 100), (3000001, 77, 5000, 90)])
+def test_long_groups(acc, gpu, rows, first, count, k):
+    rng = np.random.default_rng(rows + first)
+    ptr = np.arange(rows + 1, dtype=np.int64)
+    idx = rng.integers(0, 8, rows).astype(np.int32)
+    val = rng.random(rows).astype(np.float32)
+    val[first:first + count] += 10
+    x = np.ones(8, np.float32)
+    got = acc.GpuMatrix(acc.CSRMatrix.from_arrays(rows, 8, ptr, idx, val)).topk_fp32_host(x, k)
+    order = np.lexsort((np.arange(rows), -val))[:k]
+    np.testing.assert_array_equal(got["index"], order)
+    np.testing.assert_array_equal(got["value"], val[order])
