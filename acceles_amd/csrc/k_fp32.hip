@@ -323,12 +323,18 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
 // each group's rows (one workgroup): T, at most the K-th largest of
 // the groups' best keys, is reached by K distinct rows, so every row of the
 // Top-K has a key >= T and lies in one of the groups whose best reaches it (at
-// most K + kSelSlack).  Their best keys, and their second ones that reach T, are
-// listed in LDS; only a group whose third key reaches T can hold more such rows
-// and is read from y (the steps are dealt in turn, so neighbouring rows lie in
-// different groups and hardly any is read).  The listed keys are ranked.  A list
-// that does not fit (an order of rows that puts most of the best ones into the
-// same groups) is cut by a radix selection over the rows of those groups.
+// most K + kSelSlack).  Their keys that reach T are listed in LDS; only a group
+// whose third key exceeds T can hold more such rows and is read from y (the
+// steps are dealt in turn, so neighbouring rows lie in different groups and
+// hardly any is read).  Where the third key has T's score, all that is left of the
+// group are rows of that score, and none after T's row: only its steps up to there
+// are read (equal scores: every group's).  The listed keys are ranked.
+//
+// An order of rows that puts most of the best ones into the same groups
+// leaves T too low.  Before many rows are read, and whenever more rows reach T
+// than the list holds, T rises to the K-th best key listed and the listing
+// starts again; after kSelRounds such rounds (scores that rise in the order of
+// reading) a radix selection over the rows of those groups ends it.
 //
 // Bound: latency, and what one CU reads: at 2,000,000 rows and K = 100 it
 // takes 9 us (at 100,000 rows 6), from wavefronts' instead of workgroups' keys
@@ -337,17 +343,26 @@ __global__ __launch_bounds__(ACC_WG) void fp32_spmv(const uint32_t *ptr, const c
 // Before it, two radix passes over all scores and a final one took 32 us, and
 // above K = 256 the sorted lists of select_blocks and select_final 827 us
 // (4,999,999 rows, K = 500; 16 us here).
+// Equal scores (a query of zeros), us of the whole call, K = 100: 100,000 x 500
+// 29, 2,000,000 x 900 154, 4,999,999 x 1024 191 -- any other query takes 17, 140
+// and 179 --, before T rose and the reading ended at its row 38, 560 and 1205.
 static constexpr int kSelList = 4096;  // keys listed in LDS
 static constexpr int kSelSlack = 16;   // groups listed past the K-th, for one or two radix digits less
+static constexpr int kSelRounds = 3;   // listings that overflowed
+// Rows read before T rises: one round of loads of the workgroup, less than the
+// rise takes.  Rows of a group whose three best keys are of one score and one
+// step nearly all reach T and count more: they would have to be cut afterwards.
+static constexpr uint32_t kSelRead = 16384, kSelDense = 16;
 
 template <int V>
 __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ uint32_t hist[512];
     __shared__ uint64_t s_t[2];
-    __shared__ int s_need[2], s_n, s_m, s_scans;
-    __shared__ uint32_t s_group[1024], s_scan[1024];  // groups that reach T; those to read
-    __shared__ uint64_t s_below[1024];                // and the key below which their rows are not listed yet
+    __shared__ int s_need[2], s_n, s_scans;
+    __shared__ uint32_t s_rows;                      // rows to read, weighted
+    __shared__ uint32_t s_scan[1024], s_last[1024];  // groups to read, up to this row
+    __shared__ uint64_t s_below[1024];               // and the key below which their rows are not listed yet
     uint64_t *s_key = (uint64_t *)smem, *s_top = s_key + kSelList;  // kSelList, then 1024 keys
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const uint32_t nw = (uint32_t)a.nw, RS = (uint32_t)a.RS, rows = (uint32_t)a.rows;
@@ -364,10 +379,10 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
         if ((uint32_t)(tid + u * 1024) >= nw) k[u] = 0ull;
     if (tid == 0) {
         s_n = 0;
-        s_m = 0;
         s_scans = 0;
+        s_rows = 0u;
     }
-    const uint64_t T = wg_radix_kth<uint64_t>(
+    uint64_t T = wg_radix_kth<uint64_t>(
         [&](auto fn) {
 #pragma unroll
             for (int u = 0; u < V; ++u) fn(k[u]);
@@ -382,35 +397,35 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
         const int j = atomicAdd(&s_n, 1);
         if (j < kSelList) s_key[j] = key;
     };
-    if (!all) {
-#pragma unroll
-        for (int u = 0; u < V; ++u)
-            if (k[u] >= T) {
-                append(k[u]);
-                const uint32_t w = (uint32_t)(tid + u * 1024);
-                const int j = atomicAdd(&s_m, 1);
-                if (j < 1024) s_group[j] = w;  // K + kSelSlack of them at most: the keys are distinct
-                if (k23[u].x >= T) append(k23[u].x);
-                if (k23[u].y >= T) {
-                    const int i = atomicAdd(&s_scans, 1);
-                    if (i < 1024) {
-                        s_scan[i] = w;
-                        s_below[i] = k23[u].x;
-                    }
-                }
-            }
-    }
-    __syncthreads();
-    // fn(key) for every row of groups group(0 .. nl-1) (0: no row).  A
-    // wavefront reads U rows per lane of C groups together, and all wavefronts
-    // share a group's rows (20M x 1024: one group of 15,600 rows read by one
-    // wavefront took 36 us, 5 now); the rows' places in a group are the same for
-    // all groups.
     const uint32_t L = (uint32_t)a.gsteps * RS;  // rows of a group
-    auto scan_by = [&](auto uu, auto cc, int nl, auto group, auto fn) {
+    // group w's keys that reach T (at most 3 * (K + kSelSlack) of all groups, which fit); a group to read
+    auto list = [&](uint32_t w, uint64_t k1, uint64_t k2, uint64_t k3) {
+        if (k1 < T) return;
+        append(k1);
+        if (k2 >= T) append(k2);
+        if (k3 >= T) append(k3);
+        if (k3 > T) {
+            const int i = atomicAdd(&s_scans, 1);
+            if (i < 1024) {  // K + kSelSlack of them at most: the keys are distinct
+                s_scan[i] = w;
+                s_below[i] = k3;
+                // (T may be the lower end of a digit: its row then lies past the matrix)
+                const uint32_t end = min((uint32_t)dkey_row(T), rows - 1u);
+                const bool ties = (k3 >> 32) == (T >> 32);
+                s_last[i] = ties ? end : rows - 1u;
+                atomicAdd(&s_rows, !ties ? L : (end / (nw * RS) + 1u) * RS * (k1 - k3 < RS ? kSelDense : 1u));
+            }
+        }
+    };
+    // fn(key, i) for the rows of groups group(i), i = 0 .. nl-1, up to row
+    // last(i) (0: no row).  A wavefront reads U rows per lane of C groups
+    // together, and all wavefronts share a group's rows (20M x 1024: one group of
+    // 15,600 rows read by one wavefront took 36 us, 5 now); the rows' places in a
+    // group are the same for all groups.
+    auto scan_by = [&](auto uu, auto cc, int nl, auto group, auto last, auto fn) {
         constexpr int U = decltype(uu)::value, C = decltype(cc)::value;
         const uint32_t nc = (uint32_t)(nl + C - 1) / C, items = nc * ((L + 64 * U - 1) / (64 * U));
-        uint32_t off[U], cur = 0xFFFFFFFFu;
+        uint32_t off[U], off0 = 0u, cur = 0xFFFFFFFFu;
         for (uint32_t it = wave; it < items; it += 16) {
             const uint32_t jb = it / nc;
             const int c0 = (int)(it - jb * nc) * C;
@@ -421,18 +436,27 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
                     const uint32_t j = (jb * U + u) * 64 + lane, st = j / RS;
                     off[u] = j < L ? st * nw * RS + (j - st * RS) : 0xFFFFFFFFu;
                 }
+                off0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)off[0]);  // the first row's
             }
+            uint32_t b[C], e[C];  // the groups' first rows, and one past the last to read
+            bool any = false;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int i = min(c0 + c, nl - 1);
+                b[c] = group(i) * RS;
+                e[c] = c0 + c < nl ? last(i) + 1u : 0u;
+                any |= b[c] + off0 < e[c];
+            }
+            if (!any) continue;  // the same for the whole wavefront
             float v[C][U];
             uint32_t row[C][U];
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const uint32_t b = group(min(c0 + c, nl - 1)) * RS;
+            for (int c = 0; c < C; ++c)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    row[c][u] = c0 + c < nl && off[u] != 0xFFFFFFFFu ? b + off[u] : 0xFFFFFFFFu;
+                    row[c][u] = off[u] != 0xFFFFFFFFu && b[c] + off[u] < e[c] ? b[c] + off[u] : 0xFFFFFFFFu;
                     v[c][u] = a.y[min(row[c][u], rows - 1u)];
                 }
-            }
 #pragma unroll
             for (int c = 0; c < C; ++c)
 #pragma unroll
@@ -440,28 +464,66 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
                     fn(row[c][u] < rows ? dkey_f32(v[c][u], (int32_t)row[c][u]) : 0ull, min(c0 + c, nl - 1));
         }
     };
-    auto scan = [&](int nl, auto group, auto fn) {
-        if (L <= 64) scan_by(std::integral_constant<int, 1>(), std::integral_constant<int, 8>(), nl, group, fn);
-        else scan_by(std::integral_constant<int, 8>(), std::integral_constant<int, 2>(), nl, group, fn);
+    auto scan = [&](int nl, auto fn) {  // of the groups to read
+        auto group = [&](int i) { return s_scan[i]; };
+        auto last = [&](int i) { return s_last[i]; };
+        if (L <= 64) scan_by(std::integral_constant<int, 1>(), std::integral_constant<int, 8>(), nl, group, last, fn);
+        else scan_by(std::integral_constant<int, 8>(), std::integral_constant<int, 2>(), nl, group, last, fn);
     };
-    if (!all)
-        scan(
-            min(s_scans, 1024), [&](int i) { return s_scan[i]; },
-            [&](uint64_t key, int i) {
+    if (!all) {
+#pragma unroll
+        for (int u = 0; u < V; ++u) list((uint32_t)(tid + u * 1024), k[u], k23[u].x, k23[u].y);
+    }
+    int nl = 0;  // keys listed before any row was read
+    for (int over = -1; !all;) {  // -1: nothing read yet
+        __syncthreads();
+        nl = s_n;
+        const int scans = min(s_scans, 1024);
+        if (over >= 0 || s_rows <= kSelRead) {
+            scan(scans, [&](uint64_t key, int i) {
                 if (key >= T && key < s_below[i]) append(key);
             });
-    __syncthreads();
-    if (all || s_n > kSelList) {
-        // all rows of the groups that reach T (of every group): their K best
-        const int nl = all ? (int)nw : min(s_m, 1024);
-        auto group = [&](int i) { return all ? (uint32_t)i : s_group[i]; };
+            __syncthreads();
+            if (s_n <= kSelList || over == kSelRounds) break;
+        }
+        ++over;
+        const int have = min(s_n, kSelList);
+        T = wg_radix_kth<uint64_t>(
+            [&](auto fn) {
+                for (int i = tid; i < have; i += 1024) fn(s_key[i]);
+            },
+            a.K, hist, s_t, s_need);
+        if (tid == 0) {
+            s_n = 0;
+            s_scans = 0;
+            s_rows = 0u;
+        }
         __syncthreads();
+        for (uint32_t w = tid; w < nw; w += 1024) {
+            const ulonglong2 k2 = ((const ulonglong2 *)(a.gmax + group_pairs(a.nw)))[w];
+            list(w, a.gmax[w], k2.x, k2.y);
+        }
+    }
+    if (all || s_n > kSelList) {
+        // the K best of the listed keys and the rows of the groups to read (of every group)
+        auto each = [&](auto fn) {
+            for (int i = tid; i < nl; i += 1024) fn(s_key[i]);
+            scan_by(
+                std::integral_constant<int, 4>(), std::integral_constant<int, 1>(), all ? (int)nw : min(s_scans, 1024),
+                [&](int i) { return all ? (uint32_t)i : s_scan[i]; }, [&](int i) { return all ? rows - 1u : s_last[i]; },
+                [&](uint64_t key, int i) { fn(all || (key >= T && key < s_below[i]) ? key : 0ull); });
+        };
+        const uint64_t cut = wg_radix_kth<uint64_t>(each, a.K, hist, s_t, s_need);
         if (tid == 0) s_n = 0;
-        const uint64_t cut = wg_radix_kth<uint64_t>(
-            [&](auto fn) { scan(nl, group, [&](uint64_t key, int) { fn(key); }); }, a.K, hist, s_t, s_need);
-        scan(nl, group, [&](uint64_t key, int) {
-            if (key != 0ull && key >= cut) append(key);
+        __syncthreads();
+        each([&](uint64_t key) {
+            if (key != 0ull && key >= cut) {
+                const int j = atomicAdd(&s_n, 1);
+                if (j < 1024) s_top[j] = key;  // K of them at most: the keys are distinct
+            }
         });
+        __syncthreads();
+        if (tid < min(s_n, 1024)) s_key[tid] = s_top[tid];
         __syncthreads();
     }
     int n = min(s_n, kSelList);
