@@ -58,6 +58,44 @@ __device__ __forceinline__ int32_t slice_dot_packets(const DenseArgs &a, int64_t
     return acc;
 }
 
+// The same for one slot (slice * 64 + row in it) per lane, in any slices: 64
+// scattered rows in about the time of one slice.
+__device__ __forceinline__ int32_t slot_dot_packets(const DenseArgs &a, int64_t slot, const int8_t *qx) {
+    const uint2 sl = a.slices[slot >> 6];
+    const int cb = a.col_bits, vb = a.val_bits, E = cb + vb;
+    const uint64_t emask = (1ull << E) - 1ull;
+    const uint32_t cmask = (1u << cb) - 1u;
+    const uint32_t *p = a.words + (size_t)sl.x * 64 + (uint32_t)(slot & 63);
+    const int nd = (int)sl.y, end = (int)wave_umax(sl.y);
+    uint32_t w[2][8];  // eight dwords are decoded while the next eight are loaded (words are padded past the last slice)
+    auto load = [&](uint32_t (&v)[8], int d0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(d0 + u, max(nd - 1, 0)) * 64];
+    };
+    uint64_t buf = 0ull;
+    int nb = 0;
+    int32_t acc = 0;
+    load(w[0], 0);
+    for (int d0 = 0; d0 < end; d0 += 8) {
+        load(w[1], d0 + 8);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            buf |= (uint64_t)(d0 + u < nd ? w[0][u] : 0u) << nb;
+            nb += 32;
+            while (nb >= E) {
+                const uint32_t e = (uint32_t)(buf & emask);
+                buf >>= E;
+                nb -= E;
+                const int v = a.is_signed ? __builtin_amdgcn_sbfe(e, cb, vb) : (int)__builtin_amdgcn_ubfe(e, cb, vb);
+                acc += v * (int)qx[e & cmask];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) w[0][u] = w[1][u];
+    }
+    return acc;
+}
+
 // One workgroup per query slot of the padded batch: int8 quantization with
 // the query's own scale (quantify_util.py:31-49, 259; the rule of the packet
 // kernels), written in the B-operand layout, in plain order (rescans) and as
@@ -274,6 +312,122 @@ __device__ __forceinline__ void rescore_rows(const DenseArgs &a, const uint64_t 
     }
 }
 
+// Candidates of one (query, partition) where more than 64 rows, or those of many
+// slices besides the listed ones, may qualify (equal scores): k is left with the
+// best of them (lane i < n: the i-th, or in no order as long as 64 hold them
+// all), n returned.  nl: the number listed (keys of tk or above), in k up to 64;
+// ts: the score that another row must reach; again: the slices whose fourth key
+// does, a bit each; cand: 64 keys, then room for 704 slots; qx: the quantized
+// query (LDS); zero: it is all zeros (padding of a batch), and so are the scores.
+// A row of a slice scores its fourth key's score at most, so with the M-th best
+// key found so far only rows that this score would put above it are scored: of
+// equal scores the lower rows.  64 of them at a time, of any slices.
+__device__ __forceinline__ int select_with_rescans(const DenseArgs &a, int q, int64_t s0, int nsl, int nvl, int nl,
+                                                   uint32_t tk, int32_t ts, uint64_t *cand, const uint64_t *again,
+                                                   const int8_t *qx, bool zero, uint64_t &k) {
+    const int lane = lane_id(), M = a.M;
+    const uint4 *L = (const uint4 *)a.tk + (size_t)q * a.nslices + s0;
+    const int32_t *perm = a.perm + s0 * 64;
+    uint16_t *slots = (uint16_t *)(cand + 64);  // slot in the partition (at most 1,024 slices)
+    constexpr int B = 8;                        // slices looked at together
+    // least: the M-th best so far; the pend keys above it wait in cand
+    uint64_t least = 0ull, mask = 0ull, key[4];
+    int pend = 0, nslots = 0, b = 0, e = 0, w = 0;
+    if (nl <= 64) {
+        if (lane < nl) cand[lane] = k;
+        pend = nl;
+        b = nsl;
+        if (nl >= M) {
+            int rank = 0;
+            for (int j = 0; j < nl; ++j) rank += readlane_u64(k, j) > k;
+            least = readlane_u64(k, __builtin_ctzll(__ballot(lane < nl && rank == M - 1)));
+        }
+    }
+    bool sorted = false;
+    k = 0ull;
+    for (;;) {
+        uint64_t nk = 0ull;
+        bool last = false;
+        if (b < nsl) {  // the listed keys of 64 slices, one of each at a time
+            if (e == 0) {
+                const int i = b + lane, nv = i >= nsl ? 0 : i == nsl - 1 ? nvl : 64;
+                const uint4 l = L[min(i, nsl - 1)];
+                const uint32_t ke[4] = {l.x, l.y, l.z, l.w};
+                int32_t r[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) r[j] = perm[(size_t)min(i, nsl - 1) * 64 + tk_rho(ke[j])];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    key[j] = tk_rho(ke[j]) < nv && ke[j] >= tk ? dkey_i32(tk_score(ke[j]), r[j]) : 0ull;
+            }
+            nk = e == 0 ? key[0] : e == 1 ? key[1] : e == 2 ? key[2] : key[3];
+            e = (e + 1) & 3;
+            b += e == 0 ? 64 : 0;
+        } else {
+            // B slices at a time: their rows that may qualify
+            while (nslots < 64 && (mask != 0ull || w * 64 < nsl)) {
+                if (mask == 0ull) {
+                    mask = readlane_u64(again[w], 0);
+                    ++w;
+                    continue;
+                }
+                int sl[B];
+                int32_t row[B];
+                uint4 l[B];
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    sl[j] = mask ? (w - 1) * 64 + __builtin_ctzll(mask) : -1;
+                    mask &= mask - 1;
+                }
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    row[j] = perm[(size_t)max(sl[j], 0) * 64 + lane];
+                    l[j] = L[max(sl[j], 0)];
+                }
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    const bool has = lane == tk_rho(l[j].x) || lane == tk_rho(l[j].y) || lane == tk_rho(l[j].z) ||
+                                     lane == tk_rho(l[j].w);
+                    const bool ok = sl[j] >= 0 && row[j] >= 0 && !has && dkey_i32(tk_score(l[j].w), row[j]) > least;
+                    const uint64_t m = __ballot(ok);
+                    if (ok) slots[nslots + mbcnt64(m)] = (uint16_t)(sl[j] * 64 + lane);
+                    nslots += __popcll(m);
+                }
+            }
+            wave_sync();
+            const int ns = min(nslots, 64);
+            last = ns == 0;
+            if (!last) {  // score the last 64 of them
+                const uint32_t slot = slots[nslots - ns + min(lane, ns - 1)];
+                const int32_t row = perm[slot];
+                const int32_t sc = zero ? 0 : slot_dot_packets(a, s0 * 64 + slot, qx);
+                if (lane < ns && sc >= ts) nk = dkey_i32(sc, row);
+                nslots -= ns;
+            }
+        }
+        uint64_t m = __ballot(nk > least);
+        if (last && !sorted) {
+            wave_sync();
+            k = lane < pend ? cand[lane] : 0ull;
+            return pend;
+        }
+        if (last || pend + __popcll(m) > 64) {
+            wave_sync();
+            uint64_t v[2] = {k, lane < pend ? cand[lane] : 0ull};
+            reg_sort_desc<2>(v);
+            k = v[0];
+            sorted = true;
+            if (last) return min(__popcll(__ballot(k != 0ull)), M);
+            least = shfl_u64(k, M - 1);
+            pend = 0;
+            m = __ballot(nk > least);
+            wave_sync();
+        }
+        if (nk > least) cand[pend + mbcnt64(m)] = nk;
+        pend += __popcll(m);
+    }
+}
+
 // One wavefront per (partition p = blockIdx.x, query q = blockIdx.y*4 + wave),
 // for partitions of at most 64*U slices and M <= 32:
 //  1. ts = a score that M distinct rows of the partition reach (INT32_MIN when
@@ -281,17 +435,18 @@ __device__ __forceinline__ void rescore_rows(const DenseArgs &a, const uint64_t 
 //     of the full slices' maxima reach it (up to 64 slices: M of their listed
 //     scores).  The partition's M-th best score is >= ts, so no row below ts
 //     can be in its Top-M.
-//  2. Every listed key of a real row scoring >= ts is a candidate.  A list
-//     whose fourth key still scores >= ts may have dropped a qualifying row:
-//     that slice is rescanned exactly (all 64 rows, one dot4 pass) instead.
-//     Maxima of the partial slice (padding rows score 0) are left out of step
-//     1, and its padding rows' keys, which may have displaced real rows from
-//     its list, of step 2.
-//  3. Top-M of the candidates by (score, row) (quantify_util.py:173-196 with
-//     the lower-row tie rule), then their FP32 rescoring (out != null).
-// One prefix sum appends the candidates' slots, one gather finds their rows, a
-// count ranks them.  More than 64 candidates (heavy ties): every slice that
-// reaches ts is rescanned and merged into a sorted list of one key per lane.
+//  2. Every listed key of a real row scoring >= ts is a candidate; one prefix
+//     sum places them, one gather finds their rows.  (Padding rows of the
+//     partial slice score 0: its maximum is left out of step 1, their keys,
+//     which may have displaced real rows from its list, of this step.)
+//  3. A list whose fourth key still scores >= ts may have dropped a qualifying
+//     row, none of a score above that key's.  The other rows of its slice are
+//     scored exactly, unless M candidates score above that key (400,000 x 500,
+//     100 queries: 64 -> 61 us of a call).
+//  4. Top-M of the candidates by (score, row) (quantify_util.py:173-196 with
+//     the lower-row tie rule), ranked by counting, then their FP32 rescoring
+//     (out != null).  More than 64 candidates, or kRescans slices: select_with_
+//     rescans.
 //
 // Bound: the memory requests of the rescoring (rows of a few cache lines each,
 // anywhere in the CSR), about 0.4 ns per row.  400,000 x 500, 100 queries:
@@ -301,15 +456,17 @@ __device__ __forceinline__ void rescore_rows(const DenseArgs &a, const uint64_t 
 // us (26.2); 2,000,000 x 900, 256 queries: 65 (111).
 template <int U>
 __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
-    constexpr int kSlack = 8, kRescans = 128;
+    constexpr int kSlack = 8, kRescans = 8;  // slices rescanned one after the other
     extern __shared__ __align__(16) unsigned char smem[];
-    const int wave = threadIdx.x >> 6, lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
     const int p = blockIdx.x, q = blockIdx.y * ACC_WAVES + wave;
     if (q >= a.nq) return;  // whole wavefront; no workgroup barrier below
-    // per wavefront: 64 ranked keys and their entry ranges, 64 candidates, the slices to rescan
-    uint64_t *keys = (uint64_t *)smem + wave * 256, *cand = keys + 128;
+    // per wavefront (2 KB): 64 candidates; 64 ranked keys and their entry
+    // ranges, before that the slots to score (at most 575 of 704); the slices
+    // to rescan, a bit each
+    uint64_t *cand = (uint64_t *)smem + wave * 256, *keys = cand + 64;
     uint2 *ranges = (uint2 *)(keys + 64);
-    uint32_t *rl = (uint32_t *)(keys + 192);
+    uint64_t *again = cand + 240;
     int8_t *qx = (int8_t *)(smem + ACC_WAVES * 256 * 8) + (size_t)wave * a.cols_pad;
     float *xs = (float *)(smem + ACC_WAVES * 256 * 8 + (size_t)ACC_WAVES * a.cols_pad) + (size_t)wave * a.cols_pad;
     const int64_t s0 = a.part_slice[p];
@@ -350,90 +507,90 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
             }
         }
         // tk: the smallest list key of a score that reaches the bound (keys of
-        // one score differ in the row)
-        const uint32_t tk = t & ~63u;
-        const int32_t ts = t != 0u ? tk_score(t) : INT32_MIN;
-        auto again = [&](int u) { return u * 64 + lane < nsl && k4[u].w >= tk; };       // to rescan
-        auto rows_of = [&](int u) {                                                   // real rows of a list to take
-            const int i = u * 64 + lane;
-            return again(u) || i >= nsl ? 0 : i == nsl - 1 ? nvl : 64;
-        };
-        int c = 0;
+        // one score differ in the row); without a bound that of any row
+        const uint32_t tk = max(t & ~63u, 64u);
+        int c = 0, nr = 0;  // listed candidates of this lane, slices to rescan
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int nv = rows_of(u);
+            const int nv = u * 64 + lane == nsl - 1 ? nvl : 64;
             const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
 #pragma unroll
             for (int e = 0; e < 4; ++e) c += tk_rho(ke[e]) < nv && ke[e] >= tk ? 1 : 0;
+            const uint64_t m = __ballot(k4[u].w >= tk);
+            const int j = nr + mbcnt64(m);
+            if (k4[u].w >= tk && j < kRescans)
+                keys[j] = ((uint64_t)k4[u].w << 32) |
+                          (uint32_t)((u * 64 + lane) << 18 | tk_rho(k4[u].z) << 12 | tk_rho(k4[u].y) << 6 | tk_rho(k4[u].x));
+            nr += __popcll(m);
         }
         const int incl = (int)wave_prefix_sum((uint32_t)c);
-        const int nl = __builtin_amdgcn_readlane(incl, 63);  // listed candidates
-        int n = nl, nr = 0;
-        uint64_t k = 0ull;
+        const int nl = __builtin_amdgcn_readlane(incl, 63);
+        uint64_t k = 0ull;  // lane i < n: a candidate
+        uint32_t listed = 0u;
+        int n = 0;
         if (nl <= 64) {
             int pos = incl - c;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int nv = rows_of(u);
+                const int nv = u * 64 + lane == nsl - 1 ? nvl : 64;
                 const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (tk_rho(ke[e]) < nv && ke[e] >= tk)
                         cand[pos++] = ((uint64_t)ke[e] << 32) | (uint32_t)((u * 64 + lane) * 64 + tk_rho(ke[e]));
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {  // slices to rescan, listed so that one loop serves them all
-                const bool r = again(u);
-                const uint64_t m = __ballot(r);
-                const int j = nr + mbcnt64(m);
-                if (r && j < kRescans) rl[j] = (uint32_t)(u * 64 + lane);
-                nr += __popcll(m);
-            }
             wave_sync();
-            if (lane < nl) {
+            n = nl;
+            if (lane < n) {
                 const uint64_t e = cand[lane];
-                k = dkey_i32(tk_score((uint32_t)(e >> 32)), perm[(uint32_t)e]);
+                listed = (uint32_t)(e >> 32);
+                k = dkey_i32(tk_score(listed), perm[(uint32_t)e]);
             }
         }
-        const bool many = nl > 64 || nr > kRescans;
-        if (nr > 0 || many) {
-            const int8_t *src = a.qplain + (size_t)q * a.cols_pad;
-            for (int cc = lane; cc < a.cols_pad; cc += 64) qx[cc] = src[cc];
+        const int32_t ts = t != 0u ? tk_score(t) : INT32_MIN;
+        bool many = nl > 64 || nr > kRescans, zero = true;
+        if (nr > 0) {
+            // at most 1,024 columns, padded to whole dwords: one round trip
+            const uint32_t *src = (const uint32_t *)(a.qplain + (size_t)q * a.cols_pad);
+            const int nd = a.cols_pad / 4;
+            uint32_t v[4], any = 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = src[min(j * 64 + lane, nd - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (j * 64 + lane < nd) ((uint32_t *)qx)[j * 64 + lane] = v[j];
+                any |= v[j];
+            }
+            zero = !__any(any != 0u);
             wave_sync();
         }
-        if (!many) {
-            for (int j = 0; j < nr && n <= 64; ++j) {
-                const int64_t s = s0 + __builtin_amdgcn_readfirstlane((int)rl[j]);
-                const int32_t sc = slice_dot_packets(a, s, qx);
-                const int32_t r = a.perm[s * 64 + lane];
-                const bool pr = r >= 0 && sc >= ts;
-                const uint64_t bm = __ballot(pr);
-                if (n + __popcll(bm) <= 64 && pr) cand[n + mbcnt64(bm)] = dkey_i32(sc, r);
-                n += __popcll(bm);
+        for (int j = 0; j < nr && !many; ++j) {  // slice by slice
+            const uint64_t e = readlane_u64(keys[j], 0);
+            const uint32_t lw = (uint32_t)(e >> 32), at = (uint32_t)e;
+            // M listed candidates above its fourth key's score: no other row of it qualifies
+            if (__popcll(__ballot(listed > (lw | 63u))) >= M) continue;
+            const int s = (int)(at >> 18);
+            const int32_t r = perm[(size_t)s * 64 + lane];
+            const int32_t sc = slice_dot_packets(a, s0 + s, qx);
+            const bool in_list = lane == (int)(at & 63u) || lane == (int)(at >> 6 & 63u) || lane == (int)(at >> 12 & 63u) ||
+                                 lane == tk_rho(lw);
+            const bool ok = r >= 0 && sc >= ts && !in_list;
+            const uint64_t m = __ballot(ok);
+            many = n + __popcll(m) > 64;
+            if (ok && !many) cand[n + mbcnt64(m)] = dkey_i32(sc, r);
+            n += many ? 0 : __popcll(m);
+        }
+        if (many) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint64_t m = __ballot(k4[u].w >= tk);
+                if (lane == 0) again[u] = m;
             }
             wave_sync();
-            if (n <= 64 && lane >= nl && lane < n) k = cand[lane];
-        }
-        int rank = lane;
-        if (many || n > 64) {
-            // lane i: the i-th best key so far
-            k = 0ull;
-            for (int b = 0; b < nsl; b += 64) {
-                const int i = b + lane;
-                uint64_t mask = __ballot(i < nsl && L[min(i, nsl - 1)].x >= tk);
-                while (mask) {
-                    const int64_t s = s0 + b + __builtin_ctzll(mask);
-                    mask &= mask - 1;
-                    const int32_t sc = slice_dot_packets(a, s, qx);
-                    const int32_t r = a.perm[s * 64 + lane];
-                    const uint64_t nk = r >= 0 ? dkey_i32(sc, r) : 0ull, least = shfl_u64(k, M - 1);
-                    if (!__any(nk > least)) continue;
-                    uint64_t w[2] = {k, nk};
-                    reg_sort_desc<2>(w);
-                    k = w[0];
-                }
-            }
-            n = __popcll(__ballot(k != 0ull));
+            n = select_with_rescans(a, q, s0, nsl, nvl, nl, tk, ts, cand, again, qx, zero, k);
+        } else if (nr > 0) {
+            wave_sync();
+            if (lane >= nl && lane < n) k = cand[lane];
         }
         // the candidates' CSR entry ranges, in flight while the ranks are
         // counted (out set: the CSR is present)
@@ -442,7 +599,7 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
             const int32_t r = lane < n ? dkey_row(k) : 0;
             rg = make_uint2(a.ptr[r], a.ptr[r + 1]);
         }
-        rank = 0;
+        int rank = 0;
         for (int j = 0; j < n; ++j) rank += readlane_u64(k, j) > k;  // distinct: one per row
         nn = min(n, M);
         if (lane < n && rank < nn) {
