@@ -412,41 +412,63 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
     return a;
 }
 
-// Estimated time of a batch per layout, in us.  Measured (CK 512, K 100; batch
-// of 8, us single / packets / matrix cores): 20,000 x 500 175 / 70 / 43, 400,000
-// x 500 218 / 103 / 45, 1,000,000 x 250 4-bit 215 / 118 / 71, 2,000,000 x 900
-// 458 / 230 / 163, 5,000,000 x 1024 (20 entries per row) 468 / 296 / 402; one
-// query: 25 / 65 / 41, 31 / 98 / 47, 28 / 110 / 70, 60 / 215 / 164, 65 / 276
-// / 395.  So: a single query pays about 21 us and its packets at 7 TB/s; the
-// packet batch 55 us and 1.5 ns per 1,000 entries and 0.6 ns per slice for
-// every block of 16 or 32 queries; the matrix cores 33 us and per slice 2.4
-// ns up to 16 column blocks, 5.5 above (a 128-query block), 4.6 up to 64 queries
-// (two wavefronts per query tile: 8 queries at 2M x 900: 198 -> 163 us).
+// Estimated time of a batch per layout, in us, for M rows kept per partition.
+// Fitted to 248 measurements (3,000 to 5,000,000 rows of 3 to 300 entries, 1 to
+// 256 queries, M = 1 to 64, partitions of 2 to 7,800 slices); us single /
+// packets / matrix cores at 8 queries, CK 512 unless given:
+//   20,000 x 500 172 / 66 / 38, CK 1024 in 16 partitions 269 / 84 / 147
+//   3,000 x 120, CK 256 in 16 partitions 175 / 30 / 38
+//   400,000 x 500 209 / 98 / 42, 1,000,000 x 250 4-bit 199 / 114 / 52
+//   2,000,000 x 64, 3.5 entries per row 189 / 127 / 75
+//   2,000,000 x 900 454 / 227 / 161, 5,000,000 x 1024 459 / 294 / 400
+//   300,000 x 1024, 300 entries per row 443 / 205 / 96
+// A single query pays its launches and its packets at 7 TB/s.  The packet batch
+// pays its selection and the rescoring of its rows, per block of 16 or 32
+// queries its entries and slices, and per query the scores that it writes.  The
+// matrix cores pay per slice the decode (0.8 ns per entry) or the
+// multiplications, whichever takes longer, and the slices they expect to rescan:
+// those with four of their partition's best M rows (Poisson; the slowest
+// wavefront bounds the launch), or every row where the lists hold fewer than M.
 struct BatchCost {
     double single, sparse, dense;
 };
-BatchCost batch_cost(const acc_gpu_matrix *m, int nq) {
+BatchCost batch_cost(const acc_gpu_matrix *m, int nq, int M) {
+    const double slices = (double)m->nslices, part = std::max(1.0, slices / m->split);
+    const double mean = m->rows > 0 ? (double)m->nnz / m->rows : 0.0, cand = (double)m->split * M;
     BatchCost c;
-    c.single = nq * (21.0 + (double)m->stream_bytes / 7e6);
+    c.single = nq * (16.3 + 0.147 * M + (double)m->stream_bytes / 7e6);
     const int qb = nq <= 16 ? 16 : 32;
-    c.sparse = 55.0 + (1.5e-6 * (double)m->nnz + 0.6e-3 * (double)m->nslices) * (qb / 16) * ((nq + qb - 1) / qb);
-    c.dense = 33.0 + (m->nkb <= 16 ? 2.4e-3 : nq <= 64 ? 4.6e-3 : 5.5e-3) * (double)m->nslices * ((nq + 127) / 128);
+    c.sparse = 14.0 + 0.2 * mean + 0.04 * std::min(cand, 512.0) + 0.3 * M + 0.024 * part +
+               (1.5e-6 * (double)m->nnz + 0.47e-3 * slices) * (qb / 16) * ((nq + qb - 1) / qb) +
+               0.05e-3 * nq * slices + 0.3e-3 * nq * cand;
+    const int tiles = (nq + 31) / 32, per = tiles > 4 ? 8 : 4;
+    const double load = tiles <= 2 ? 1.0 : tiles <= 4 ? 1.5 : 2.4;  // of a slice, by the tiles multiplied
+    c.dense = 20.0 + 0.23e-3 * nq * cand +
+              load * ((tiles + per - 1) / per) * std::max(0.8e-6 * (double)m->nnz, (m->nkb > 16 ? 4.8e-3 : 1.7e-3) * slices);
+    const double l = M / part, full = part * (1.0 - std::exp(-l) * (1.0 + l + l * l / 2.0 + l * l * l / 6.0));
+    const double rescans = std::min(part, full + 1.5 * std::sqrt(full));
+    if (M > 32 || m->max_part_slices > 1024) c.dense += 22.0 + 0.012 * part + 8.0 * rescans;  // the collector (k_dense.hip)
+    else c.dense += 4 * (int64_t)(m->rows / m->split / 64) < M ? 14.0 : (1.0 + 0.05 * mean) * rescans;
     return c;
 }
 
-// Layout of a batch of nq queries: ACC_BATCH_SINGLE, _SPARSE or _DENSE.  All
-// give the same results; untuned, the one of the lowest estimate, except that
-// a crossover the caller has set decides where the matrix cores are used.
-int batch_layout(const acc_gpu_matrix *m, int nq) {
+// Layout of a batch of nq queries that keeps M rows per partition: ACC_BATCH_
+// SINGLE, _SPARSE or _DENSE.  All give the same results; untuned, the one of the
+// lowest estimate (the matrix cores from 16 queries on unless another one is a
+// tenth lower: from there they win nearly everywhere, by factors, and the estimates
+// are off by up to a half), except that a crossover the caller has set decides
+// where the matrix cores are used.
+int batch_layout(const acc_gpu_matrix *m, int nq, int M) {
     if (m->batch_mode != ACC_BATCH_AUTO) return m->batch_mode;
     if (m->ntune > 0) {
-        int pick = m->tune_layout[0];
-        for (int i = 0; i < m->ntune; ++i)
+        int pick = m->tune_layout[0];  // batches below the first tuned size use its layout
+        for (int i = 1; i < m->ntune; ++i)
             if (m->tune_nq[i] <= nq) pick = m->tune_layout[i];
         return pick;
     }
-    const BatchCost c = batch_cost(m, nq);
-    const bool dense = m->dense_ok && (m->dense_min_nq > 0 ? nq >= m->dense_min_nq : c.dense < std::min(c.single, c.sparse));
+    const BatchCost c = batch_cost(m, nq, M);
+    const double other = std::min(c.single, c.sparse);
+    const bool dense = m->dense_ok && (m->dense_min_nq > 0 ? nq >= m->dense_min_nq : c.dense * (nq >= 16 ? 0.9 : 1.0) < other);
     return dense ? ACC_BATCH_DENSE : c.single < c.sparse ? ACC_BATCH_SINGLE : ACC_BATCH_SPARSE;
 }
 
@@ -983,7 +1005,7 @@ extern "C" int acc_gpu_topk_lowbit(acc_gpu_matrix *m, const float *x_dev, int k,
 static int run_batch(acc_gpu_matrix *m, BatchWs &ws, const float *x_dev, int nq, const int32_t *k_host, bool upload_k,
                      int kmax, int ck, acc_element *out_dev, int out_stride, hipStream_t st) {
     const int M = ck / m->split;
-    int layout = batch_layout(m, nq);
+    int layout = batch_layout(m, nq, M);
     // the packet kernels' query table of a 16-query block must fit in LDS
     if (layout == ACC_BATCH_SPARSE && (size_t)m->cols * (16 + 8) > 65536) layout = ACC_BATCH_SINGLE;
     if (layout == ACC_BATCH_SINGLE) {
@@ -1040,7 +1062,7 @@ void batch_ws_destroy(BatchWorkspace *w, int device) {
 
 int64_t batch_ws_bytes(const BatchWorkspace *w) { return w ? w->bytes : 0; }
 
-int batch_layout_of(const acc_gpu_matrix *m, int nq) { return batch_layout(m, nq); }
+int batch_layout_of(const acc_gpu_matrix *m, int nq, int ck) { return batch_layout(m, nq, ck / m->split); }
 
 int topk_lowbit_batch_ws(acc_gpu_matrix *m, BatchWorkspace *w, const float *x_dev, int nq, const int32_t *k_host,
                          int ck, acc_element *out_dev, int out_stride, void *stream) {

@@ -73,7 +73,7 @@ struct BatchWorkspace;
 BatchWorkspace *batch_ws_create();
 void batch_ws_destroy(BatchWorkspace *w, int device);
 int64_t batch_ws_bytes(const BatchWorkspace *w);
-int batch_layout_of(const acc_gpu_matrix *m, int nq);  // ACC_BATCH_* a batch of nq queries uses
+int batch_layout_of(const acc_gpu_matrix *m, int nq, int ck);  // ACC_BATCH_* a batch of nq queries uses
 int topk_lowbit_batch_ws(acc_gpu_matrix *m, BatchWorkspace *w, const float *x_dev, int nq, const int32_t *k_host,
                          int ck, acc_element *out_dev, int out_stride, void *stream);
 

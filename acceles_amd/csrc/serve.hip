@@ -342,7 +342,7 @@ extern "C" int acc_server_add_matrix(acc_server *s, const acc_csr *csr, const ac
         if (rc == ACC_OK && hipMemset(x, 0, (size_t)s->o.max_batch * csr->cols * 4) != hipSuccess) rc = ACC_ERR_DEVICE;
         std::vector<int32_t> ks((size_t)s->o.max_batch, 1);
         for (int b = 1; rc == ACC_OK && b <= s->o.max_batch; ++b) {
-            if ((b & (b - 1)) != 0 && b != s->o.max_batch && acc::batch_layout_of(m, b) == acc::batch_layout_of(m, b + 1))
+            if ((b & (b - 1)) != 0 && b != s->o.max_batch && acc::batch_layout_of(m, b, s->o.ck) == acc::batch_layout_of(m, b + 1, s->o.ck))
                 continue;
             rc = acc::topk_lowbit_batch_ws(m, w, x, b, ks.data(), s->o.ck, o, 1, nullptr);
             if (rc == ACC_OK && hipDeviceSynchronize() != hipSuccess) rc = fail(ACC_ERR_DEVICE, "warm-up batch failed");

@@ -331,8 +331,8 @@ int acc_gpu_topk_lowbit_batch(acc_gpu_matrix *m, const float *x_dev, int nq,
  * column sum past one byte, |score| >= 2^25, or more than 1024 columns);
  * ACC_BATCH_AUTO uses them when they can and the
  * batch has at least min_dense_batch queries (0 keeps the current rule; until
- * a value is set, the layout of the lowest estimated time for the matrix and
- * the batch size is used, ACC_BATCH_SINGLE and _SPARSE included). */
+ * a value is set, the layout of the lowest estimated time for the matrix, the
+ * batch size and ck is used, ACC_BATCH_SINGLE and _SPARSE included). */
 #define ACC_BATCH_AUTO 0
 #define ACC_BATCH_SPARSE 1
 #define ACC_BATCH_DENSE 2
