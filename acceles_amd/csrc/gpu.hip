@@ -766,6 +766,34 @@ extern "C" int acc_event_destroy(void *event) {
 // upload / info / destroy
 // ---------------------------------------------------------------------------
 
+// Unsigned 8-bit values are stored as v - 128 in the slice image.
+static bool image_offset(const acc_packed *pk) { return !pk->is_signed && pk->bits == 8; }
+
+// Why the matrix cores cannot score the matrix exactly (empty: they can).
+static std::string dense_refusal(const acc_packed *pk) {
+    // a byte of the slice image holds the sum of a row's values in one
+    // column (rows may name a column twice): v - 128 for unsigned
+    // 8-bit, else v
+    const int64_t lo = image_offset(pk) ? 0 : -128, hi = image_offset(pk) ? 255 : 127;
+    const int64_t maxv = std::max<int64_t>({(int64_t)pk->merged_max, -(int64_t)pk->merged_min, 1});
+    if (pk->merged_min < lo || pk->merged_max > hi)
+        return "a row's values in one column sum past one byte (a row names a column twice)";
+    if (maxv * 128 * (int64_t)pk->cols >= (int64_t(1) << 25)) return "scores may reach 2^25 (too many columns for the value width)";
+    if (pk->cols > kPkMaxCols) return "more than 1024 columns";
+    return "";
+}
+
+// What acc_gpu_upload allocates for certain (never more than it does, so that
+// what fits is not refused): all that grows with the matrix, of the image packets
+// three bytes per entry of a matrix that repeats no column in a row.
+int64_t acc::upload_bytes(const acc_csr *csr, const acc_packed *pk) {
+    const int64_t rows = csr->rows, nnz = csr->nnz(), slices = pk->nslices();
+    int64_t b = (rows + 1) * 4 + (nnz + kRowPad) * (int64_t)(4 + sizeof(colx_t)) + rows * 4 + (int64_t)fp32_sel_keys(rows) * 8;
+    b += ((int64_t)pk->words.size() + (int64_t)kWordPad) * 4 + slices * (int64_t)(sizeof(uint2) + 64 * 4 + sizeof(int4) + 1);
+    if (pk->dup_rows == 0 && dense_refusal(pk).empty()) b += pk->nnz_kept * 3 + slices * (int64_t)sizeof(uint2);
+    return b;
+}
+
 extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int device, acc_gpu_matrix **out) {
     if (!out || (!csr && !pk)) return fail(ACC_ERR_ARG, "need a CSR and/or packed matrix");
     if (csr && pk && (csr->rows != pk->rows || csr->cols != pk->cols))
@@ -897,22 +925,9 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         }
         m->cols_pad = (m->cols + 31) & ~31;
         m->nkb = m->cols_pad / 32;
-        m->u8off = (!m->is_signed && m->bits == 8) ? 1 : 0;
-        {
-            // a byte of the slice image holds the sum of a row's values in one
-            // column (rows may name a column twice): v - 128 for unsigned
-            // 8-bit, else v
-            const int64_t lo = m->u8off ? 0 : -128, hi = m->u8off ? 255 : 127;
-            const int64_t maxv = std::max<int64_t>({(int64_t)pk->merged_max, -(int64_t)pk->merged_min, 1});
-            if (pk->merged_min < lo || pk->merged_max > hi)
-                m->dense_why = "a row's values in one column sum past one byte (a row names a column twice)";
-            else if (maxv * 128 * (int64_t)m->cols >= (int64_t(1) << 25))
-                m->dense_why = "scores may reach 2^25 (too many columns for the value width)";
-            else if (m->cols > kPkMaxCols)
-                m->dense_why = "more than 1024 columns";
-            else
-                m->dense_ok = true;
-        }
+        m->u8off = image_offset(pk) ? 1 : 0;
+        m->dense_why = dense_refusal(pk);
+        m->dense_ok = m->dense_why.empty();
         if (m->dense_ok) {
             // the matrix-core scores' own copy of the slices: image bytes and
             // their offsets in a decode wavefront's 16 image rows, repeated

@@ -65,6 +65,9 @@ int bits_for(int32_t n);  // ceil(log2(n)), at least 1
 // 4 * column of n entries (cols <= 8192): the columns as the device reads them.
 void column_offsets(const int32_t *idx, int64_t n, uint16_t *out);
 
+// Device bytes that acc_gpu_upload holds for a matrix at least, before the workspaces.
+int64_t upload_bytes(const acc_csr *csr, const acc_packed *pk);
+
 // Batched low-bit queries with a workspace of the caller's (acc_gpu_topk_
 // lowbit_batch uses the handle's own, so one handle runs one batch at a
 // time): several workspaces keep several batches of one matrix in flight on

@@ -290,16 +290,6 @@ extern "C" int acc_server_create(const acc_server_opts *opts, acc_server **out) 
     return ACC_OK;
 }
 
-// Device bytes acc_gpu_upload will hold for this matrix, before the
-// workspaces: the FP32 CSR (4-byte row pointers), the packets with their
-// padding, metadata and slot map, and per-row scores.
-static int64_t upload_estimate(const acc_csr *csr, const acc_packed *pk) {
-    const int64_t nnz = csr->nnz();
-    int64_t b = ((int64_t)csr->rows + 1) * 4 + nnz * 8 + (int64_t)csr->rows * 4;
-    b += (int64_t)pk->words.size() * 4 + (int64_t)pk->nslices() * (8 + 4 + 1 + 256) + 32 * 64 * 4;
-    return b;
-}
-
 extern "C" int acc_server_add_matrix(acc_server *s, const acc_csr *csr, const acc_packed *pk, int *matrix_id) {
     if (!s || !csr || !pk || !matrix_id) return fail(ACC_ERR_ARG, "a server, the FP32 CSR and its packets are required");
     if (csr->cols > s->max_cols) return fail(ACC_ERR_ARG, "cols must be <= 8192");
@@ -307,7 +297,7 @@ extern "C" int acc_server_add_matrix(acc_server *s, const acc_csr *csr, const ac
     // admission: the matrix's bytes are reserved under the lock before the
     // upload, so concurrent additions cannot both pass against the same room;
     // the reservation is corrected to the measured bytes afterwards
-    const int64_t reserved = upload_estimate(csr, pk);
+    const int64_t reserved = acc::upload_bytes(csr, pk);
     if (!s->mem.reserve(reserved)) return fail(ACC_ERR_BUDGET, "matrix does not fit in the server's memory budget");
     auto release = [&](int rc) {
         s->mem.release(reserved);
