@@ -32,6 +32,7 @@ static constexpr size_t kWordPad = 32 * 64;  // dwords past the packets (>= wide
 // and save the selection about 5 us whatever the size (400,000 rows: 15.1 ->
 // 10.0 us), so they pay up to some 100,000 slices.
 static constexpr int64_t kTop3Slices = 65536;
+static constexpr size_t stop_dwords(int64_t nslices) { return nslices <= kTop3Slices ? 4 : 1; }
 static constexpr int kPkMaxCols = 1024;  // matrix-core scores: B operands of 32 column blocks in registers
 static constexpr size_t kPkLdsMax = 160 * 1024;  // LDS of a pk_scores workgroup at most
 
@@ -55,7 +56,7 @@ struct BatchWs {
     size_t corr_n = 0;
     uint32_t *tk = nullptr;      // four-key slice lists
     size_t tk_n = 0;
-    int4 *stop = nullptr;        // single-query passes: slices' largest scores
+    int32_t *stop = nullptr;     // single-query passes: slices' largest scores
     size_t stop_n = 0;
     float *y = nullptr;          // FP32 plans: scores
     size_t y_n = 0;
@@ -98,7 +99,7 @@ struct acc_gpu_matrix {
     int4 *d_items = nullptr;         // per workgroup
     int nitems = 0;
     std::vector<int32_t> part_row_begin;
-    int4 *d_stop = nullptr;          // per slice: the largest INT32 scores of the last query
+    int32_t *d_stop = nullptr;       // per slice: the largest INT32 scores of the last query (stop_dwords)
     uint64_t *d_resc = nullptr;      // split * kMaxM
     int32_t *d_crow = nullptr, *d_cscore = nullptr;  // split * kMaxM (candidate outputs)
     int64_t *d_part_slice = nullptr;                 // split + 1
@@ -251,7 +252,7 @@ int lds_limit(const void *fn, size_t bytes);
 // Top-K into out (K > 0) and/or the per-partition candidates into
 // crow/cscore (p*M + i).
 LowbitArgs lowbit_args(acc_gpu_matrix *m, const float *x, int M, int K, acc_element *out, int32_t *crow,
-                       int32_t *cscore, int4 *stop = nullptr, uint64_t *resc = nullptr) {
+                       int32_t *cscore, int32_t *stop = nullptr, uint64_t *resc = nullptr) {
     LowbitArgs a;
     a.words = m->d_words;
     a.slices = m->d_slices;
@@ -260,7 +261,7 @@ LowbitArgs lowbit_args(acc_gpu_matrix *m, const float *x, int M, int K, acc_elem
     a.part_slice = m->d_part_slice;
     a.nvalid = m->d_nvalid;
     a.stop = stop ? stop : m->d_stop;
-    a.top3 = m->nslices <= kTop3Slices ? 1 : 0;
+    a.top3 = stop_dwords(m->nslices) > 1 ? 1 : 0;
     a.x = x;
     a.cols = m->cols;
     a.col_bits = m->col_bits;
@@ -309,7 +310,7 @@ int launch_lowbit_stage(acc_gpu_matrix *m, const LowbitArgs &a, int stage, hipSt
 int launch_lowbit(acc_gpu_matrix *m, const float *x, int M, int K, acc_element *out, int32_t *crow, int32_t *cscore,
                   hipStream_t st, BatchWs *ws = nullptr) {
     if (ws) {
-        int rc = ws_grow(*ws, &ws->stop, &ws->stop_n, (size_t)m->nslices);
+        int rc = ws_grow(*ws, &ws->stop, &ws->stop_n, (size_t)m->nslices * stop_dwords(m->nslices));
         if (rc == ACC_OK) rc = ws_grow(*ws, &ws->resc, &ws->resc_n, (size_t)m->split * kMaxM);
         if (rc != ACC_OK) return rc;
     }
@@ -789,7 +790,7 @@ static std::string dense_refusal(const acc_packed *pk) {
 int64_t acc::upload_bytes(const acc_csr *csr, const acc_packed *pk) {
     const int64_t rows = csr->rows, nnz = csr->nnz(), slices = pk->nslices();
     int64_t b = (rows + 1) * 4 + (nnz + kRowPad) * (int64_t)(4 + sizeof(colx_t)) + rows * 4 + (int64_t)fp32_sel_keys(rows) * 8;
-    b += ((int64_t)pk->words.size() + (int64_t)kWordPad) * 4 + slices * (int64_t)(sizeof(uint2) + 64 * 4 + sizeof(int4) + 1);
+    b += ((int64_t)pk->words.size() + (int64_t)kWordPad) * 4 + slices * (int64_t)(sizeof(uint2) + 64 * 4 + 4 * stop_dwords(slices) + 1);
     if (pk->dup_rows == 0 && dense_refusal(pk).empty()) b += pk->nnz_kept * 3 + slices * (int64_t)sizeof(uint2);
     return b;
 }
@@ -898,7 +899,7 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         TRY(dalloc(m, &m->d_slices, sl.size()));
         TRY(dalloc(m, &m->d_perm, pk->perm.size()));
         TRY(dalloc(m, &m->d_items, items.size()));
-        TRY(dalloc(m, &m->d_stop, (size_t)m->nslices));
+        TRY(dalloc(m, &m->d_stop, (size_t)m->nslices * stop_dwords(m->nslices)));
         TRY(dalloc(m, &m->d_resc, (size_t)m->split * kMaxM));
         TRY(dalloc(m, &m->d_crow, (size_t)m->split * kMaxM));
         TRY(dalloc(m, &m->d_cscore, (size_t)m->split * kMaxM));

@@ -129,10 +129,13 @@ __global__ __launch_bounds__(LB_WG) void lowbit_slicemax(LowbitArgs a) {
             hold_group(w[j]);
             acc = decode_group<E, SIGNED>(w[j], dnd[j], qx, a.col_bits, a.val_bits, acc);
             if (dend[j]) {
-                // without the top three: second and third unknown
-                const int4 t = a.top3 ? top3(acc)
-                                      : make_int4(__builtin_amdgcn_readlane(wave_max_lane63(acc), 63), INT32_MAX, INT32_MAX, 0);
-                if (lane == 0) a.stop[ds[j]] = t;
+                if (a.top3) {
+                    const int4 t = top3(acc);
+                    if (lane == 0) ((int4 *)a.stop)[ds[j]] = t;
+                } else {
+                    const int32_t t = wave_max_lane63(acc);
+                    if (lane == 63) a.stop[ds[j]] = t;
+                }
                 acc = 0;
             }
             issue((j + 2) % RING, false);
@@ -190,7 +193,11 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
     const int p = blockIdx.x;
     const int64_t s0 = a.part_slice[p];
     const int nsl = (int)(a.part_slice[p + 1] - s0);
-    const int4 *stop = a.stop + s0;
+    const int sw = a.top3 ? 4 : 1;  // dwords per slice
+    const int32_t *stop = a.stop + s0 * sw;
+    auto scores = [&](int i) {  // of slice i; without the top three second and third are unknown
+        return a.top3 ? ((const int4 *)stop)[i] : make_int4(stop[i], INT32_MAX, INT32_MAX, 0);
+    };
     const int32_t *perm = a.perm + s0 * 64;
     const bool regs = nsl <= V * SEL_WG, one = nsl <= SEL_WG;
     // the query and the thread's slices; one uniform test around loads with
@@ -200,14 +207,17 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
     load_query(a.x, a.cols, xr);
     int4 st[V];
     int32_t r1 = -1, r2 = -1;  // one: the rows of the slice's two best scores
-    auto load = [&](auto n) {
+    auto load = [&](auto n, auto get) {
 #pragma unroll
         for (int u = 0; u < V; ++u)
-            st[u] = u < decltype(n)::value ? stop[min(tid + u * SEL_WG, nsl - 1)] : make_int4(0, 0, 0, 0);
+            st[u] = u < decltype(n)::value ? get(min(tid + u * SEL_WG, nsl - 1)) : make_int4(0, 0, 0, 0);
     };
-    if (nsl <= 0 || !regs) load(std::integral_constant<int, 0>());
-    else if (one) load(std::integral_constant<int, 1>());
-    else load(std::integral_constant<int, V>());
+    auto three = [&](int i) { return ((const int4 *)stop)[i]; };
+    auto largest = [&](int i) { return make_int4(stop[i], INT32_MAX, INT32_MAX, 0); };
+    if (nsl <= 0 || !regs) load(std::integral_constant<int, 0>(), three);
+    else if (!a.top3) load(std::integral_constant<int, V>(), largest);
+    else if (one) load(std::integral_constant<int, 1>(), three);
+    else load(std::integral_constant<int, V>(), three);
     // every slice is full except a partition's last one
     const int nfull = nsl <= 0 || a.nvalid[s0 + nsl - 1] == 64 ? nsl : nsl - 1;
     if (tid == 0) {
@@ -239,7 +249,7 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
 #pragma unroll
                 for (int u = 0; u < V; ++u) fn(mkey(st[u].x, tid + u * SEL_WG < nfull));
             } else {
-                for (int i = tid; i < nsl; i += SEL_WG) fn(mkey(stop[i].x, i < nfull));
+                for (int i = tid; i < nsl; i += SEL_WG) fn(mkey(stop[(size_t)i * sw], i < nfull));
             }
         },
         a.M, s_hist, s_t32, s_need, kSlack);
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
         for (int u = 0; u < V; ++u)
             if (u * SEL_WG < nsl) offer(tid + u * SEL_WG, st[u]);
     } else {
-        for (int b = 0; b < nsl; b += SEL_WG) offer(b + tid, stop[min(b + tid, nsl - 1)]);
+        for (int b = 0; b < nsl; b += SEL_WG) offer(b + tid, scores(min(b + tid, nsl - 1)));
     }
     lds_barrier();
     const int ncand = s_cnt;
@@ -414,7 +424,7 @@ __global__ __launch_bounds__(SEL_WG) void lowbit_select(LowbitArgs a) {
         WaveTopM<2> col;
         col.init(colbuf + wave * WaveTopM<2>::cap, a.M);
         for (int b = wave * 64; b < nsl; b += SEL_WG) {
-            uint64_t mask = __ballot(b + lane < nsl && stop[min(b + lane, nsl - 1)].x >= ts);
+            uint64_t mask = __ballot(b + lane < nsl && stop[(size_t)min(b + lane, nsl - 1) * sw] >= ts);
             while (mask) {
                 const int l = __builtin_ctzll(mask);
                 mask &= mask - 1;

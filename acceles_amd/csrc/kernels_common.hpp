@@ -606,8 +606,8 @@ struct LowbitArgs {
     const int4 *items;          // per workgroup: (partition, first slice, end slice, 0)
     const int64_t *part_slice;  // split + 1 slice offsets
     const uint8_t *nvalid;      // rows per slice (64 except a partition's last)
-    int4 *stop;                 // per slice: its three largest INT32 scores, the lanes of the first two
-    int top3;                   // stop holds three scores (0: the largest only)
+    int32_t *stop;              // top3: per slice its three largest INT32 scores and the lanes of the
+    int top3;                   // first two (16 bytes); else its largest score only
     const float *x;             // FP32 query (cols)
     int cols, col_bits, val_bits;
     int split, M;               // partitions, rows kept per partition
