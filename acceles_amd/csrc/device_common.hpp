@@ -353,9 +353,3 @@ struct WaveTopM {
         }
     }
 };
-
-__device__ __forceinline__ int next_pow2(int v) {
-    int p = 1;
-    while (p < v) p <<= 1;
-    return p;
-}

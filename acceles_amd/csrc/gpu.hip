@@ -291,7 +291,7 @@ int launch_lowbit_stage(acc_gpu_matrix *m, const LowbitArgs &a, int stage, hipSt
         lowbit_fn ksel = get_lowbit_select(m->entry_bits, m->is_signed != 0);
         if (!ksel) return fail(ACC_ERR_ARG, "unsupported entry width");
         const size_t lds_sel = 64 + 8 * 4096 + 4 * (size_t)((m->cols + 15) & ~15);  // key list, FP32 query
-        int rc = lds_limit((const void *)ksel, lds_sel + 49152);                    // plus about 44 KB static
+        int rc = lds_limit((const void *)ksel, lds_sel + 32768);                    // plus 29 KB static
         if (rc != ACC_OK) return rc;
         LAUNCH(m, 1, ksel, dim3(m->split), dim3(SEL_WG), lds_sel, st, a);
     } else if (a.K <= 256 && m->split * a.M <= 4 * SEL_WG) {
@@ -550,8 +550,7 @@ int launch_dense(acc_gpu_matrix *m, BatchWs &ws, const float *X, int nq, int M, 
 
     LAUNCH(m, 0, get_dense_prep(), dim3(nqb * QB), dim3(ACC_WG), 0, st, a);
     if ((rc = check_launch()) != ACC_OK) return rc;
-    dense_fn fs = pk_kernel(m, tpw, wide, rows);
-    if (!fs) return fail(ACC_ERR_ARG, "unsupported entry width");
+    const dense_fn fs = pk_kernel(m, tpw, wide, rows);
     // two slice images (one multiplied while the other is cleared and refilled)
     const size_t img = (size_t)64 * (m->cols_pad + 16);
     const size_t lds_s = 2 * img + kPkLdsTail + (rows ? (size_t)NT * 2048 : 0);  // and the row tiles' lists
@@ -614,8 +613,8 @@ size_t radix_select_keys(int64_t n, int K) {
     return total;
 }
 
-// Keys of an FP32 query's selection buffer: the radix passes', or the two
-// largest of every wavefront's rows.
+// Keys of an FP32 query's selection buffer: the radix passes', or the three
+// largest of every group's rows (wavefronts or workgroups).
 size_t fp32_sel_keys(int64_t rows) { return std::max<size_t>(radix_select_keys(rows, 256), 3 * kMaxGroups); }
 
 // Radix Top-K (K <= 256) of n scores; buf holds radix_select_keys(n, K) keys.

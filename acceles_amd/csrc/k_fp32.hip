@@ -2,13 +2,13 @@
 //   fp32_spmv       FP32 CSR SpMV (cpu_mkl_baseline.cpp:261);
 //   fp32_select_groups
 //                   Top-K of its scores (cpu_mkl_baseline.cpp:128-149) from
-//                   the two best keys of each wavefront's rows; together they
-//                   are the plain FP32 CSR Top-K path
+//                   the three best keys of each group's rows (wavefronts or
+//                   workgroups); together they are the plain FP32 CSR Top-K path
 //                   (host_spmv_topk_csr_gpu.cu:171-231 is the GPU spec);
 //   select_radix_pass / select_radix_final (K <= 256),
 //   select_blocks / select_final (any K <= 960)
 //                   Top-K of any score vector, and of a matrix with fewer
-//                   than K wavefronts' worth of rows;
+//                   than K groups' worth of rows;
 //   spmv_fp64       FP64 exact scores for precision/recall reporting.
 #include "kernels_common.hpp"
 

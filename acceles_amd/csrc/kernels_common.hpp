@@ -5,9 +5,11 @@
 //   lowbit_slicemax query quantization (quantify_util.py:31-49, 259) and the
 //                   INT32 SpMV over sliced packets (quantify_util.py:5-6;
 //                   spmv_ucsr_top_k_multicore.hpp:195-355 on the FPGA),
-//                   keeping the maximum of each 64-row slice;
-//   lowbit_select   per partition: exact threshold from the slice maxima,
-//                   rescan of the slices that reach it, its Top-M
+//                   keeping the three largest scores of each 64-row slice
+//                   (of many slices the largest);
+//   lowbit_select   per partition: a threshold that about M of them reach,
+//                   the listed rows that reach it, exact rescan of the slices
+//                   that may hold more, its Top-M
 //                   (quantify_util.py:173-196, host_spmv_ucsr.cpp:691-748)
 //                   and the FP32 rescoring of those rows
 //                   (quantify_util.py:354-367);
@@ -17,10 +19,12 @@
 // costs microseconds per workgroup.
 //   lowbit_scores   INT32 scores of every row (parity checks).
 //   fp32_spmv       plain FP32 CSR SpMV (cpu_mkl_baseline.cpp:261).
-//   select_blocks / select_final
-//                   Top-K of a score vector (cpu_mkl_baseline.cpp:128-149);
-//                   with fp32_spmv it is the plain FP32 CSR Top-K path
-//                   (host_spmv_topk_csr_gpu.cu:171-231 is the GPU spec).
+//   fp32_select_groups
+//                   Top-K of its scores; together they are the plain FP32 CSR
+//                   Top-K path (host_spmv_topk_csr_gpu.cu:171-231 is the GPU
+//                   spec).
+//   select_radix_pass / _final, select_blocks / select_final
+//                   Top-K of any score vector (cpu_mkl_baseline.cpp:128-149).
 //   spmv_fp64       FP64 exact scores for precision/recall reporting.
 #pragma once
 
@@ -711,15 +715,17 @@ struct QTable {
 //   pk_scores      v_mfma_i32_32x32x32_i8 over each 64-row slice and a block
 //                  of queries: decode wavefronts expand the slice's image
 //                  packets (the same slices re-encoded at upload: per entry
-//                  the image byte and cols - column, a row's repeated columns
-//                  merged) into an LDS image of the A operands, each MFMA wavefront
+//                  the image byte and its offset in a decode wavefront's 16 image
+//                  rows, a row's repeated columns merged) into an LDS image of
+//                  the A operands, each MFMA wavefront
 //                  holds its query tile's B operands in registers; per (query,
 //                  slice) only the four best (score, row-in-slice) keys are
 //                  kept;
-//   dense_select   per (partition, query): threshold = the M-th best slice
-//                  maximum, candidates from the four-key lists, exact rescan
-//                  (from the packets) of any slice whose list may have dropped
-//                  a candidate, Top-M, and the FP32 rescoring of those M rows;
+//   dense_select_regs, dense_select
+//                  per (partition, query): threshold = about the M-th best
+//                  slice maximum, candidates from the four-key lists, exact
+//                  scores (from the packets) of rows that a list may have
+//                  dropped, Top-M, and the FP32 rescoring of those M rows;
 //   batch_topk     per query: its Top-K[q] of the rescored keys.
 //
 // Image of a slice (LDS): row r of the slice at r * (cols_pad + 16), one
