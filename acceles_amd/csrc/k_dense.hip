@@ -458,7 +458,7 @@ template <int U>
 __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
     constexpr int kSlack = 8, kRescans = 8;  // slices rescanned one after the other
     extern __shared__ __align__(16) unsigned char smem[];
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
+    const int wave = threadIdx.x >> 6, lane = lane_id();
     const int p = blockIdx.x, q = blockIdx.y * ACC_WAVES + wave;
     if (q >= a.nq) return;  // whole wavefront; no workgroup barrier below
     // per wavefront (2 KB): 64 candidates; 64 ranked keys and their entry
@@ -516,12 +516,7 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
             const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
 #pragma unroll
             for (int e = 0; e < 4; ++e) c += tk_rho(ke[e]) < nv && ke[e] >= tk ? 1 : 0;
-            const uint64_t m = __ballot(k4[u].w >= tk);
-            const int j = nr + mbcnt64(m);
-            if (k4[u].w >= tk && j < kRescans)
-                keys[j] = ((uint64_t)k4[u].w << 32) |
-                          (uint32_t)((u * 64 + lane) << 18 | tk_rho(k4[u].z) << 12 | tk_rho(k4[u].y) << 6 | tk_rho(k4[u].x));
-            nr += __popcll(m);
+            nr += __popcll(__ballot(k4[u].w >= tk));
         }
         const int incl = (int)wave_prefix_sum((uint32_t)c);
         const int nl = __builtin_amdgcn_readlane(incl, 63);
@@ -550,6 +545,17 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
         const int32_t ts = t != 0u ? tk_score(t) : INT32_MIN;
         bool many = nl > 64 || nr > kRescans, zero = true;
         if (nr > 0) {
+            int i = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint64_t m = __ballot(k4[u].w >= tk);
+                const int j = i + mbcnt64(m);
+                if (k4[u].w >= tk && j < kRescans)
+                    keys[j] = ((uint64_t)k4[u].w << 32) |
+                              (uint32_t)((u * 64 + lane) << 18 | tk_rho(k4[u].z) << 12 | tk_rho(k4[u].y) << 6 | tk_rho(k4[u].x));
+                if (lane == 0) again[u] = m;
+                i += __popcll(m);
+            }
             // at most 1,024 columns, padded to whole dwords: one round trip
             const uint32_t *src = (const uint32_t *)(a.qplain + (size_t)q * a.cols_pad);
             const int nd = a.cols_pad / 4;
@@ -581,11 +587,7 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
             n += many ? 0 : __popcll(m);
         }
         if (many) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint64_t m = __ballot(k4[u].w >= tk);
-                if (lane == 0) again[u] = m;
-            }
+            if (nr == 0 && lane < U) again[lane] = 0ull;
             wave_sync();
             n = select_with_rescans(a, q, s0, nsl, nvl, nl, tk, ts, cand, again, qx, zero, k);
         } else if (nr > 0) {
