@@ -37,10 +37,12 @@
 // stored column is its address.
 //
 // The area: 896 entries at 6 bytes leave five workgroups per CU at 900
-// columns.  2,000,000 x 900 (rows of 30-90, G = 16): 141 us, 5.1 TB/s; with
+// columns.  2,000,000 x 900 (rows of 30-90, G = 16): 138 us, 5.2 TB/s; with
 // areas of 768 / 1024 / 1536 entries 145 / 162 / 143 us; loading the rows'
 // entries with 4-byte loads and 4-byte columns 286 us.  4,999,999 x 1024
-// power-law rows (G = 8): 196 us (768: 211, 1024: 232; before: 258).
+// power-law rows (G = 8): 175 us (258 with such loads; under the profiler, which
+// adds a tenth to this kernel, 196 against 211 with 768 entries and 232 with
+// 1024: the other figures for these rows below are under it too).
 // 100,000 x 500 (rows of 50-90, G = 32): 11.2 us (before: 15.3).
 static constexpr int kFp32Stage = 896;   // entries per wavefront staged in LDS
 static constexpr int kFp32Slack = 128;   // readable past them (the last batch of a row reads up to U*G - 1 further)

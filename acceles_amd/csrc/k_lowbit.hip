@@ -55,9 +55,9 @@ __device__ __forceinline__ int4 top3(int32_t v) {
 // may be too high; lowbit_select rescans it.  Without top3 only the largest
 // is known, and lowbit_select rescans every slice that it needs.
 //
-// Bound: HBM (20,000,000 x 1024: 146 us, 6.4 TB/s of packets; 159 before the
-// decode took four instructions per entry instead of six and the loads stayed
-// in flight).  Small matrices: latency (400,000 x 500: 12.4 us, 13.4 before
+// Bound: HBM (20,000,000 x 1024: 142 us, 6.5 TB/s of packets; 146 when 16 bytes
+// per slice were written there too, 159 before the decode took four instructions
+// per entry instead of six and the loads stayed in flight).  Small matrices: latency (400,000 x 500: 12.4 us, 13.4 before
 // the first packets were loaded ahead of the query's quantization).
 template <int E, bool SIGNED>
 __global__ __launch_bounds__(LB_WG) void lowbit_slicemax(LowbitArgs a) {
