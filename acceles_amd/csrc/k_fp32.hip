@@ -415,7 +415,8 @@ __global__ __launch_bounds__(1024) void fp32_select_groups(SelectGroupsArgs a) {
                 const uint32_t end = min((uint32_t)dkey_row(T), rows - 1u);
                 const bool ties = (k3 >> 32) == (T >> 32);
                 s_last[i] = ties ? end : rows - 1u;
-                atomicAdd(&s_rows, !ties ? L : (end / (nw * RS) + 1u) * RS * (k1 - k3 < RS ? kSelDense : 1u));
+                const uint32_t n = !ties ? L : (end / (nw * RS) + 1u) * RS * (k1 - k3 < RS ? kSelDense : 1u);
+                atomicAdd(&s_rows, min(n, 1u << 20));  // (the sum of 1,024 of them fits)
             }
         }
     };
