@@ -103,6 +103,7 @@ struct acc_gpu_matrix {
     uint64_t *d_resc = nullptr;      // split * kMaxM
     int32_t *d_crow = nullptr, *d_cscore = nullptr;  // split * kMaxM (candidate outputs)
     int64_t *d_part_slice = nullptr;                 // split + 1
+    int32_t *d_part_row = nullptr;                   // split + 1 first rows (null: rows dealt out otherwise)
     int64_t max_part_slices = 0;                     // slices of the largest partition
     uint32_t *d_pwords = nullptr;                    // image packets (matrix-core scores)
     uint2 *d_pslices = nullptr;
@@ -259,6 +260,7 @@ LowbitArgs lowbit_args(acc_gpu_matrix *m, const float *x, int M, int K, acc_elem
     a.perm = m->d_perm;
     a.items = m->d_items;
     a.part_slice = m->d_part_slice;
+    a.part_row = m->d_part_row;
     a.nvalid = m->d_nvalid;
     a.stop = stop ? stop : m->d_stop;
     a.top3 = stop_dwords(m->nslices) > 1 ? 1 : 0;
@@ -904,6 +906,16 @@ extern "C" int acc_gpu_upload(const acc_csr *csr, const acc_packed *pk, int devi
         TRY(dalloc(m, &m->d_cscore, (size_t)m->split * kMaxM));
         TRY(dalloc(m, &m->d_part_slice, (size_t)m->split + 1));
         COPY(m->d_part_slice, pk->part_slice_begin.data(), ((size_t)m->split + 1) * 8);
+        bool in_range = pk->shuffle_seed == 0;  // each partition holds the rows of its range (a file may say otherwise)
+        for (int p = 0; p < m->split && in_range; ++p)
+            for (int64_t i = pk->part_slice_begin[(size_t)p] * 64; i < pk->part_slice_begin[(size_t)p + 1] * 64; ++i) {
+                const int32_t r = pk->perm[(size_t)i];
+                in_range = in_range && (r < 0 || (r >= pk->part_row_begin[(size_t)p] && r < pk->part_row_begin[(size_t)p + 1]));
+            }
+        if (in_range) {
+            TRY(dalloc(m, &m->d_part_row, (size_t)m->split + 1));
+            COPY(m->d_part_row, pk->part_row_begin.data(), ((size_t)m->split + 1) * 4);
+        }
         for (int p = 0; p < m->split; ++p)
             m->max_part_slices = std::max<int64_t>(m->max_part_slices,
                                                    pk->part_slice_begin[(size_t)p + 1] - pk->part_slice_begin[(size_t)p]);

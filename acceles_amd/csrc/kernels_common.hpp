@@ -609,6 +609,7 @@ struct LowbitArgs {
     const int32_t *perm;        // slot -> row (-1: padding lane)
     const int4 *items;          // per workgroup: (partition, first slice, end slice, 0)
     const int64_t *part_slice;  // split + 1 slice offsets
+    const int32_t *part_row;    // split + 1 first rows (null: rows are dealt to partitions in another order)
     const uint8_t *nvalid;      // rows per slice (64 except a partition's last)
     int32_t *stop;              // top3: per slice its three largest INT32 scores and the lanes of the
     int top3;                   // first two (16 bytes); else its largest score only
