@@ -306,50 +306,4 @@ struct WaveTopM {
         wave_sync();
         n += c;
     }
-    // Offers U keys per lane at once: the lanes' counts are prefix-summed
-    // over the wavefront and the admitted keys are written to their slots in
-    // one pass.  When they do not all fit, the buffer is filled, compacted
-    // (which may raise the admission threshold) and the rest offered again.
-    template <int U>
-    __device__ void push_many(const bool (&pred)[U], const uint64_t (&key)[U]) {
-        const int lane = lane_id();
-        bool pend[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) pend[u] = pred[u];
-        for (;;) {
-            int c = 0;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                pend[u] = pend[u] && key[u] > thr;
-                c += pend[u] ? 1 : 0;
-            }
-            int incl = c;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int t = __shfl_up(incl, o);
-                if (lane >= o) incl += t;
-            }
-            const int tot = __builtin_amdgcn_readlane(incl, 63);
-            if (tot == 0) return;
-            const int room = cap - n;  // >= cap - M >= 64 after a compaction
-            int pos = incl - c;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (pend[u]) {
-                    if (pos < room) {
-                        buf[n + pos] = key[u];
-                        pend[u] = false;
-                    }
-                    ++pos;
-                }
-            }
-            wave_sync();
-            if (tot <= room) {
-                n += tot;
-                return;
-            }
-            n = cap;
-            compact();
-        }
-    }
 };

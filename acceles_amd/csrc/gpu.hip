@@ -398,6 +398,7 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
     a.pslices = m->d_pslices;
     a.perm = m->d_perm;
     a.part_slice = m->d_part_slice;
+    a.part_row = m->d_part_row;
     a.nvalid = m->d_nvalid;
     a.nslices = m->nslices;
     a.cols = m->cols;
@@ -419,7 +420,7 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
 // Fitted to 952 measurements (3,000 to 5,000,000 rows of 3 to 300 entries, 1 to
 // 256 queries, M = 1 to 64, partitions of 2 to 7,800 slices); us single /
 // packets / matrix cores at 8 queries, CK 512 unless given:
-//   20,000 x 500 172 / 66 / 38, CK 1024 in 16 partitions 269 / 84 / 147
+//   20,000 x 500 172 / 66 / 38, CK 1024 in 16 partitions 273 / 84 / 132
 //   3,000 x 120, CK 256 in 16 partitions 175 / 30 / 38
 //   400,000 x 500 209 / 98 / 42, 1,000,000 x 250 4-bit 199 / 114 / 52
 //   2,000,000 x 64, 3.5 entries per row 189 / 127 / 75
@@ -431,7 +432,8 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
 // matrix cores pay per slice the decode (0.8 ns per entry) or the
 // multiplications, whichever takes longer, and the slices they expect to rescan:
 // those with four of their partition's best M rows (Poisson; the slowest
-// wavefront bounds the launch), or every row where the lists hold fewer than M.
+// wavefront bounds the launch), or every row where the lists hold fewer than M;
+// past 48 rows more than the 64 candidates that one step ranks.
 struct BatchCost {
     double single, sparse, dense;
 };
@@ -449,9 +451,10 @@ BatchCost batch_cost(const acc_gpu_matrix *m, int nq, int M) {
     c.dense = 20.0 + 0.23e-3 * nq * cand +
               load * ((tiles + per - 1) / per) * std::max(0.8e-6 * (double)m->nnz, (m->nkb > 16 ? 4.8e-3 : 1.7e-3) * slices);
     const double l = M / part, full = part * (1.0 - std::exp(-l) * (1.0 + l + l * l / 2.0 + l * l * l / 6.0));
-    const double rescans = std::min(part, full + 1.5 * std::sqrt(full));
-    if (M > 32 || m->max_part_slices > 1024) c.dense += 22.0 + 0.012 * part + 8.0 * rescans;  // the collector (k_dense.hip)
-    else c.dense += 4 * (int64_t)(m->rows / m->split / 64) < M ? 14.0 : (1.0 + 0.05 * mean) * rescans;
+    if (m->max_part_slices > 1024) c.dense += 25.0 + 0.0145 * part;  // the lists are streamed (dense_select)
+    if (4 * (int64_t)(m->rows / m->split / 64) < M) c.dense += 3.0 + (2.5 + 0.07 * mean) * part;
+    else if (M > 48) c.dense += 2.0 + 0.27 * mean + (1.5 + 0.065 * mean) * std::min(part, full + 2.0 * std::sqrt(full));
+    else c.dense += (1.0 + 0.05 * mean) * std::min(part, full + 1.5 * std::sqrt(full));
     return c;
 }
 
@@ -568,9 +571,9 @@ int launch_dense(acc_gpu_matrix *m, BatchWs &ws, const float *X, int nq, int M, 
     if ((rc = check_launch()) != ACC_OK) return rc;
     // per wavefront: two key buffers, the int8 query (rescans), the FP32 query (rescoring)
     const size_t lds_sel = (size_t)ACC_WAVES * 256 * 8 + (size_t)ACC_WAVES * m->cols_pad * 5;
-    // up to 1,024 slices per partition and M <= 32: the lists in registers, for
-    // the largest partition (more registers, fewer wavefronts per SIMD)
-    const dense_fn fsel = get_dense_select(m->max_part_slices, M);
+    // up to 1,024 slices per partition: the lists in registers, for the largest
+    // partition (more registers, fewer wavefronts per SIMD)
+    const dense_fn fsel = get_dense_select(m->max_part_slices);
     if ((rc = lds_limit((const void *)fsel, lds_sel)) != ACC_OK) return rc;
     LAUNCH(m, 2, fsel, dim3(m->split, (nq + ACC_WAVES - 1) / ACC_WAVES), dim3(ACC_WG), lds_sel, st, a);
     if ((rc = check_launch()) != ACC_OK) return rc;

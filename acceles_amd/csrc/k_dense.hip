@@ -153,50 +153,6 @@ __global__ __launch_bounds__(ACC_WG) void dense_prep(DenseArgs a) {
     }
 }
 
-// Offers the listed keys (k4[u] = the list of slice s0 + b + u*64 + lane) scoring >= ts to the collector; a
-// slice whose list may have dropped such a row is rescanned exactly (from its
-// packets).  Keys of padding rows are discarded, and since they may have
-// displaced real rows from a list, every list whose fourth key scores >= ts
-// is rescanned.  Rows are looked up for the offered keys only.
-template <int U>
-__device__ __forceinline__ void offer_lists(const DenseArgs &a, WaveTopM<2> &cb, const uint4 (&k4)[U], const int (&nv)[U],
-                                   int64_t s0, int b, int32_t ts, int q, int8_t *qx, bool &have_qx) {
-    const int lane = lane_id();
-    bool rescan[U], pass[U * 4];
-    uint64_t key[U * 4];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        rescan[u] = nv[u] > 0 && tk_score(k4[u].w) >= ts;
-        const int64_t s = min(s0 + b + u * 64 + lane, a.nslices - 1);
-        const uint32_t ke[4] = {k4[u].x, k4[u].y, k4[u].z, k4[u].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            pass[u * 4 + e] = !rescan[u] && tk_rho(ke[e]) < nv[u] && tk_score(ke[e]) >= ts;
-            const int32_t r = pass[u * 4 + e] ? a.perm[s * 64 + tk_rho(ke[e])] : 0;
-            key[u * 4 + e] = dkey_i32(tk_score(ke[e]), r);
-        }
-    }
-    cb.push_many<U * 4>(pass, key);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        uint64_t mask = __ballot(rescan[u]);
-        while (mask) {
-            const int l = __builtin_ctzll(mask);
-            mask &= mask - 1;
-            if (!have_qx) {
-                const int8_t *src = a.qplain + (size_t)q * a.cols_pad;
-                for (int c = lane; c < a.cols_pad; c += 64) qx[c] = src[c];
-                wave_sync();
-                have_qx = true;
-            }
-            const int64_t s = s0 + b + u * 64 + l;
-            const int32_t sc = slice_dot_packets(a, s, qx);
-            const int32_t r = a.perm[s * 64 + lane];
-            cb.push(r >= 0 && sc >= ts, dkey_i32(sc, r));
-        }
-    }
-}
-
 // Copies the FP32 query (cols values) into this wavefront's LDS: eight
 // clamped loads per lane are issued together per 512 columns (a loop of
 // single loads would wait for each one before its LDS write).
@@ -209,46 +165,6 @@ __device__ __forceinline__ void stage_query(float *xs, const float *xq, int cols
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (c0 + u * 64 + lane < cols) xs[c0 + u * 64 + lane] = t[u];
-    }
-}
-
-// Stage-1 outputs of one (query, partition) and its FP32 rescoring
-// (quantify_util.py:354-367): keys[0, nn) are the partition's Top-M in rank
-// order (LDS); slot i of the candidate list is keys[i] or empty past nn.
-// Each group of G lanes rescores C candidates at once in the declared order
-// (strided fmaf, then the butterfly), so the scores equal those of every
-// other rescoring path; xs is the FP32 query, staged in LDS.
-__device__ __forceinline__ void emit_candidates(const DenseArgs &a, const uint64_t *keys, int nn, size_t base,
-                                                const float *xs) {
-    const int lane = lane_id(), M = a.M;
-    if (a.cand_rows_out)
-        for (int i = lane; i < M; i += 64) {
-            const uint64_t key = i < nn ? keys[i] : 0ull;
-            a.cand_rows_out[base + i] = key ? dkey_row(key) : -1;
-            a.cand_scores_out[base + i] = key ? dkey_score_i32(key) : 0;
-        }
-    if (!a.out) return;
-    constexpr int C = 4;
-    const int G = a.G, groups = 64 / G, grp = lane / G;
-    wave_sync();
-    for (int i0 = 0; i0 < M; i0 += groups * C) {
-        int32_t r[C];
-        bool valid[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int i = i0 + c * groups + grp;
-            const uint64_t key = keys[min(i, 63)];
-            valid[c] = i < nn;
-            r[c] = valid[c] ? dkey_row(key) : 0;
-        }
-        float sc[C];
-        group_dot_rt_multi<C, 4>(a.ptr, a.idx, a.val, xs, r, valid, G, sc);
-        if ((lane & (G - 1)) == 0)
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const int i = i0 + c * groups + grp;
-                if (i < M) a.resc[base + i] = valid[c] ? dkey_f32(sc[c], r[c]) : 0ull;
-            }
     }
 }
 
@@ -312,31 +228,99 @@ __device__ __forceinline__ void rescore_rows(const DenseArgs &a, const uint64_t 
     }
 }
 
+// Top-M of the n candidates k (lane i < n; ranked by counting) into keys, with
+// their CSR entry ranges (in flight meanwhile), then the stage-1 outputs of
+// this (query, partition) and the FP32 rescoring of those rows.
+__device__ __forceinline__ void finish_rows(const DenseArgs &a, uint64_t k, int n, uint64_t *keys, uint2 *ranges, size_t base,
+                                            const float *xs) {
+    const int lane = lane_id(), M = a.M;
+    uint2 rg = make_uint2(0u, 0u);
+    if (a.out && n > 0) {  // out set: the CSR is present
+        const int32_t r = lane < n ? dkey_row(k) : 0;
+        rg = make_uint2(a.ptr[r], a.ptr[r + 1]);
+    }
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += readlane_u64(k, j) > k;  // distinct: one per row
+    const int nn = min(n, M);
+    if (lane < n && rank < nn) {
+        keys[rank] = k;
+        ranges[rank] = rg;
+    }
+    wave_sync();
+    if (a.cand_rows_out)
+        for (int i = lane; i < M; i += 64) {
+            a.cand_rows_out[base + i] = i < nn ? dkey_row(keys[i]) : -1;
+            a.cand_scores_out[base + i] = i < nn ? dkey_score_i32(keys[i]) : 0;
+        }
+    if (!a.out) return;
+    switch (a.G) {
+        case 2: return rescore_rows<2>(a, keys, ranges, nn, base, xs);
+        case 4: return rescore_rows<4>(a, keys, ranges, nn, base, xs);
+        case 8: return rescore_rows<8>(a, keys, ranges, nn, base, xs);
+        case 16: return rescore_rows<16>(a, keys, ranges, nn, base, xs);
+        default: return rescore_rows<32>(a, keys, ranges, nn, base, xs);
+    }
+}
+
+// The query's int8 values into this wavefront's LDS (at most 1,024 columns, padded
+// to whole dwords: one round trip); true if all are zero (padding of a batch).
+__device__ __forceinline__ bool stage_qx(const DenseArgs &a, int q, int8_t *qx) {
+    const uint32_t *src = (const uint32_t *)(a.qplain + (size_t)q * a.cols_pad);
+    const int nd = a.cols_pad / 4, lane = lane_id();
+    uint32_t v[4], any = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = src[min(j * 64 + lane, nd - 1)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (j * 64 + lane < nd) ((uint32_t *)qx)[j * 64 + lane] = v[j];
+        any |= v[j];
+    }
+    wave_sync();
+    return !__any(any != 0u);
+}
+
+// The partition's n best rows for a query of zeros: every score is 0, so its first
+// M; lane i < n: the i-th.
+__device__ __forceinline__ uint64_t first_rows(const DenseArgs &a, int p, int &n) {
+    const int32_t r0 = a.part_row[p];
+    n = min(a.M, (int)(a.part_row[p + 1] - r0));
+    return lane_id() < n ? dkey_i32(0, r0 + lane_id()) : 0ull;
+}
+
 // Candidates of one (query, partition) where more than 64 rows, or those of many
 // slices besides the listed ones, may qualify (equal scores): k is left with the
 // best of them (lane i < n: the i-th, or in no order as long as 64 hold them
 // all), n returned.  nl: the number listed (keys of tk or above), in k up to 64;
-// ts: the score that another row must reach; again: the slices whose fourth key
-// does, a bit each; cand: 64 keys, then room for 704 slots; qx: the quantized
-// query (LDS); zero: it is all zeros (padding of a batch), and so are the scores.
+// ts: the score that another row must reach; cand: 64 keys, then 384 dwords
+// (LDS); qx, zero: stage_qx's.
 // A row of a slice scores its fourth key's score at most, so with the M-th best
 // key found so far only rows that this score would put above it are scored: of
-// equal scores the lower rows.  64 of them at a time, of any slices.
-__device__ __forceinline__ int select_with_rescans(const DenseArgs &a, int q, int64_t s0, int nsl, int nvl, int nl,
-                                                   uint32_t tk, int32_t ts, uint64_t *cand, const uint64_t *again,
-                                                   const int8_t *qx, bool zero, uint64_t &k) {
+// equal scores the lower rows.  64 of them at a time, of any slices.  G: blocks of
+// 64 slices listed together; B: slices looked at together.
+template <int G, int B>
+__device__ __forceinline__ int select_rows(const DenseArgs &a, int q, int64_t s0, int nsl, int nvl, int nl, uint32_t tk,
+                                           int32_t ts, uint64_t *cand, const int8_t *qx, bool zero, uint64_t &k) {
     const int lane = lane_id(), M = a.M;
     const uint4 *L = (const uint4 *)a.tk + (size_t)q * a.nslices + s0;
     const int32_t *perm = a.perm + s0 * 64;
-    uint16_t *slots = (uint16_t *)(cand + 64);  // slot in the partition (at most 1,024 slices)
-    constexpr int B = 8;                        // slices looked at together
+    uint32_t *slots = (uint32_t *)(cand + 64);  // slots in the partition to score
+    uint64_t *stage = cand + 64;                // before that, listed keys
+    constexpr int kSlots = 384;
     // least: the M-th best so far; the pend keys above it wait in cand
-    uint64_t least = 0ull, mask = 0ull, key[4];
-    int pend = 0, nslots = 0, b = 0, e = 0, w = 0;
-    if (nl <= 64) {
+    uint64_t least = 0ull, mask = 0ull;
+    int pend = 0, nslots = 0, g = 0, b = -64;
+    int c = 0, tot = 0, pos = 0, j0 = 0;  // listed keys of a group: a lane's, all, a lane's first place, the next to take
+    uint32_t ke[4 * G];
+    int32_t row[4 * G];
+    uint4 l = make_uint4(0u, 0u, 0u, 0u);
+    const bool every = ts == INT32_MIN;  // no bound: the lists hold fewer than M rows, every row is scored
+    if (every) {
+        g = nsl;
+        b = 0;
+    } else if (nl <= 64) {
         if (lane < nl) cand[lane] = k;
         pend = nl;
-        b = nsl;
+        g = nsl;
         if (nl >= M) {
             int rank = 0;
             for (int j = 0; j < nl; ++j) rank += readlane_u64(k, j) > k;
@@ -347,63 +331,107 @@ __device__ __forceinline__ int select_with_rescans(const DenseArgs &a, int q, in
     k = 0ull;
     for (;;) {
         uint64_t nk = 0ull;
-        bool last = false;
-        if (b < nsl) {  // the listed keys of 64 slices, one of each at a time
-            if (e == 0) {
-                const int i = b + lane, nv = i >= nsl ? 0 : i == nsl - 1 ? nvl : 64;
-                const uint4 l = L[min(i, nsl - 1)];
-                const uint32_t ke[4] = {l.x, l.y, l.z, l.w};
-                int32_t r[4];
+        bool last = false, score = false;
+        uint32_t slot = 0u;
+        int ns = 64;
+        if (every) {
+            last = b >= nsl;
+            score = !last;
+            slot = (uint32_t)(b * 64 + lane);
+            ++b;
+        } else if (g < nsl) {  // the listed keys of 64 * G slices, 64 of them at a time
+            if (j0 >= tot) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) r[j] = perm[(size_t)min(i, nsl - 1) * 64 + tk_rho(ke[j])];
+                for (int u = 0; u < G; ++u) {
+                    const int i = g + u * 64 + lane;
+                    const uint4 v = L[min(i, nsl - 1)];
+                    const int nv = i >= nsl ? 0 : i == nsl - 1 ? nvl : 64;
+                    ke[4 * u] = tk_rho(v.x) < nv ? v.x : 0u;
+                    ke[4 * u + 1] = tk_rho(v.y) < nv ? v.y : 0u;
+                    ke[4 * u + 2] = tk_rho(v.z) < nv ? v.z : 0u;
+                    ke[4 * u + 3] = tk_rho(v.w) < nv ? v.w : 0u;
+                }
+                // (the score of the M-th best: rows are looked up for what may pass it)
+                const uint32_t lo = max(tk, least != 0ull ? (uint32_t)(dkey_score_i32(least) + (1 << 25)) << 6 : 0u);
+                c = 0;
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    key[j] = tk_rho(ke[j]) < nv && ke[j] >= tk ? dkey_i32(tk_score(ke[j]), r[j]) : 0ull;
+                for (int e = 0; e < 4 * G; ++e) {
+                    const bool ok = ke[e] >= lo;
+                    row[e] = perm[ok ? (size_t)(g + (e >> 2) * 64 + lane) * 64 + tk_rho(ke[e]) : 0];
+                    ke[e] = ok ? ke[e] : 0u;
+                }
+#pragma unroll
+                for (int e = 0; e < 4 * G; ++e) {
+                    if (ke[e] != 0u && dkey_i32(tk_score(ke[e]), row[e]) <= least) ke[e] = 0u;
+                    c += ke[e] != 0u ? 1 : 0;
+                }
+                const int incl = (int)wave_prefix_sum((uint32_t)c);
+                pos = incl - c;
+                tot = __builtin_amdgcn_readlane(incl, 63);
+                j0 = 0;
             }
-            nk = e == 0 ? key[0] : e == 1 ? key[1] : e == 2 ? key[2] : key[3];
-            e = (e + 1) & 3;
-            b += e == 0 ? 64 : 0;
+            if (tot > 0) {
+                int at = pos - j0;
+#pragma unroll
+                for (int e = 0; e < 4 * G; ++e)
+                    if (ke[e] != 0u) {
+                        if (at >= 0 && at < 64) stage[at] = dkey_i32(tk_score(ke[e]), row[e]);
+                        ++at;
+                    }
+                wave_sync();
+                if (lane < tot - j0) nk = stage[lane];
+                wave_sync();
+            }
+            j0 += 64;
+            if (j0 >= tot) {
+                g += 64 * G;
+                tot = 0;
+            }
         } else {
-            // B slices at a time: their rows that may qualify
-            while (nslots < 64 && (mask != 0ull || w * 64 < nsl)) {
+            // the rows that may qualify of the slices whose fourth key does
+            while (nslots < 64 && (mask != 0ull || b + 64 < nsl)) {
                 if (mask == 0ull) {
-                    mask = readlane_u64(again[w], 0);
-                    ++w;
+                    b += 64;
+                    l = L[min(b + lane, nsl - 1)];
+                    mask = __ballot(b + lane < nsl && l.w >= tk && dkey_i32(tk_score(l.w), 0) > least);
                     continue;
                 }
                 int sl[B];
-                int32_t row[B];
-                uint4 l[B];
+                int32_t r[B];
+                uint64_t rest = mask;
 #pragma unroll
                 for (int j = 0; j < B; ++j) {
-                    sl[j] = mask ? (w - 1) * 64 + __builtin_ctzll(mask) : -1;
+                    sl[j] = rest ? __builtin_ctzll(rest) : -1;
+                    rest &= rest - 1;
+                }
+#pragma unroll
+                for (int j = 0; j < B; ++j) r[j] = perm[(size_t)(b + max(sl[j], 0)) * 64 + lane];
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    if (sl[j] < 0 || nslots > kSlots - 64) continue;
                     mask &= mask - 1;
-                }
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    row[j] = perm[(size_t)max(sl[j], 0) * 64 + lane];
-                    l[j] = L[max(sl[j], 0)];
-                }
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    const bool has = lane == tk_rho(l[j].x) || lane == tk_rho(l[j].y) || lane == tk_rho(l[j].z) ||
-                                     lane == tk_rho(l[j].w);
-                    const bool ok = sl[j] >= 0 && row[j] >= 0 && !has && dkey_i32(tk_score(l[j].w), row[j]) > least;
+                    const uint32_t lw = (uint32_t)__builtin_amdgcn_readlane((int)l.w, sl[j]);
+                    bool ok = r[j] >= 0 && dkey_i32(tk_score(lw), r[j]) > least;
+                    if (!__any(ok)) continue;
+                    ok = ok && lane != tk_rho(lw) && lane != tk_rho((uint32_t)__builtin_amdgcn_readlane((int)l.x, sl[j])) &&
+                         lane != tk_rho((uint32_t)__builtin_amdgcn_readlane((int)l.y, sl[j])) &&
+                         lane != tk_rho((uint32_t)__builtin_amdgcn_readlane((int)l.z, sl[j]));
                     const uint64_t m = __ballot(ok);
-                    if (ok) slots[nslots + mbcnt64(m)] = (uint16_t)(sl[j] * 64 + lane);
+                    if (ok) slots[nslots + mbcnt64(m)] = (uint32_t)((b + sl[j]) * 64 + lane);
                     nslots += __popcll(m);
                 }
             }
             wave_sync();
-            const int ns = min(nslots, 64);
+            ns = min(nslots, 64);
             last = ns == 0;
-            if (!last) {  // score the last 64 of them
-                const uint32_t slot = slots[nslots - ns + min(lane, ns - 1)];
-                const int32_t row = perm[slot];
-                const int32_t sc = zero ? 0 : slot_dot_packets(a, s0 * 64 + slot, qx);
-                if (lane < ns && sc >= ts) nk = dkey_i32(sc, row);
-                nslots -= ns;
-            }
+            score = !last;
+            if (score) slot = slots[nslots - ns + min(lane, ns - 1)];  // the last 64 of them
+            nslots -= ns;
+        }
+        if (score) {
+            const int32_t r = perm[slot];
+            const int32_t sc = zero ? 0 : every ? slice_dot_packets(a, s0 + b - 1, qx) : slot_dot_packets(a, s0 * 64 + slot, qx);
+            if (lane < ns && r >= 0 && sc >= ts) nk = dkey_i32(sc, r);
         }
         uint64_t m = __ballot(nk > least);
         if (last && !sorted) {
@@ -429,12 +457,14 @@ __device__ __forceinline__ int select_with_rescans(const DenseArgs &a, int q, in
 }
 
 // One wavefront per (partition p = blockIdx.x, query q = blockIdx.y*4 + wave),
-// for partitions of at most 64*U slices and M <= 32:
+// for partitions of at most 64*U slices:
 //  1. ts = a score that M distinct rows of the partition reach (INT32_MIN when
 //     there are not M): at least M and, equal scores aside, at most M + kSlack
-//     of the full slices' maxima reach it (up to 64 slices: M of their listed
-//     scores).  The partition's M-th best score is >= ts, so no row below ts
-//     can be in its Top-M.
+//     of the full slices' maxima reach it; up to 128 slices exactly M of their
+//     whole lists (few maxima, or low ones, would make every list drop rows
+//     that qualify: 400,000 x 500 in 64 partitions of 98 slices, M = 64, 64
+//     queries: 160 -> 129 us of a call).  The partition's M-th best score is
+//     >= ts, so no row below ts can be in its Top-M.
 //  2. Every listed key of a real row scoring >= ts is a candidate; one prefix
 //     sum places them, one gather finds their rows.  (Padding rows of the
 //     partial slice score 0: its maximum is left out of step 1, their keys,
@@ -445,8 +475,7 @@ __device__ __forceinline__ int select_with_rescans(const DenseArgs &a, int q, in
 //     100 queries: 64 -> 61 us of a call).
 //  4. Top-M of the candidates by (score, row) (quantify_util.py:173-196 with
 //     the lower-row tie rule), ranked by counting, then their FP32 rescoring
-//     (out != null).  More than 64 candidates, or kRescans slices: select_with_
-//     rescans.
+//     (out != null).  More than 64 candidates, or kRescans slices: select_rows.
 //
 // Bound: the memory requests of the rescoring (rows of a few cache lines each,
 // anywhere in the CSR), about 0.4 ns per row.  400,000 x 500, 100 queries:
@@ -457,16 +486,15 @@ __device__ __forceinline__ int select_with_rescans(const DenseArgs &a, int q, in
 template <int U>
 __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
     constexpr int kSlack = 8, kRescans = 8;  // slices rescanned one after the other
+    constexpr bool kExact = U <= 2;  // bound: the lists, not only the maxima
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int p = blockIdx.x, q = blockIdx.y * ACC_WAVES + wave;
     if (q >= a.nq) return;  // whole wavefront; no workgroup barrier below
     // per wavefront (2 KB): 64 candidates; 64 ranked keys and their entry
-    // ranges, before that the slots to score (at most 575 of 704); the slices
-    // to rescan, a bit each
+    // ranges, before that the slices to rescan or the slots to score
     uint64_t *cand = (uint64_t *)smem + wave * 256, *keys = cand + 64;
     uint2 *ranges = (uint2 *)(keys + 64);
-    uint64_t *again = cand + 240;
     int8_t *qx = (int8_t *)(smem + ACC_WAVES * 256 * 8) + (size_t)wave * a.cols_pad;
     float *xs = (float *)(smem + ACC_WAVES * 256 * 8 + (size_t)ACC_WAVES * a.cols_pad) + (size_t)wave * a.cols_pad;
     const int64_t s0 = a.part_slice[p];
@@ -476,7 +504,8 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
     const int M = a.M;
     const size_t base = ((size_t)q * a.split + p) * M;
 
-    int nn = 0;          // candidates kept, ranked in keys
+    uint64_t k = 0ull;  // lane i < n: a candidate
+    int n = 0;
     if (nsl > 0) {
         // unconditional loads (clamped into the partition, masked after) so
         // that the lists and the query for the rescoring arrive in one round
@@ -488,23 +517,20 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
         if (a.out) stage_query(xs, a.X + (size_t)q * a.cols, a.cols);
         uint32_t t;
         {
-            uint32_t v[U];
+            uint32_t v[kExact ? 4 * U : U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int i = u * 64 + lane;
                 if (i >= nsl) k4[u] = make_uint4(0u, 0u, 0u, 0u);
-                v[u] = i < nsl - 1 || nvl == 64 ? k4[u].x : 0u;
+                const bool full = i < nsl - 1 || nvl == 64;
+                v[u] = full ? k4[u].x : 0u;
+                if constexpr (kExact) {
+                    v[U + u] = full ? k4[u].y : 0u;
+                    v[2 * U + u] = full ? k4[u].z : 0u;
+                    v[3 * U + u] = full ? k4[u].w : 0u;
+                }
             }
-            if (nsl <= 64) {
-                // few slices: their whole lists (distinct rows), exactly --
-                // fewer than M maxima, or a low one, would make every list
-                // drop rows that qualify
-                const bool full = lane < nsl - 1 || nvl == 64;
-                const uint32_t w[4] = {full ? k4[0].x : 0u, full ? k4[0].y : 0u, full ? k4[0].z : 0u, full ? k4[0].w : 0u};
-                t = wave_bound_u32<4>(w, M, 0);
-            } else {
-                t = wave_bound_u32<U>(v, M, kSlack);
-            }
+            t = wave_bound_u32(v, M, kExact ? 0 : kSlack);
         }
         // tk: the smallest list key of a score that reaches the bound (keys of
         // one score differ in the row); without a bound that of any row
@@ -520,9 +546,7 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
         }
         const int incl = (int)wave_prefix_sum((uint32_t)c);
         const int nl = __builtin_amdgcn_readlane(incl, 63);
-        uint64_t k = 0ull;  // lane i < n: a candidate
         uint32_t listed = 0u;
-        int n = 0;
         if (nl <= 64) {
             int pos = incl - c;
 #pragma unroll
@@ -544,7 +568,8 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
         }
         const int32_t ts = t != 0u ? tk_score(t) : INT32_MIN;
         bool many = nl > 64 || nr > kRescans, zero = true;
-        if (nr > 0) {
+        if (nr > 0 || many) zero = stage_qx(a, q, qx);
+        if (nr > 0 && !many) {
             int i = 0;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -553,21 +578,8 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
                 if (k4[u].w >= tk && j < kRescans)
                     keys[j] = ((uint64_t)k4[u].w << 32) |
                               (uint32_t)((u * 64 + lane) << 18 | tk_rho(k4[u].z) << 12 | tk_rho(k4[u].y) << 6 | tk_rho(k4[u].x));
-                if (lane == 0) again[u] = m;
                 i += __popcll(m);
             }
-            // at most 1,024 columns, padded to whole dwords: one round trip
-            const uint32_t *src = (const uint32_t *)(a.qplain + (size_t)q * a.cols_pad);
-            const int nd = a.cols_pad / 4;
-            uint32_t v[4], any = 0u;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = src[min(j * 64 + lane, nd - 1)];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (j * 64 + lane < nd) ((uint32_t *)qx)[j * 64 + lane] = v[j];
-                any |= v[j];
-            }
-            zero = !__any(any != 0u);
             wave_sync();
         }
         for (int j = 0; j < nr && !many; ++j) {  // slice by slice
@@ -586,101 +598,74 @@ __global__ __launch_bounds__(ACC_WG) void dense_select_regs(DenseArgs a) {
             if (ok && !many) cand[n + mbcnt64(m)] = dkey_i32(sc, r);
             n += many ? 0 : __popcll(m);
         }
-        if (many) {
-            if (nr == 0 && lane < U) again[lane] = 0ull;
-            wave_sync();
-            n = select_with_rescans(a, q, s0, nsl, nvl, nl, tk, ts, cand, again, qx, zero, k);
+        // (expected false: 20,000 x 500, 8 queries, 41.6 us of a call; 42.8 with
+        // the block below laid out before the ordinary path)
+        if (__builtin_expect(many, false)) {
+            if (zero && a.part_row)
+                k = first_rows(a, p, n);
+            else
+                n = select_rows<2, 8>(a, q, s0, nsl, nvl, nl, tk, ts, cand, qx, zero, k);
         } else if (nr > 0) {
             wave_sync();
             if (lane >= nl && lane < n) k = cand[lane];
         }
-        // the candidates' CSR entry ranges, in flight while the ranks are
-        // counted (out set: the CSR is present)
-        uint2 rg = make_uint2(0u, 0u);
-        if (a.out) {
-            const int32_t r = lane < n ? dkey_row(k) : 0;
-            rg = make_uint2(a.ptr[r], a.ptr[r + 1]);
-        }
-        int rank = 0;
-        for (int j = 0; j < n; ++j) rank += readlane_u64(k, j) > k;  // distinct: one per row
-        nn = min(n, M);
-        if (lane < n && rank < nn) {
-            keys[rank] = k;
-            ranges[rank] = rg;
-        }
-        wave_sync();
     }
-    if (a.cand_rows_out)
-        for (int i = lane; i < M; i += 64) {
-            a.cand_rows_out[base + i] = i < nn ? dkey_row(keys[i]) : -1;
-            a.cand_scores_out[base + i] = i < nn ? dkey_score_i32(keys[i]) : 0;
-        }
-    if (!a.out) return;
-    switch (a.G) {
-        case 2: return rescore_rows<2>(a, keys, ranges, nn, base, xs);
-        case 4: return rescore_rows<4>(a, keys, ranges, nn, base, xs);
-        case 8: return rescore_rows<8>(a, keys, ranges, nn, base, xs);
-        case 16: return rescore_rows<16>(a, keys, ranges, nn, base, xs);
-        default: return rescore_rows<32>(a, keys, ranges, nn, base, xs);
-    }
+    finish_rows(a, k, n, keys, ranges, base, xs);
 }
 
-// The same for any partition and M <= 64, by a collector of the offered keys:
-// the lists are streamed twice (threshold = the M-th best full-slice maximum,
-// then offers).
+// The same for partitions of any size: the threshold is the M-th best full-slice
+// maximum (a sorted buffer of them), the lists are streamed twice (threshold,
+// then candidates).  400,000 x 500 in one partition of 6,250 slices, 8 queries,
+// M = 32: 158 -> 139 us of a call; queries of zeros 34,600 -> 44 (a collector
+// was offered every row of each slice whose list was full of ties).
 __global__ __launch_bounds__(ACC_WG) void dense_select(DenseArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int p = blockIdx.x, q = blockIdx.y * ACC_WAVES + wave;
     if (q >= a.nq) return;  // whole wavefront; no workgroup barrier below
-    uint64_t *bufA = (uint64_t *)smem + wave * 256, *bufB = bufA + 128;
+    uint64_t *cand = (uint64_t *)smem + wave * 256, *keys = cand + 64;
+    uint2 *ranges = (uint2 *)(keys + 64);
     int8_t *qx = (int8_t *)(smem + ACC_WAVES * 256 * 8) + (size_t)wave * a.cols_pad;
     float *xs = (float *)(smem + ACC_WAVES * 256 * 8 + (size_t)ACC_WAVES * a.cols_pad) + (size_t)wave * a.cols_pad;
-    const float *xq = a.X + (size_t)q * a.cols;
     const int64_t s0 = a.part_slice[p];
     const int nsl = (int)(a.part_slice[p + 1] - s0);
     const uint4 *L = (const uint4 *)a.tk + (size_t)q * a.nslices + s0;
     const int M = a.M;
-    const size_t base = ((size_t)q * a.split + p) * M;
-    bool have_qx = false;
 
-    if (a.out) stage_query(xs, xq, a.cols);
-    WaveTopM<2> cb;
-    cb.init(bufB, M);
-    constexpr int U = 4;
-    int32_t ts = INT32_MIN;
-    {
-        WaveTopM<2> ca;
-        ca.init(bufA, M);
-        for (int b = 0; b < nsl; b += 64 * U) {
-            uint32_t k[U];
+    uint64_t k = 0ull;
+    int n = 0;
+    const bool zero = nsl > 0 && stage_qx(a, q, qx);
+    if (zero && a.part_row) {
+        k = first_rows(a, p, n);
+    } else if (nsl > 0) {
+        const int nvl = (int)a.nvalid[s0 + nsl - 1];  // every slice is full except a partition's last one
+        uint32_t t = 0u;
+        {
+            constexpr int U = 4;
+            WaveTopM<2> ca;
+            ca.init(cand, M);
+            for (int b = 0; b < nsl; b += 64 * U) {
+                uint32_t v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = b + u * 64 + lane;
-                k[u] = i < nsl && a.nvalid[s0 + i] == 64 ? L[i].x : 0u;
+                for (int u = 0; u < U; ++u) {
+                    const int i = b + u * 64 + lane;
+                    v[u] = i < nsl - 1 || (i == nsl - 1 && nvl == 64) ? L[i].x : 0u;
+                }
+                static_assert(U == 4, "four pushes below");
+                ca.push(v[0] != 0u, ((uint64_t)v[0] << 32) | (uint32_t)(b + lane));
+                ca.push(v[1] != 0u, ((uint64_t)v[1] << 32) | (uint32_t)(b + 64 + lane));
+                ca.push(v[2] != 0u, ((uint64_t)v[2] << 32) | (uint32_t)(b + 128 + lane));
+                ca.push(v[3] != 0u, ((uint64_t)v[3] << 32) | (uint32_t)(b + 192 + lane));
             }
-            static_assert(U == 4, "four pushes below");
-            ca.push(k[0] != 0u, ((uint64_t)k[0] << 32) | (uint32_t)(b + lane));
-            ca.push(k[1] != 0u, ((uint64_t)k[1] << 32) | (uint32_t)(b + 64 + lane));
-            ca.push(k[2] != 0u, ((uint64_t)k[2] << 32) | (uint32_t)(b + 128 + lane));
-            ca.push(k[3] != 0u, ((uint64_t)k[3] << 32) | (uint32_t)(b + 192 + lane));
+            ca.compact();
+            if (ca.n >= M) t = (uint32_t)(ca.buf[M - 1] >> 32);
         }
-        ca.compact();
-        if (ca.n >= M) ts = tk_score((uint32_t)(ca.buf[M - 1] >> 32));
+        wave_sync();
+        n = select_rows<4, 16>(a, q, s0, nsl, nvl, 65, max(t & ~63u, 64u),
+                               t != 0u ? tk_score(t) : INT32_MIN, cand, qx, zero, k);
     }
-    for (int b = 0; b < nsl; b += 64 * U) {
-        uint4 k4[U];
-        int nv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = b + u * 64 + lane;
-            k4[u] = i < nsl ? L[i] : make_uint4(0u, 0u, 0u, 0u);
-            nv[u] = i < nsl ? (int)a.nvalid[s0 + i] : 0;
-        }
-        offer_lists<U>(a, cb, k4, nv, s0, b, ts, q, qx, have_qx);
-    }
-    cb.compact();
-    emit_candidates(a, cb.buf, cb.n, base, xs);
+    if (a.out) stage_query(xs, a.X + (size_t)q * a.cols, a.cols);
+    finish_rows(a, k, n, keys, ranges, ((size_t)q * a.split + p) * M, xs);
 }
 
 // One workgroup per query: each wavefront sorts a quarter of the query's
@@ -707,8 +692,9 @@ __global__ __launch_bounds__(ACC_WG) void batch_topk_radix(DenseArgs a) {
 }
 
 dense_fn get_dense_prep() { return dense_prep; }
-dense_fn get_dense_select(int64_t part_slices, int M) {
-    if (M > 32 || part_slices > 1024) return dense_select;
+dense_fn get_dense_select(int64_t part_slices) {
+    if (part_slices > 1024) return dense_select;
+    if (part_slices <= 128) return part_slices <= 64 ? dense_select_regs<1> : dense_select_regs<2>;
     return part_slices <= 256 ? dense_select_regs<4> : part_slices <= 512 ? dense_select_regs<8> : dense_select_regs<16>;
 }
 dense_fn get_batch_topk_radix(int V) {

@@ -280,74 +280,6 @@ __device__ __forceinline__ float group_dot_range(const colx_t *idx, const float 
     return p;
 }
 
-// The same dot products for C rows at once, given their entry ranges
-// [lo[c], hi[c]) (lo = hi for an empty or invalid row), against x: their
-// loads are issued together, so C rows cost the memory round trips of one.
-// Each row is summed in the order of group_dot_rt (entries g, g+G, ... with
-// fmaf, then the butterfly), so the results are the same floats.
-template <int C, int U = 4>
-__device__ __forceinline__ void group_dot_ranges_multi(const colx_t *idx, const float *val, const float *x,
-                                                       const uint32_t (&lo)[C], const uint32_t (&hi)[C], int G,
-                                                       float (&out)[C]) {
-    const int g = lane_id() & (G - 1);
-    uint32_t b[C], e[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        b[c] = lo[c] + g;
-        e[c] = hi[c];
-        out[c] = 0.f;
-    }
-    for (uint32_t o = 0;; o += U * G) {
-        bool any = false;
-#pragma unroll
-        for (int c = 0; c < C; ++c) any = any || b[c] + o < e[c];
-        if (!any) break;
-        float v[C][U], xv[C][U];
-        uint32_t cl[C][U];
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            // clamped into the matrix (some row has entries while the loop
-            // runs): unconditional loads issue together
-            const uint32_t last = e[c] > 0u ? e[c] - 1u : 0u;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t jj = min(b[c] + o + u * G, last);
-                v[c][u] = val[jj];
-                cl[c][u] = idx[jj];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int u = 0; u < U; ++u) xv[c][u] = x_at(x, cl[c][u]);
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (b[c] + o + u * G < e[c]) out[c] = __builtin_fmaf(v[c][u], xv[c][u], out[c]);
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        for (int s = G >> 1; s >= 1; s >>= 1) out[c] = out[c] + __shfl_xor(out[c], s);
-}
-
-// group_dot_ranges_multi for rows r[c] (r[c] is a row of the matrix also for
-// invalid candidates, so the bound loads are unconditional and issue together).
-template <int C, int U = 4>
-__device__ __forceinline__ void group_dot_rt_multi(const uint32_t *ptr, const colx_t *idx, const float *val,
-                                                   const float *x, const int32_t (&r)[C],
-                                                   const bool (&valid)[C], int G, float (&out)[C]) {
-    uint32_t lo[C], hi[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const uint32_t p0 = ptr[r[c]], p1 = ptr[r[c] + 1];
-        lo[c] = valid[c] ? p0 : 0u;
-        hi[c] = valid[c] ? p1 : 0u;
-    }
-    group_dot_ranges_multi<C, U>(idx, val, x, lo, hi, G, out);
-}
-
-
 // One workgroup of ACC_WG threads: the K best of total <= ACC_WAVES*64*R
 // ranking keys (0 = empty) into out[0, K), then (value -inf, index -1) past
 // the nonzero keys.  Each wavefront sorts its 64*R keys in registers and
@@ -758,6 +690,7 @@ struct DenseArgs {
     const uint2 *pslices;        // per slice: (offset in groups, groups of decode wavefront w in byte w)
     const int32_t *perm;
     const int64_t *part_slice;   // split + 1
+    const int32_t *part_row;     // split + 1 first rows (null: rows are dealt to partitions in another order)
     const uint8_t *nvalid;       // valid rows per slice (a prefix of its lanes)
     int64_t nslices;
     int cols, cols_pad, nkb, col_bits, val_bits, is_signed, u8off;
@@ -817,7 +750,7 @@ batch_fn get_batch_select();                                   // k_batch.hip
 batch_fn get_batch_final(int R);
 typedef void (*dense_fn)(DenseArgs);
 dense_fn get_dense_prep();                                     // k_dense.hip
-dense_fn get_dense_select(int64_t part_slices, int M);
+dense_fn get_dense_select(int64_t part_slices);
 dense_fn get_batch_topk_radix(int V);
 dense_fn get_batch_topk(int R);
 dense_fn get_pk_scores_8();                               // k_pkmfma_a.hip

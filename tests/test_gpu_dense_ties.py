@@ -79,3 +79,43 @@ def test_time_of_ties(acc, gpu, kind):
     usual = call_us(acc, g, queries("usual", 8, 500, rng), 512, 100)
     ties = call_us(acc, g, queries(kind, 8, 500, rng), 512, 100)
     assert ties < 4 * usual, (ties, usual)  # slice after slice rescanned: 10 to 30 times
+
+
+# up to 64 rows a partition, of 1 to 1,094 slices (each way to hold their lists; past 1,024 they are streamed), fewer rows or
+# listed rows than M, rows shuffled over the partitions or not: the three layouts agree on ties, and a query of zeros ranks
+# the rows in their order
+@pytest.mark.parametrize("rows,split,M", [(700, 8, 64), (8330, 2, 64), (20000, 16, 64), (30000, 2, 64), (65800, 4, 33), (70000, 2, 64),
+                                          (70000, 1, 64), (70000, 1, 20), (140000, 2, 48), (300, 20, 17)])
+@pytest.mark.parametrize("seed", [0, 7])
+@pytest.mark.parametrize("kind", ["zeros", "few", "usual"])
+def test_every_layout_of_ties(acc, gpu, rows, split, M, seed, kind):
+    rng = np.random.default_rng(rows + M)
+    cols, nq, ck = 90, 5, split * M
+    k = min(ck, rows, 960)
+    csr = matrix(acc, kind, rows, cols, (4, 12), False, rng)
+    g = acc.GpuMatrix(csr, csr.pack(bits=8, split=split, shuffle_seed=seed))
+    x = queries(kind, nq, cols, rng)
+    x[nq - 1] = -0.0
+    X = acc.DeviceBuffer.from_numpy(x)
+    got = {}
+    for mode in (acc.BATCH_SPARSE, acc.BATCH_DENSE, acc.BATCH_SINGLE):
+        g.set_batch_mode(mode)
+        out = acc.DeviceBuffer.from_numpy(np.full((nq, k, 2), 9, np.int32))
+        g.topk_lowbit_batch(X, np.full(nq, k, np.int32), ck, out, k)
+        acc.synchronize()
+        got[mode] = out.numpy()
+    np.testing.assert_array_equal(got[acc.BATCH_DENSE], got[acc.BATCH_SPARSE])
+    np.testing.assert_array_equal(got[acc.BATCH_SINGLE], got[acc.BATCH_SPARSE])
+
+
+# more than 32 rows a partition; more than 1,024 slices
+@pytest.mark.parametrize("split,M", [(16, 64), (1, 20)])
+@pytest.mark.parametrize("kind", ["zeros", "few"])
+def test_time_of_ties_in_every_layout(acc, gpu, kind, split, M):
+    rng = np.random.default_rng(8)
+    csr = matrix(acc, kind, 200000, 300, (5, 30), False, rng)
+    g = acc.GpuMatrix(csr, csr.pack(bits=8, split=split))
+    g.set_batch_mode(acc.BATCH_DENSE)
+    usual = call_us(acc, g, queries("usual", 8, 300, rng), split * M, 20)
+    ties = call_us(acc, g, queries(kind, 8, 300, rng), split * M, 20)
+    assert ties < 4 * usual, (ties, usual)  # slice after slice rescanned: 10 to 200 times
