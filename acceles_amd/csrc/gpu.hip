@@ -417,7 +417,7 @@ DenseArgs dense_args(const acc_gpu_matrix *m) {
 }
 
 // Estimated time of a batch per layout, in us, for M rows kept per partition.
-// Fitted to 952 measurements (3,000 to 5,000,000 rows of 3 to 300 entries, 1 to
+// Fitted to 1,216 measurements (3,000 to 5,000,000 rows of 3 to 300 entries, 1 to
 // 256 queries, M = 1 to 64, partitions of 2 to 7,800 slices); us single /
 // packets / matrix cores at 8 queries, CK 512 unless given:
 //   20,000 x 500 172 / 66 / 38, CK 1024 in 16 partitions 273 / 84 / 132
